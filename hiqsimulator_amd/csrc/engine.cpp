@@ -2,6 +2,7 @@
 #include "engine.hpp"
 
 #include "batch.hpp"
+#include "gate_prog.hpp"
 #include "sched.hpp"
 
 #include <algorithm>
@@ -525,6 +526,8 @@ void Engine::set_pass_mode(int mode)
 void Engine::drain_queue(size_t keep)
 {
      if (queue_.size() <= keep || queue_.empty()) return;
+     int passes = 0;
+     if (gate_items(queue_, keep, passes)) return;
      int width = 4;
      for (const auto& g: queue_) width = std::max(width, static_cast<int>(g.t.size() + g.c.size()));
      tile_items(queue_, width, keep);
@@ -1097,6 +1100,8 @@ int Engine::apply_tiled(const std::vector<Gate>& gates, int op_width)
           pg.m = g.m;
           items.push_back(std::move(pg));
      }
+     int passes = 0;
+     if (gate_items(items, 0, passes)) return passes;
      if (n >= kTileBits) return tile_items(items, op_width, 0);
      // small states: every op is one plain fused pass
      GateList gl;
@@ -1125,6 +1130,71 @@ int Engine::apply_tiled(const std::vector<Gate>& gates, int op_width)
           dense_or_diag(M, p32, 0, false);
      }
      return nc;
+}
+
+Engine::ProgSlot& Engine::program_slot(size_t need)
+{
+     ProgSlot& ps = prog_[prog_next_];
+     prog_next_ = (prog_next_ + 1) % kProgSlots;
+     if (ps.busy) check(hipEventSynchronize(ps.ev), "hipEventSynchronize");
+     ps.busy = false;
+     if (need > ps.cap) {
+          if (ps.h) check(hipHostFree(ps.h), "hipHostFree");
+          if (ps.d) check(hipFree(ps.d), "hipFree");
+          ps.h = ps.d = nullptr;
+          ps.cap = 0;
+          const size_t cap = std::max(need, size_t(1) << 20);
+          check(hipHostMalloc(reinterpret_cast<void**>(&ps.h), cap, hipHostMallocDefault), "hipHostMalloc(program)");
+          check(hipMalloc(reinterpret_cast<void**>(&ps.d), cap), "hipMalloc(program)");
+          ps.cap = cap;
+     }
+     if (!ps.ev) check(hipEventCreateWithFlags(&ps.ev, hipEventDisableTiming), "hipEventCreate");
+     return ps;
+}
+
+bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes)
+{
+     passes = 0;
+     const int n = n_qubits();
+     if (n < gate_tile_bits(prec_) || n > 40) return false;
+     std::vector<GateUnit> units(items.size());
+     for (size_t i = 0; i < items.size(); ++i)
+          if (!make_gate_unit(items[i].m.a.data(), items[i].t, items[i].c, units[i])) return false;
+     // The passes go out in groups of 1, 2, 4, ...: the first runs while the
+     // others are planned and compiled.
+     GatePassPlanner planner(units, n, prec_);
+     GatePassPlan plan;
+     for (size_t group = 1; planner.remaining().size() > keep; group *= 2) {
+          std::vector<GatePass> gp;
+          std::vector<GateStage> stages;
+          std::vector<char> ops;
+          while (gp.size() < group && planner.remaining().size() > keep && planner.next(plan)) {
+               gp.emplace_back();
+               compile_gate_pass(units, plan, n, prec_, gp.back(), stages, ops);
+          }
+          for (const auto& p: gp) check_gate_pass(p, stages, ops, prec_, n);
+          const size_t stage_bytes = (stages.size() * sizeof(GateStage) + 255) / 256 * 256;
+          const size_t need = stage_bytes + ops.size();
+          ProgSlot& ps = program_slot(need);
+          std::memcpy(ps.h, stages.data(), stages.size() * sizeof(GateStage));
+          std::memcpy(ps.h + stage_bytes, ops.data(), ops.size());
+          check(hipMemcpyAsync(ps.d, ps.h, need, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync(program)");
+          for (const auto& p: gp) {
+               begin_timed(kTile);
+               check(launch_gate_pass(d_state_, prec_, n, p, reinterpret_cast<const GateStage*>(ps.d), ps.d + stage_bytes,
+                                      stream_),
+                     "gate pass");
+               end_timed();
+               ++passes;
+          }
+          check(hipEventRecord(ps.ev, stream_), "hipEventRecord");
+          ps.busy = true;
+     }
+     std::vector<PosGate> rest;
+     rest.reserve(planner.remaining().size());
+     for (int i: planner.remaining()) rest.push_back(std::move(items[i]));
+     items.swap(rest);
+     return true;
 }
 
 int Engine::tile_items(std::vector<PosGate>& items, int op_width, size_t keep)
@@ -1191,22 +1261,7 @@ int Engine::tile_items(std::vector<PosGate>& items, int op_width, size_t keep)
      }
      const size_t ops_bytes = (ops.size() * sizeof(TileOp) + 255) / 256 * 256;
      const size_t need = ops_bytes + mats.size();
-     // staging slot: waits only for the launches of kProgSlots groups ago
-     ProgSlot& ps = prog_[prog_next_];
-     prog_next_ = (prog_next_ + 1) % kProgSlots;
-     if (ps.busy) check(hipEventSynchronize(ps.ev), "hipEventSynchronize");
-     ps.busy = false;
-     if (need > ps.cap) {
-          if (ps.h) check(hipHostFree(ps.h), "hipHostFree");
-          if (ps.d) check(hipFree(ps.d), "hipFree");
-          ps.h = ps.d = nullptr;
-          ps.cap = 0;
-          const size_t cap = std::max(need, size_t(1) << 20);
-          check(hipHostMalloc(reinterpret_cast<void**>(&ps.h), cap, hipHostMallocDefault), "hipHostMalloc(program)");
-          check(hipMalloc(reinterpret_cast<void**>(&ps.d), cap), "hipMalloc(program)");
-          ps.cap = cap;
-     }
-     if (!ps.ev) check(hipEventCreateWithFlags(&ps.ev, hipEventDisableTiming), "hipEventCreate");
+     ProgSlot& ps = program_slot(need);
      std::memcpy(ps.h, ops.data(), ops.size() * sizeof(TileOp));
      std::memcpy(ps.h + ops_bytes, mats.data(), mats.size());
      check(hipMemcpyAsync(ps.d, ps.h, need, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync(program)");

@@ -197,6 +197,14 @@ private:
      // `items` (the rest keep program order).  Needs n >= kTileBits.
      // Returns the number of HBM passes launched.
      int tile_items(std::vector<PosGate>& items, int op_width, size_t keep);
+     // The same by gate programs (gate_prog.hpp), for states of 13 or more
+     // qubits and lists whose gates mix at most two qubits each; false (and
+     // nothing done) for others.
+     bool gate_items(std::vector<PosGate>& items, size_t keep, int& passes);
+     // A free staging slot of at least `bytes`; waits for the launches of
+     // kProgSlots groups ago.
+     struct ProgSlot;
+     ProgSlot& program_slot(size_t bytes);
      void release_buffer(void*& p);
      void collect_retired();
      // A same-size out-of-place result in d_tmp_ becomes the state: the

@@ -1,0 +1,215 @@
+// Gate programs: a gate list applied to a state tile by tile, gate by gate.
+//
+// A tile program (batch.hpp) multiplies fused 2^k x 2^k matrices into LDS
+// tiles; its cost is that of the dense products, whatever the gates were.
+// Most gates are one-qubit gates, controlled gates and phases, and applied by
+// themselves they take a fraction of the fused product's operations: with one
+// coefficient factored out into a scale that a whole pass shares, H, Rx and
+// Ry cost two fused multiply-adds an amplitude, a phase two, a CNOT none
+// (against 48 for a 4-qubit product that holds about eight such gates).
+// Also, only the qubits that a gate mixes have to lie in the tile: control
+// and diagonal qubits are conditions on the index, which a tile can evaluate
+// wherever they are, so a pass takes gates that a dense plan cannot.
+//
+// A pass covers tiles of 2^13 amplitudes in complex128 and 2^14 in complex64:
+// index bits 0..3 (runs of 16 amplitudes: 256 and 128 bytes) and nine or ten
+// chosen bits.  A workgroup of 512 threads holds its tile in registers, 16 or
+// 32 amplitudes (four or five tile bits, 64 registers either way) a thread.
+// The pass is a list of stages; each keeps four or five tile bits in the
+// thread and applies every gate that mixes only those, in program order, and
+// between stages the tile is regrouped through LDS.
+//
+// This header: the device records, the host planner (which gates go into
+// which pass and stage) and the compiler from gates to records.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <complex>
+#include <cstddef>
+#include <cstdint>
+#include <vector>
+
+#include "kernels.hpp"
+
+namespace hq {
+
+constexpr int kGateLow = 4;                     // index bits 0..3 are always tile bits
+constexpr int kGateThr = 9;                     // tile bits of the thread index
+constexpr int kGateThreads = 1 << kGateThr;
+// Tile bits in a thread's registers, and all tile bits.
+constexpr int gate_reg(Prec p) { return p == Prec::C128 ? 4 : 5; }
+constexpr int gate_tile_bits(Prec p) { return kGateThr + gate_reg(p); }
+constexpr int gate_high(Prec p) { return gate_tile_bits(p) - kGateLow; }  // chosen bits
+constexpr int kGateMaxReg = 5, kGateMaxTile = kGateThr + kGateMaxReg, kGateMaxHigh = kGateMaxTile - kGateLow;
+constexpr size_t kGateMaxStages = 255;      // a pass's stage count is a byte
+constexpr size_t kGateMaxStageUnits = 512;  // and a stage's record count 16 bits
+
+// ---- device records ---------------------------------------------------------
+// Opcodes.  b is the register bit (0..4) an op acts on.
+enum GateCode : uint32_t {
+     // A layer: rotations on any of the register bits, then phases on them,
+     // then controlled swaps between them, in one record.  aux: rotation kind
+     // of bit b at 2 b (kGateKind*), phase flag of bit b at 10 + b.  c: two
+     // coefficients a bit.  With phases, `count` is 1 and the next record's c
+     // holds a factor a bit.  omask and oval are no condition but up to 16
+     // bytes (target * 8 + control), tcond their number.
+     kGateLayer = 0,
+     kGateRM = 1,     // +b: a' = a + c0 z, z' = -z + c1 a (real c)
+     kGateR4 = 6,     // +b: real 2 x 2 matrix c0..c3
+     kGateG = 11,     // +b: complex 2 x 2 matrix c0..c7, where the register condition holds
+     kGateXA = 16,    // +b: a and z change places
+     kGateX = 21,     // +b: the same where the register condition holds
+     kGateXC = 26,    // the same for target aux / 8 under control aux % 8, register bits
+     kGatePAll = 27,  // every amplitude times c0 + i c1
+     kGatePT = 28,    // the same where the register condition holds
+     kGatePA = 29,    // +b: amplitudes with bit b times the product of the next `count`
+                      // records' factors (two doubles at c) whose conditions hold
+     kGatePL = 34,    // the same for every amplitude
+     kGateG2 = 35,    // + pair: complex 4 x 4 matrix in the coefficients of the next four
+                      // records, on the register pair, where the register condition holds
+     kGateCodes = 45
+};
+// Rotation kinds of a layer.
+enum GateKind : uint32_t {
+     kGateKindNone = 0,
+     kGateKindReal = 1,  // a' = a + c0 z, z' = z + c1 a
+     kGateKindH = 2,     // a' = a + z, z' = a - z
+     kGateKindImag = 3   // a' = a + i c0 z, z' = z + i c1 a
+};
+// Register pairs of kGateG2: (0,1) (0,2) (1,2) (0,3) (1,3) (2,3) (0,4) (1,4) (2,4) (3,4).
+constexpr uint32_t gate_pair(int b0, int b1) { return static_cast<uint32_t>(b1 * (b1 - 1) / 2 + b0); }
+constexpr uint32_t kGateMaxList = 255;  // `count` is a byte
+
+// One op.  But for layers it applies where (tile base index & omask) == oval,
+// (thread & tmask) == tval and, for the ops that say so, (amplitude &
+// regmask) == regval.
+template <typename R>
+struct GateOp {
+     uint32_t code;   // opcode | count << 8 | aux << 16; aux = regmask | regval << 5 where that is asked
+     uint32_t tcond;  // tmask | tval << 16
+     uint64_t omask, oval;
+     R c[10];
+};
+static_assert(sizeof(GateOp<double>) == 104 && sizeof(GateOp<float>) == 64 &&
+                  offsetof(GateOp<double>, c) == offsetof(GateOp<float>, c),
+              "record sizes");
+inline size_t gate_op_bytes(Prec p) { return p == Prec::C128 ? sizeof(GateOp<double>) : sizeof(GateOp<float>); }
+
+// One stage: LDS byte offsets of the thread bits and the register bits (the
+// slot of an amplitude is the XOR of its bits' offsets) and its ops.
+struct GateStage {
+     uint16_t thr_lds[kGateThr];
+     uint16_t reg_lds[kGateMaxReg];
+     uint16_t nops, pad;
+     uint32_t op_first;
+};
+static_assert(sizeof(GateStage) == 36, "record size");
+
+// One pass over a state: the chosen bits, the index bits of the first
+// stage's (load) and the last stage's (store) thread and register bits, and
+// the stages.
+struct GatePass {
+     uint8_t hpos[kGateMaxHigh];
+     uint8_t in_thr[kGateThr], in_reg[kGateMaxReg];
+     uint8_t out_thr[kGateThr], out_reg[kGateMaxReg];
+     uint8_t nstages, pad;
+     uint32_t stage_first;
+};
+static_assert(sizeof(GatePass) == 44, "record size");
+
+// One pass of one state inside a launch over many states.
+struct GateItem {
+     uint64_t state_off;    // first amplitude of the state
+     uint64_t block_start;  // first workgroup
+     uint32_t log_blocks;   // log2 of its tiles
+     GatePass pass;
+};
+static_assert(sizeof(GateItem) == 64, "record size");
+
+// Slot of tile rank r in LDS, as an XOR mask over the slots: the low bits
+// hold the low rank bits XOR-ed with a linear map of the others.  64 banks of
+// 4 bytes serve 32 lanes without a conflict when their low five (8-byte
+// slots, complex128) or six (4-byte slots, complex64) slot bits are distinct.
+// The columns below form binary linear codes of minimum distance 5: whichever
+// ranks are in registers, five of the others have independent columns, and
+// those are given to the first five lane bits.
+inline uint32_t gate_slot(Prec p, int rank)
+{
+     constexpr uint8_t c5[13] = {1, 2, 4, 8, 16, 31, 7, 25, 11, 10, 5, 23, 20};
+     constexpr uint8_t c6[14] = {1, 2, 4, 8, 16, 32, 47, 25, 51, 29, 30, 59, 60, 53};
+     if (p == Prec::C128) return (rank >= 5 ? 1u << rank : 0u) | c5[rank];
+     return (rank >= 6 ? 1u << rank : 0u) | c6[rank];
+}
+constexpr uint32_t gate_slot_bytes(Prec p) { return p == Prec::C128 ? 8 : 4; }
+
+// ---- host: gates ------------------------------------------------------------
+// A gate split by what it does to each of its index bits: `a` are the bits it
+// mixes (at most two), `d` the bits it only depends on (controls, and
+// targets in which its matrix is block diagonal).  Branch: what happens to
+// the mixed bits where (index & cmask) == cval; u is the factor (no mixed
+// bit), the 2 x 2 or the 4 x 4 matrix (bit l <-> act[l]), row-major.
+// Identity branches are left out.
+struct GateBranch {
+     uint64_t cmask = 0, cval = 0;
+     std::complex<double> u[16];
+};
+struct GateUnit {
+     uint64_t a = 0, d = 0;
+     int na = 0;
+     uint8_t act[2] = {0, 0};
+     std::vector<GateBranch> br;
+};
+// The unit of a gate (2^t x 2^t matrix m, row-major, bit l <-> targets[l];
+// positions below 62); false when it mixes more than two bits.
+bool make_gate_unit(const std::complex<double>* m, const std::vector<int64_t>& targets,
+                    const std::vector<int64_t>& ctrls, GateUnit& out);
+
+// ---- host: planning ---------------------------------------------------------
+struct GatePassPlan {
+     uint64_t bits = 0;                     // the tile's index bits
+     std::vector<uint64_t> regs;            // per stage: the bits its gates mix
+     std::vector<std::vector<int>> stages;  // per stage: unit indices, program order
+};
+
+// One pass at a time from the front of the list.  A unit is taken if the bits
+// it mixes lie in the tile and it commutes with every unit skipped before it:
+// neither mixes a bit that the other touches.
+class GatePassPlanner {
+public:
+     GatePassPlanner(const std::vector<GateUnit>& units, int n, Prec prec);
+     bool next(GatePassPlan& out);
+     // Indices of the units not planned yet, in program order.
+     const std::vector<int>& remaining() const { return rem_; }
+
+private:
+     uint64_t choose(const std::vector<int>& list, uint64_t fixed, uint64_t allowed, int k) const;
+     void take(std::vector<int>& list, uint64_t S, size_t cap, std::vector<int>& out) const;
+     const std::vector<GateUnit>& units_;
+     int n_;
+     Prec prec_;
+     std::vector<int> rem_;
+};
+
+// ---- host: compilation ------------------------------------------------------
+// Appends the records of one pass: its stages to `stages`, its ops (of the
+// state's precision) to `ops`.  pass.stage_first and the stages' op_first
+// count from the beginning of the arrays.  `ops` always ends in one spare
+// record (the kernel reads one ahead).
+void compile_gate_pass(const std::vector<GateUnit>& units, const GatePassPlan& plan, int n, Prec prec,
+                       GatePass& pass, std::vector<GateStage>& stages, std::vector<char>& ops);
+// Throws unless every record of the pass stays inside the tile, the arrays
+// and a state of 2^n amplitudes.
+void check_gate_pass(const GatePass& pass, const std::vector<GateStage>& stages, const std::vector<char>& ops,
+                     Prec prec, int n);
+
+// ---- launches (gate_kernels.hip) --------------------------------------------
+// One pass over a state of 2^n amplitudes (gate_tile_bits <= n <= 40); stages and ops are
+// device arrays, ops with one spare record at the end.
+hipError_t launch_gate_pass(void* psi, Prec prec, int n_qubits, const GatePass& pass, const GateStage* stages,
+                            const void* ops, hipStream_t s);
+// The same for many states of one arena.
+hipError_t launch_gate_items(void* arena, Prec prec, const GateItem* items, int nitems, const GateStage* stages,
+                             const void* ops, uint64_t total_blocks, hipStream_t s);
+
+}  // namespace hq
