@@ -197,9 +197,9 @@ private:
      // `items` (the rest keep program order).  Needs n >= kTileBits.
      // Returns the number of HBM passes launched.
      int tile_items(std::vector<PosGate>& items, int op_width, size_t keep);
-     // The same by gate programs (gate_prog.hpp), for states of 13 or more
-     // qubits and lists whose gates mix at most two qubits each; false (and
-     // nothing done) for others.
+     // The same by gate programs (gate_prog.hpp), for states of at least
+     // gate_min_qubits and lists whose gates mix at most two qubits each;
+     // false (and nothing done) for others.
      bool gate_items(std::vector<PosGate>& items, size_t keep, int& passes);
      // A free staging slot of at least `bytes`; waits for the launches of
      // kProgSlots groups ago.

@@ -582,27 +582,6 @@ __global__ void __launch_bounds__(kGateThreads) __attribute__((amdgpu_waves_per_
      gate_program<R>(psi, P, stages + P.stage_first, ops, swizzle_block(b, swz), lds);
 }
 
-template <typename R>
-__global__ void __launch_bounds__(kGateThreads) __attribute__((amdgpu_waves_per_eu(4)))
-    k_gate_items(VT<R>* __restrict__ arena, const GateItem* __restrict__ items, const int nitems,
-                 const GateStage* __restrict__ stages, const GateOp<R>* __restrict__ ops, const int swz,
-                 const uint64_t total_blocks)
-{
-     __shared__ __align__(16) char lds[sizeof(R) << Shape<R>::T];
-     const uint64_t b = block_linear();
-     if (b >= total_blocks) return;  // padding of the 2-D grid (whole block)
-     int lo = 0, hi = nitems - 1;
-     while (lo < hi) {
-          const int mid = (lo + hi + 1) >> 1;
-          if (items[mid].block_start <= b) lo = mid;
-          else hi = mid - 1;
-     }
-     const GateItem it = load_record(items + lo);
-     const int lb = static_cast<int>(it.log_blocks);
-     gate_program<R>(arena + it.state_off, it.pass, stages + it.pass.stage_first, ops,
-                     swizzle_block(b - it.block_start, swz < lb ? swz : lb), lds);
-}
-
 }  // namespace
 
 hipError_t launch_gate_pass(void* psi, Prec prec, int n_qubits, const GatePass& pass, const GateStage* stages,
@@ -624,22 +603,6 @@ hipError_t launch_gate_pass(void* psi, Prec prec, int n_qubits, const GatePass& 
           hipLaunchKernelGGL((k_gate_pass<float>), grid_2d(blocks), dim3(kGateThreads), 0, s,
                              static_cast<float2*>(psi), pass, stages, static_cast<const GateOp<float>*>(ops), swz,
                              blocks);
-     return hipGetLastError();
-}
-
-hipError_t launch_gate_items(void* arena, Prec prec, const GateItem* items, int nitems, const GateStage* stages,
-                             const void* ops, uint64_t total_blocks, hipStream_t s)
-{
-     if (nitems <= 0 || total_blocks == 0) return hipSuccess;
-     const int swz = get_block_swizzle();
-     if (prec == Prec::C128)
-          hipLaunchKernelGGL((k_gate_items<double>), grid_2d(total_blocks), dim3(kGateThreads), 0, s,
-                             static_cast<double2*>(arena), items, nitems, stages,
-                             static_cast<const GateOp<double>*>(ops), swz, total_blocks);
-     else
-          hipLaunchKernelGGL((k_gate_items<float>), grid_2d(total_blocks), dim3(kGateThreads), 0, s,
-                             static_cast<float2*>(arena), items, nitems, stages,
-                             static_cast<const GateOp<float>*>(ops), swz, total_blocks);
      return hipGetLastError();
 }
 

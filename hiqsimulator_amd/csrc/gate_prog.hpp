@@ -41,6 +41,15 @@ constexpr int kGateThreads = 1 << kGateThr;
 constexpr int gate_reg(Prec p) { return p == Prec::C128 ? 4 : 5; }
 constexpr int gate_tile_bits(Prec p) { return kGateThr + gate_reg(p); }
 constexpr int gate_high(Prec p) { return gate_tile_bits(p) - kGateLow; }  // chosen bits
+// Smallest states that run as gate programs.  Complex128: from one tile on.
+// The kernels alone cross over at 21 qubits (20 random layers: 224 against
+// 166 us at 16 qubits, 315 against 280 at 20, 368 against 436 at 21, 8.2
+// against 11.5 ms at 26), where the tiles fill the chip; below that a call is
+// bound by its host work, which is less (703 against 877 us a call at 16
+// qubits, 1189 against 1265 at 20).  Complex64 keeps the tile programs there:
+// their kernels are ahead by more (20 qubits: 221 against 314 us; 22: 459
+// against 403).
+constexpr int gate_min_qubits(Prec p) { return p == Prec::C128 ? 13 : 21; }
 constexpr int kGateMaxReg = 5, kGateMaxTile = kGateThr + kGateMaxReg, kGateMaxHigh = kGateMaxTile - kGateLow;
 constexpr size_t kGateMaxStages = 255;      // a pass's stage count is a byte
 constexpr size_t kGateMaxStageUnits = 512;  // and a stage's record count 16 bits
@@ -117,15 +126,6 @@ struct GatePass {
      uint32_t stage_first;
 };
 static_assert(sizeof(GatePass) == 44, "record size");
-
-// One pass of one state inside a launch over many states.
-struct GateItem {
-     uint64_t state_off;    // first amplitude of the state
-     uint64_t block_start;  // first workgroup
-     uint32_t log_blocks;   // log2 of its tiles
-     GatePass pass;
-};
-static_assert(sizeof(GateItem) == 64, "record size");
 
 // Slot of tile rank r in LDS, as an XOR mask over the slots: the low bits
 // hold the low rank bits XOR-ed with a linear map of the others.  64 banks of
@@ -208,8 +208,4 @@ void check_gate_pass(const GatePass& pass, const std::vector<GateStage>& stages,
 // device arrays, ops with one spare record at the end.
 hipError_t launch_gate_pass(void* psi, Prec prec, int n_qubits, const GatePass& pass, const GateStage* stages,
                             const void* ops, hipStream_t s);
-// The same for many states of one arena.
-hipError_t launch_gate_items(void* arena, Prec prec, const GateItem* items, int nitems, const GateStage* stages,
-                             const void* ops, uint64_t total_blocks, hipStream_t s);
-
 }  // namespace hq

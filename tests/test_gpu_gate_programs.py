@@ -40,7 +40,7 @@ def oracle_state(oracle_mod, n, gates):
     return o.get_state()
 
 
-@pytest.mark.parametrize("n", [12, 13, 14, 15, 17])
+@pytest.mark.parametrize("n", [12, 13, 14, 15, 17, 20, 21])
 @pytest.mark.parametrize("flow", ["tiled", "run"])
 def test_gate_programs_match_oracle(engine_mod, oracle_mod, n, flow):
     gates = gates_of(n, 64, 40 + n)
