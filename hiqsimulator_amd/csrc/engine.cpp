@@ -1152,6 +1152,12 @@ Engine::ProgSlot& Engine::program_slot(size_t need)
      return ps;
 }
 
+void Engine::program_done(ProgSlot& ps)
+{
+     check(hipEventRecord(ps.ev, stream_), "hipEventRecord");
+     ps.busy = true;
+}
+
 bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes)
 {
      passes = 0;
@@ -1187,8 +1193,7 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes)
                end_timed();
                ++passes;
           }
-          check(hipEventRecord(ps.ev, stream_), "hipEventRecord");
-          ps.busy = true;
+          program_done(ps);
      }
      std::vector<PosGate> rest;
      rest.reserve(planner.remaining().size());
@@ -1277,8 +1282,7 @@ int Engine::tile_items(std::vector<PosGate>& items, int op_width, size_t keep)
                 "tile pass");
           end_timed();
      }
-     check(hipEventRecord(ps.ev, stream_), "hipEventRecord");
-     ps.busy = true;
+     program_done(ps);
      // the launched items leave the list; the rest keep program order
      std::vector<PosGate> rest;
      rest.reserve(items.size());
@@ -1368,25 +1372,60 @@ cplx Engine::expectation(const std::vector<uint64_t>& xm, const std::vector<uint
                }
           return r;
      };
+     std::vector<PauliTermIn> list;
+     list.reserve(xm.size());
+     for (size_t t = 0; t < xm.size(); ++t)
+          list.push_back({to_bits(xm[t]), to_bits(zm[t]), coeff[t] * ipow(__builtin_popcountll(xm[t] & zm[t]))});
      cplx total(0.0, 0.0);
-     for (size_t t0 = 0; t0 < xm.size(); t0 += kMaxOuts / 2) {
-          const size_t t1 = std::min(xm.size(), t0 + kMaxOuts / 2);
+     if (n_qubits() >= kPauliMinQubits) {
+          // groups of terms in shared passes; what is left over goes below
+          PauliPlan plan = plan_pauli(list, n_qubits(), false);
+          list = std::move(plan.others);
+          if (!plan.passes.empty()) {
+               const PauliGroup* groups = nullptr;
+               const PauliTerm* terms = nullptr;
+               ProgSlot& ps = upload_pauli(plan, groups, terms);
+               for (size_t p0 = 0; p0 < plan.passes.size(); p0 += kMaxOuts / 2) {
+                    const size_t p1 = std::min(plan.passes.size(), p0 + kMaxOuts / 2);
+                    for (size_t p = p0; p < p1; ++p) {
+                         begin_timed(kPauli);
+                         check(launch_pauli_sum(d_state_, prec_, n_qubits(), plan.passes[p], groups, terms, d_scratch_,
+                                                d_scratch_ + kReduceScratchDoubles + 2 * (p - p0), stream_),
+                               "pauli_sum");
+                         end_timed();
+                    }
+                    read_out(h_out_, 2 * (p1 - p0));
+                    for (size_t p = 0; p < p1 - p0; ++p) total += cplx(h_out_[2 * p], h_out_[2 * p + 1]);
+               }
+               program_done(ps);
+          }
+     }
+     for (size_t t0 = 0; t0 < list.size(); t0 += kMaxOuts / 2) {
+          const size_t t1 = std::min(list.size(), t0 + kMaxOuts / 2);
           for (size_t t = t0; t < t1; ++t) {
                begin_timed(kPauli);
-               check(launch_pauli_expectation(d_state_, prec_, n_amps_, to_bits(xm[t]),
-                                              to_bits(zm[t]), d_scratch_,
-                                              d_scratch_ + kReduceScratchDoubles + 2 * (t - t0),
-                                              stream_),
+               check(launch_pauli_expectation(d_state_, prec_, n_amps_, list[t].x, list[t].z, d_scratch_,
+                                              d_scratch_ + kReduceScratchDoubles + 2 * (t - t0), stream_),
                      "pauli_expectation");
                end_timed();
           }
           read_out(h_out_, 2 * (t1 - t0));
-          for (size_t t = t0; t < t1; ++t) {
-               const cplx s(h_out_[2 * (t - t0)], h_out_[2 * (t - t0) + 1]);
-               total += coeff[t] * ipow(__builtin_popcountll(xm[t] & zm[t])) * s;
-          }
+          for (size_t t = t0; t < t1; ++t) total += list[t].c * cplx(h_out_[2 * (t - t0)], h_out_[2 * (t - t0) + 1]);
      }
      return total;
+}
+
+Engine::ProgSlot& Engine::upload_pauli(const PauliPlan& plan, const PauliGroup*& groups, const PauliTerm*& terms)
+{
+     const size_t gb = (plan.groups.size() * sizeof(PauliGroup) + 255) / 256 * 256;
+     const size_t need = gb + plan.terms.size() * sizeof(PauliTerm);
+     ProgSlot& ps = program_slot(need);
+     std::memcpy(ps.h, plan.groups.data(), plan.groups.size() * sizeof(PauliGroup));
+     std::memcpy(ps.h + gb, plan.terms.data(), plan.terms.size() * sizeof(PauliTerm));
+     check(hipMemcpyAsync(ps.d, ps.h, need, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync(pauli)");
+     groups = reinterpret_cast<const PauliGroup*>(ps.d);
+     terms = reinterpret_cast<const PauliTerm*>(ps.d + gb);
+     return ps;
 }
 
 void Engine::apply_pauli_sum(const std::vector<uint64_t>& xm, const std::vector<uint64_t>& zm,
@@ -1415,14 +1454,39 @@ void Engine::apply_pauli_sum(const std::vector<uint64_t>& xm, const std::vector<
      }
      settle();
      ensure_tmp(n_amps_);
-     begin_timed(kFillCopy);
-     check(launch_fill(d_tmp_, prec_, n_amps_, 0.0, 0.0, stream_), "fill");
-     end_timed();
-     for (size_t t = 0; t < xm.size(); ++t) {
-          const cplx c = coeff[t] * ipow(__builtin_popcountll(xm[t] & zm[t]));
+     std::vector<PauliTermIn> list;
+     list.reserve(xm.size());
+     for (size_t t = 0; t < xm.size(); ++t)
+          list.push_back({X[t], Z[t], coeff[t] * ipow(__builtin_popcountll(xm[t] & zm[t]))});
+     bool written = false;
+     if (n_qubits() >= kPauliMinQubits) {
+          PauliPlan plan = plan_pauli(list, n_qubits(), true);
+          list = std::move(plan.others);
+          if (!plan.passes.empty()) {
+               const PauliGroup* groups = nullptr;
+               const PauliTerm* terms = nullptr;
+               ProgSlot& ps = upload_pauli(plan, groups, terms);
+               for (const auto& p: plan.passes) {
+                    PauliApply a;
+                    a.src = d_state_;
+                    a.dst = d_tmp_;
+                    a.accumulate = written;
+                    begin_timed(kPauli);
+                    check(launch_pauli_apply(a, prec_, n_qubits(), p, groups, terms, stream_), "pauli_apply");
+                    end_timed();
+                    written = true;
+               }
+               program_done(ps);
+          }
+     }
+     if (!written) {
+          begin_timed(kFillCopy);
+          check(launch_fill(d_tmp_, prec_, n_amps_, 0.0, 0.0, stream_), "fill");
+          end_timed();
+     }
+     for (const auto& t: list) {
           begin_timed(kPauli);
-          check(launch_pauli_accumulate(d_tmp_, d_state_, prec_, n_amps_, X[t], Z[t], c.real(),
-                                        c.imag(), stream_),
+          check(launch_pauli_accumulate(d_tmp_, d_state_, prec_, n_amps_, t.x, t.z, t.c.real(), t.c.imag(), stream_),
                 "pauli_accumulate");
           end_timed();
      }
@@ -1492,29 +1556,91 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
      constexpr int kMaxTerms = 64;
      void* pw = w.p;
      void* po = out.p;
-     for (uint64_t s = 0; s < steps; ++s) {
-          check(launch_copy(po, pw, prec_, n_amps_, stream_), "copy");
-          void* pa = a.p;
-          void* pb = b.p;
-          check(launch_copy(pa, pw, prec_, n_amps_, stream_), "copy");
-          for (int k = 1; k <= kMaxTerms; ++k) {
-               // b = (-i tau / k) H a; out += b
-               const cplx f = cplx(0, -tau / k);
-               check(launch_fill(pb, prec_, n_amps_, 0.0, 0.0, stream_), "fill");
-               for (size_t j = 0; j < X.size(); ++j) {
-                    const cplx c = f * C[j];
-                    check(launch_pauli_accumulate(pb, pa, prec_, n_amps_, X[j], Z[j], c.real(), c.imag(), stream_),
-                          "pauli_accumulate");
+     PauliPlan plan;
+     if (n_qubits() >= kPauliMinQubits) {
+          std::vector<PauliTermIn> list;
+          for (size_t j = 0; j < X.size(); ++j) list.push_back({X[j], Z[j], C[j]});
+          plan = plan_pauli(list, n_qubits(), true);
+     }
+     if (steps && !plan.passes.empty() && plan.others.empty()) {
+          // Term k of a step is one pass over the state per plan pass; the
+          // last one also adds it to the sum and takes its norm, on which the
+          // following terms decide on the device whether they are still
+          // needed.  The host queues as many terms as could be: with norm
+          // bound (tau l1)^k / k! |psi| they are below the limit from there on.
+          double* const outs = d_scratch_ + kReduceScratchDoubles;
+          check(launch_masked_norm(pw, prec_, n_qubits(), 0, 0, d_scratch_, outs, stream_), "norm");
+          read_out(h_out_, 1);
+          bool hermitian = true;
+          for (const auto& c: coeff) hermitian = hermitian && c.imag() == 0.0;
+          const double xl = std::abs(tau) * l1;
+          const PauliGroup* groups = nullptr;
+          const PauliTerm* terms = nullptr;
+          ProgSlot& ps = upload_pauli(plan, groups, terms);
+          for (uint64_t s = 0; s < steps; ++s) {
+               // (a step of a sum that is not Hermitian grows the norm by at most e^xl)
+               const double log_norm = 0.5 * std::log(h_out_[0]) + (hermitian ? 0.1 : xl * static_cast<double>(s + 1));
+               int last = kMaxTerms;
+               for (int k = 1; k < kMaxTerms; ++k)
+                    if (log_norm + k * std::log(xl) - std::lgamma(k + 1.0) < std::log(1e-12) - 1.0) {
+                         last = k;
+                         break;
+                    }
+               void* src = pw;
+               void* dst = a.p;
+               for (int k = 1; k <= last; ++k) {
+                    // dst = (-i tau / k) H src; out (+)= dst
+                    for (size_t p = 0; p < plan.passes.size(); ++p) {
+                         PauliApply q;
+                         q.src = src;
+                         q.dst = dst;
+                         q.accumulate = p > 0;
+                         q.fr = 0;
+                         q.fi = -tau / k;
+                         if (k > 1) {
+                              q.skip = outs + (k - 1);
+                              q.skip_below = 1e-24;
+                         }
+                         if (p + 1 == plan.passes.size()) {
+                              q.o_src = k == 1 ? pw : po;
+                              q.o_dst = po;
+                              q.scratch = d_scratch_;
+                              q.norm = outs + k;
+                         }
+                         check(launch_pauli_apply(q, prec_, n_qubits(), plan.passes[p], groups, terms, stream_), "pauli_apply");
+                    }
+                    src = dst;
+                    dst = dst == a.p ? b.p : a.p;
                }
-               check(launch_pauli_accumulate(po, pb, prec_, n_amps_, 0, 0, 1.0, 0.0, stream_), "accumulate");
-               check(launch_masked_norm(pb, prec_, n_qubits(), 0, 0, d_scratch_, d_scratch_ + kReduceScratchDoubles,
-                                        stream_),
-                     "norm");
-               read_out(h_out_, 1);
-               std::swap(pa, pb);
-               if (h_out_[0] < 1e-24) break;
+               std::swap(pw, po);
           }
-          std::swap(pw, po);
+          program_done(ps);
+     }
+     else {
+          for (uint64_t s = 0; s < steps; ++s) {
+               check(launch_copy(po, pw, prec_, n_amps_, stream_), "copy");
+               void* pa = a.p;
+               void* pb = b.p;
+               check(launch_copy(pa, pw, prec_, n_amps_, stream_), "copy");
+               for (int k = 1; k <= kMaxTerms; ++k) {
+                    // b = (-i tau / k) H a; out += b
+                    const cplx f = cplx(0, -tau / k);
+                    check(launch_fill(pb, prec_, n_amps_, 0.0, 0.0, stream_), "fill");
+                    for (size_t j = 0; j < X.size(); ++j) {
+                         const cplx c = f * C[j];
+                         check(launch_pauli_accumulate(pb, pa, prec_, n_amps_, X[j], Z[j], c.real(), c.imag(), stream_),
+                               "pauli_accumulate");
+                    }
+                    check(launch_pauli_accumulate(po, pb, prec_, n_amps_, 0, 0, 1.0, 0.0, stream_), "accumulate");
+                    check(launch_masked_norm(pb, prec_, n_qubits(), 0, 0, d_scratch_, d_scratch_ + kReduceScratchDoubles,
+                                             stream_),
+                          "norm");
+                    read_out(h_out_, 1);
+                    std::swap(pa, pb);
+                    if (h_out_[0] < 1e-24) break;
+               }
+               std::swap(pw, po);
+          }
      }
      if (c0 != cplx(0, 0)) {
           const cplx ph = std::exp(cplx(0, -t) * c0);

@@ -20,6 +20,7 @@
 
 #include "fusion.hpp"
 #include "kernels.hpp"
+#include "pauli_prog.hpp"
 
 namespace hq {
 
@@ -205,6 +206,10 @@ private:
      // kProgSlots groups ago.
      struct ProgSlot;
      ProgSlot& program_slot(size_t bytes);
+     // Uploads the plan of a Pauli sum into a staging slot; program_done()
+     // after the launches that use it.
+     ProgSlot& upload_pauli(const PauliPlan& plan, const PauliGroup*& groups, const PauliTerm*& terms);
+     void program_done(ProgSlot& ps);
      void release_buffer(void*& p);
      void collect_retired();
      // A same-size out-of-place result in d_tmp_ becomes the state: the

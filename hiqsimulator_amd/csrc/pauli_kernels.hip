@@ -1,0 +1,322 @@
+// gfx950 kernels of the planned Pauli sums (pauli_prog.hpp).
+//
+// Bound: HBM for a few groups a pass (one read of the state; apply: a read
+// and one or two writes more), vector issue beyond about twenty terms.
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "device_common.hpp"
+#include "pauli_prog.hpp"
+
+namespace hq {
+namespace {
+
+template <typename T>
+__device__ __forceinline__ T load_words(const T* __restrict__ p)
+{
+     constexpr int N = sizeof(T) / 4;
+     const uint32_t* const q = reinterpret_cast<const uint32_t*>(p);
+     uint32_t w[N];
+#pragma unroll
+     for (int i = 0; i < N; ++i) w[i] = q[i];
+     T r;
+     __builtin_memcpy(&r, w, sizeof(T));
+     return r;
+}
+
+// Where a tile lies and where a thread's amplitudes lie in it: amplitude k of
+// thread t is tile rank index k * 512 + t.
+template <int A>
+struct TileAt {
+     static constexpr int KB = A == 8 ? 3 : (A == 4 ? 2 : (A == 2 ? 1 : 0));
+     static constexpr int H = kPauliThr + KB - kPauliLow;
+     uint64_t lane;   // index bits of the thread
+     uint64_t reg[A]; // index bits of the amplitude number (uniform)
+
+     __device__ __forceinline__ TileAt(const PauliPass& P, uint32_t tid)
+     {
+          lane = tid & ((1u << kPauliLow) - 1u);
+#pragma unroll
+          for (int j = 0; j < kPauliThr - kPauliLow; ++j)
+               lane |= static_cast<uint64_t>((tid >> (kPauliLow + j)) & 1u) << P.hpos[j];
+#pragma unroll
+          for (int k = 0; k < A; ++k) {
+               uint64_t o = 0;
+#pragma unroll
+               for (int j = 0; j < KB; ++j) o |= static_cast<uint64_t>((k >> j) & 1) << P.hpos[kPauliThr - kPauliLow + j];
+               reg[k] = o;
+          }
+     }
+     __device__ __forceinline__ uint64_t base(const PauliPass& P, uint64_t tix) const
+     {
+          uint64_t b = tix << kPauliLow;
+#pragma unroll
+          for (int j = 0; j < H; ++j) {
+               const uint64_t lo = b & ((1ull << P.hpos[j]) - 1ull);
+               b = ((b ^ lo) << 1) | lo;
+          }
+          return b;
+     }
+};
+
+// w[k] = sum over the group's terms of c (-1)^{|i & z|} for amplitude k.  The
+// sign splits into the tile's (uniform), the thread's and the amplitude
+// number's (uniform, as a factor +-1).
+template <int A>
+__device__ __forceinline__ void weights(double (&w)[A], const PauliTerm* __restrict__ terms, const PauliGroup& g,
+                                        uint64_t base, uint32_t tid)
+{
+#pragma unroll
+     for (int k = 0; k < A; ++k) w[k] = 0;
+     PauliTerm cur = load_words(terms + g.first);
+     for (uint32_t t = 0; t < g.count; ++t) {
+          asm volatile("" : "+s"(cur.z_tile));
+          __builtin_amdgcn_sched_barrier(0);
+          const PauliTerm nxt = load_words(terms + g.first + t + 1);  // (one spare record at the end)
+          const uint32_t uni = static_cast<uint32_t>(__popcll(base & cur.z_out));
+          const uint32_t sgn = (__popc(tid & cur.z_tile & (kPauliThreads - 1u)) + uni) << 31;
+          const double c = __hiloint2double(__double2hiint(cur.c) ^ static_cast<int>(sgn), __double2loint(cur.c));
+          const uint32_t zk = cur.z_tile >> kPauliThr;
+#pragma unroll
+          for (int k = 0; k < A; ++k) {
+               const double s = __hiloint2double(0x3ff00000 | static_cast<int>(__popc(static_cast<uint32_t>(k) & zk) << 31), 0);
+               w[k] = fma(c, s, w[k]);
+          }
+          cur = nxt;
+     }
+}
+
+template <typename R, int A>
+__global__ void __launch_bounds__(kPauliThreads)
+    k_pauli_sum(const VT<R>* __restrict__ psi, const PauliPass P, const PauliGroup* __restrict__ groups,
+                const PauliTerm* __restrict__ terms, const uint64_t ntiles, double* __restrict__ partials)
+{
+     using V = VT<R>;
+     __shared__ V tile[kPauliThreads * A];
+     const uint32_t tid = threadIdx.x;
+     const TileAt<A> at(P, tid);
+     double acc[2] = {0.0, 0.0};
+     for (uint64_t tix = blockIdx.x; tix < ntiles; tix += gridDim.x) {
+          const uint64_t base = at.base(P, tix);
+          V x[A];
+#pragma unroll
+          for (int k = 0; k < A; ++k) x[k] = ld_nt(psi + base + at.lane + at.reg[k]);
+          __syncthreads();  // the previous tile has been read
+#pragma unroll
+          for (int k = 0; k < A; ++k) tile[k * kPauliThreads + tid] = x[k];
+          __syncthreads();
+          for (uint32_t g = 0; g < P.ngroups; ++g) {
+               const PauliGroup G = load_words(groups + P.group_first + g);
+               double w[A];
+               weights<A>(w, terms, G, base, tid);
+               double s = 0;
+#pragma unroll
+               for (int k = 0; k < A; ++k) {
+                    const V y = tile[(k * kPauliThreads + tid) ^ G.x];
+                    const double yr = y.x, yi = y.y, xr = x[k].x, xi = x[k].y;
+                    const double q = (G.kind & 1u) ? yr * xi - yi * xr : yr * xr + yi * xi;
+                    s = fma(w[k], q, s);
+               }
+               if (G.kind & 2u) acc[1] += s;
+               else acc[0] += s;
+          }
+     }
+     // wave sums, then one partial a block
+     __shared__ double red[2][kPauliThreads / 64];
+#pragma unroll
+     for (int o = 0; o < 2; ++o) {
+          double v = acc[o];
+          for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+          if ((tid & 63) == 0) red[o][tid >> 6] = v;
+     }
+     __syncthreads();
+     if (tid < 2) {
+          double v = 0;
+          for (int i = 0; i < kPauliThreads / 64; ++i) v += red[tid][i];
+          partials[tid * gridDim.x + blockIdx.x] = v;
+     }
+}
+
+// Sum of the partials of NOUT outputs; with skip (below) the old value stays.
+__global__ void __launch_bounds__(kBlock)
+    k_sum_partials(const double* __restrict__ partials, const int nblocks, double* __restrict__ out,
+                   const double* __restrict__ skip, const double skip_below)
+{
+     const int o = blockIdx.x;
+     if (skip && skip[0] < skip_below) {
+          if (threadIdx.x == 0) out[o] = skip[0];
+          return;
+     }
+     double v = 0;
+     for (int i = threadIdx.x; i < nblocks; i += kBlock) v += partials[o * nblocks + i];
+     for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+     __shared__ double red[kBlock / 64];
+     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+     __syncthreads();
+     if (threadIdx.x == 0) {
+          double s = 0;
+          for (int i = 0; i < kBlock / 64; ++i) s += red[i];
+          out[o] = s;
+     }
+}
+
+template <typename R>
+struct ApplyArgs {
+     const VT<R>* src;
+     VT<R>* dst;
+     const VT<R>* o_src;
+     VT<R>* o_dst;
+     const double* skip;
+     double skip_below;
+     R fr, fi;
+     int accumulate;
+};
+
+template <typename R, int A>
+__global__ void __launch_bounds__(kPauliThreads)
+    k_pauli_apply(const ApplyArgs<R> a, const PauliPass P, const PauliGroup* __restrict__ groups,
+                  const PauliTerm* __restrict__ terms, const uint64_t ntiles, double* __restrict__ partials)
+{
+     using V = VT<R>;
+     if (a.skip && a.skip[0] < a.skip_below) return;  // the whole grid
+     __shared__ V tile[kPauliThreads * A];
+     const uint32_t tid = threadIdx.x;
+     const TileAt<A> at(P, tid);
+     double norm = 0;
+     for (uint64_t tix = blockIdx.x; tix < ntiles; tix += gridDim.x) {
+          const uint64_t base = at.base(P, tix);
+          V o[A];
+#pragma unroll
+          for (int k = 0; k < A; ++k) o[k] = a.src[base + at.lane + at.reg[k]];
+          __syncthreads();  // the previous tile has been read
+#pragma unroll
+          for (int k = 0; k < A; ++k) {
+               tile[k * kPauliThreads + tid] = o[k];
+               o[k].x = o[k].y = 0;
+          }
+          __syncthreads();
+          for (uint32_t g = 0; g < P.ngroups; ++g) {
+               const PauliGroup G = load_words(groups + P.group_first + g);
+               double w[A];
+               weights<A>(w, terms, G, base, tid);
+               const bool im = G.kind & 1u;
+#pragma unroll
+               for (int k = 0; k < A; ++k) {
+                    const V y = tile[(k * kPauliThreads + tid) ^ G.x];
+                    const R v = static_cast<R>(w[k]);
+                    // times v, or times i v
+                    o[k].x = fma(v, im ? -y.y : y.x, o[k].x);
+                    o[k].y = fma(v, im ? y.x : y.y, o[k].y);
+               }
+          }
+#pragma unroll
+          for (int k = 0; k < A; ++k) {
+               const uint64_t i = base + at.lane + at.reg[k];
+               V b;
+               b.x = fma(-a.fi, o[k].y, a.fr * o[k].x);
+               b.y = fma(a.fi, o[k].x, a.fr * o[k].y);
+               if (a.accumulate) {
+                    const V d = a.dst[i];
+                    b.x += d.x;
+                    b.y += d.y;
+               }
+               a.dst[i] = b;
+               if (a.o_dst) {
+                    V s = a.o_src[i];
+                    s.x += b.x;
+                    s.y += b.y;
+                    a.o_dst[i] = s;
+                    const double br = b.x, bi = b.y;
+                    norm += br * br + bi * bi;
+               }
+          }
+     }
+     if (!a.o_dst) return;
+     for (int d = 32; d > 0; d >>= 1) norm += __shfl_xor(norm, d, 64);
+     __shared__ double red[kPauliThreads / 64];
+     if ((tid & 63) == 0) red[tid >> 6] = norm;
+     __syncthreads();
+     if (tid == 0) {
+          double v = 0;
+          for (int i = 0; i < kPauliThreads / 64; ++i) v += red[i];
+          partials[blockIdx.x] = v;
+     }
+}
+
+bool pass_fits(const PauliPass& p, int n)
+{
+     if (n < kPauliMinQubits || n > 40) return false;
+     const int H = pauli_tile_bits(n) - kPauliLow;
+     for (int j = 0; j < H; ++j)
+          if (p.hpos[j] < kPauliLow || p.hpos[j] >= n || (j && p.hpos[j] <= p.hpos[j - 1])) return false;
+     return true;
+}
+
+template <typename R, int A>
+void sum_launch(const void* psi, const PauliPass& p, const PauliGroup* g, const PauliTerm* t, uint64_t ntiles, int grid,
+                double* scratch, hipStream_t s)
+{
+     hipLaunchKernelGGL((k_pauli_sum<R, A>), dim3(grid), dim3(kPauliThreads), 0, s, static_cast<const VT<R>*>(psi), p, g,
+                        t, ntiles, scratch);
+}
+template <typename R, int A>
+void apply_launch(const PauliApply& a, const PauliPass& p, const PauliGroup* g, const PauliTerm* t, uint64_t ntiles,
+                  int grid, hipStream_t s)
+{
+     ApplyArgs<R> k{};
+     k.src = static_cast<const VT<R>*>(a.src);
+     k.dst = static_cast<VT<R>*>(a.dst);
+     k.o_src = static_cast<const VT<R>*>(a.o_src);
+     k.o_dst = static_cast<VT<R>*>(a.o_dst);
+     k.skip = a.skip;
+     k.skip_below = a.skip_below;
+     k.fr = static_cast<R>(a.fr);
+     k.fi = static_cast<R>(a.fi);
+     k.accumulate = a.accumulate ? 1 : 0;
+     hipLaunchKernelGGL((k_pauli_apply<R, A>), dim3(grid), dim3(kPauliThreads), 0, s, k, p, g, t, ntiles, a.scratch);
+}
+
+// f<A>() for the amplitudes a thread of an n-qubit state's tile holds.
+#define HQ_PAULI(RR, CALL)                                  \
+     switch (pauli_tile_bits(n) - kPauliThr) {              \
+          case 0: { using R = RR; constexpr int A = 1; CALL; } break; \
+          case 1: { using R = RR; constexpr int A = 2; CALL; } break; \
+          case 2: { using R = RR; constexpr int A = 4; CALL; } break; \
+          default: { using R = RR; constexpr int A = 8; CALL; } break; \
+     }
+
+}  // namespace
+
+hipError_t launch_pauli_sum(const void* psi, Prec prec, int n, const PauliPass& pass, const PauliGroup* groups,
+                            const PauliTerm* terms, double* scratch, double* out, hipStream_t s)
+{
+     if (!pass_fits(pass, n)) return hipErrorInvalidValue;
+     const uint64_t ntiles = 1ull << (n - pauli_tile_bits(n));
+     const int grid = static_cast<int>(ntiles < kReduceBlocks ? ntiles : kReduceBlocks);
+     if (prec == Prec::C128) HQ_PAULI(double, (sum_launch<R, A>(psi, pass, groups, terms, ntiles, grid, scratch, s)))
+     else HQ_PAULI(float, (sum_launch<R, A>(psi, pass, groups, terms, ntiles, grid, scratch, s)))
+     const hipError_t e = hipGetLastError();
+     if (e != hipSuccess) return e;
+     hipLaunchKernelGGL(k_sum_partials, dim3(2), dim3(kBlock), 0, s, scratch, grid, out, nullptr, 0.0);
+     return hipGetLastError();
+}
+
+hipError_t launch_pauli_apply(const PauliApply& a, Prec prec, int n, const PauliPass& pass, const PauliGroup* groups,
+                              const PauliTerm* terms, hipStream_t s)
+{
+     if (!pass_fits(pass, n) || a.src == a.dst || (a.o_dst && (!a.o_src || !a.scratch || !a.norm)))
+          return hipErrorInvalidValue;
+     const uint64_t ntiles = 1ull << (n - pauli_tile_bits(n));
+     const int grid = static_cast<int>(ntiles < kReduceBlocks ? ntiles : kReduceBlocks);
+     if (prec == Prec::C128) HQ_PAULI(double, (apply_launch<R, A>(a, pass, groups, terms, ntiles, grid, s)))
+     else HQ_PAULI(float, (apply_launch<R, A>(a, pass, groups, terms, ntiles, grid, s)))
+     const hipError_t e = hipGetLastError();
+     if (e != hipSuccess || !a.o_dst) return e;
+     hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kBlock), 0, s, a.scratch, grid, a.norm, a.skip, a.skip_below);
+     return hipGetLastError();
+}
+
+#undef HQ_PAULI
+
+}  // namespace hq

@@ -1,0 +1,108 @@
+// Planning of Pauli sums.  See pauli_prog.hpp.
+#include "pauli_prog.hpp"
+
+#include <map>
+#include <tuple>
+
+namespace hq {
+
+namespace {
+inline int popc(uint64_t x) { return __builtin_popcountll(x); }
+}  // namespace
+
+PauliPlan plan_pauli(const std::vector<PauliTermIn>& in, int n, bool apply)
+{
+     PauliPlan plan;
+     const int T = pauli_tile_bits(n), H = T - kPauliLow;
+     const uint64_t low = (uint64_t(1) << kPauliLow) - 1;
+     // real coefficients by (x, kind); terms of one x stay in list order
+     struct Z {
+          uint64_t z;
+          double c;
+     };
+     std::vector<uint64_t> xs;  // in order of first use
+     std::map<std::pair<uint64_t, uint32_t>, std::vector<Z>> by;
+     std::map<uint64_t, bool> known;
+     for (const auto& t: in) {
+          if (popc(t.x & ~low) > H) {
+               plan.others.push_back(t);
+               continue;
+          }
+          // Expectation: the pair i, i ^ x of a term adds twice the real part
+          // of conj(psi[i ^ x]) psi[i] when |x & z| is even, twice i times
+          // its imaginary part when it is odd.  Apply: the sign at the source
+          // i = j ^ x is the one at j times (-1)^{|x & z|}.
+          const bool odd = popc(t.x & t.z) & 1;
+          std::complex<double> c = t.c;
+          uint32_t kind = 0;
+          if (apply) {
+               if (odd) c = -c;
+          }
+          else if (odd) {
+               kind = 1;
+               c = std::complex<double>(-c.imag(), c.real());
+          }
+          if (known.emplace(t.x, true).second) xs.push_back(t.x);
+          // real part of the coefficient, then its imaginary part
+          if (!(c.real() == 0.0)) by[{t.x, kind}].push_back(Z{t.z, c.real()});
+          if (!(c.imag() == 0.0)) by[{t.x, apply ? 1u : kind | 2u}].push_back(Z{t.z, c.imag()});
+     }
+     std::vector<uint64_t> left;
+     bool diagonal = false;
+     for (uint64_t x: xs) {
+          if (x) left.push_back(x);
+          else diagonal = true;
+     }
+     while (!left.empty() || diagonal) {
+          // the first x left, then always the one that needs the fewest new bits
+          uint64_t bits = low;
+          std::vector<uint64_t> here;
+          if (diagonal) here.push_back(0);
+          diagonal = false;
+          for (;;) {
+               int best = -1, need = H + 1;
+               for (size_t i = 0; i < left.size(); ++i) {
+                    const int k = popc(left[i] & ~bits);
+                    if (popc(bits | left[i]) <= T && k < need) {
+                         need = k;
+                         best = static_cast<int>(i);
+                         if (k == 0) break;
+                    }
+               }
+               if (best < 0) break;
+               bits |= left[best];
+               here.push_back(left[best]);
+               left.erase(left.begin() + best);
+          }
+          for (int p = 0; p < n && popc(bits) < T; ++p) bits |= uint64_t(1) << p;
+          int rank[64], r = 0;
+          PauliPass pass{};
+          for (int p = 0; p < 64; ++p) {
+               rank[p] = -1;
+               if (!((bits >> p) & 1)) continue;
+               if (r >= kPauliLow) pass.hpos[r - kPauliLow] = static_cast<uint8_t>(p);
+               rank[p] = r++;
+          }
+          auto to_tile = [&](uint64_t m) {
+               uint32_t t = 0;
+               for (uint64_t b = m & bits; b; b &= b - 1) t |= 1u << rank[__builtin_ctzll(b)];
+               return t;
+          };
+          pass.group_first = static_cast<uint32_t>(plan.groups.size());
+          for (uint64_t x: here)
+               for (uint32_t kind = 0; kind < 4; ++kind) {
+                    const auto it = by.find({x, kind});
+                    if (it == by.end()) continue;
+                    PauliGroup g{to_tile(x), kind, static_cast<uint32_t>(plan.terms.size()),
+                                 static_cast<uint32_t>(it->second.size())};
+                    for (const Z& z: it->second) plan.terms.push_back(PauliTerm{z.z & ~bits, to_tile(z.z), 0, z.c});
+                    plan.groups.push_back(g);
+               }
+          pass.ngroups = static_cast<uint32_t>(plan.groups.size()) - pass.group_first;
+          plan.passes.push_back(pass);
+     }
+     plan.terms.push_back(PauliTerm{0, 0, 0, 0.0});
+     return plan;
+}
+
+}  // namespace hq

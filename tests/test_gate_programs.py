@@ -1,6 +1,6 @@
-"""Gate programs on the host: the unit splitter, the planner and the compiler
-against a plain interpreter of the compiled records (tests/native/
-gate_prog_test.cpp), built with g++ under AddressSanitizer and
+"""Gate programs and Pauli sums on the host: the unit splitter, the planners and the compiler
+against plain interpreters of the compiled records (tests/native/
+gate_prog_test.cpp, pauli_prog_test.cpp), built with g++ under AddressSanitizer and
 UndefinedBehaviorSanitizer."""
 import os
 import subprocess
@@ -12,13 +12,14 @@ CSRC = os.path.join(os.path.dirname(HERE), "hiqsimulator_amd", "csrc")
 SAN = ["-fsanitize=address,undefined", "-fno-sanitize-recover=all", "-fno-omit-frame-pointer"]
 
 
-def test_gate_programs_under_sanitizers(tmp_path):
+@pytest.mark.parametrize("unit,said", [("gate_prog", "gate programs ok"), ("pauli_prog", "pauli plans ok")])
+def test_programs_under_sanitizers(tmp_path, unit, said):
     hip_inc = "/opt/rocm/include"
     if not os.path.isdir(os.path.join(hip_inc, "hip")):
         pytest.skip("HIP headers not installed")
-    exe = str(tmp_path / "gate_prog_test")
+    exe = str(tmp_path / (unit + "_test"))
     subprocess.run(["g++", "-O1", "-g", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I" + hip_inc] + SAN +
-                   [os.path.join(CSRC, "gate_prog.cpp"), os.path.join(HERE, "native", "gate_prog_test.cpp"), "-o", exe],
+                   [os.path.join(CSRC, unit + ".cpp"), os.path.join(HERE, "native", unit + "_test.cpp"), "-o", exe],
                    check=True)
     out = subprocess.run([exe], capture_output=True, text=True, timeout=600)
-    assert out.returncode == 0 and "gate programs ok" in out.stdout, out.stdout[-2000:] + out.stderr[-4000:]
+    assert out.returncode == 0 and said in out.stdout, out.stdout[-2000:] + out.stderr[-4000:]
