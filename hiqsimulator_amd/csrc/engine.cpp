@@ -1382,14 +1382,13 @@ cplx Engine::expectation(const std::vector<uint64_t>& xm, const std::vector<uint
           PauliPlan plan = plan_pauli(list, n_qubits(), false);
           list = std::move(plan.others);
           if (!plan.passes.empty()) {
-               const PauliGroup* groups = nullptr;
                const PauliTerm* terms = nullptr;
-               ProgSlot& ps = upload_pauli(plan, groups, terms);
+               ProgSlot& ps = upload_pauli(plan, terms);
                for (size_t p0 = 0; p0 < plan.passes.size(); p0 += kMaxOuts / 2) {
                     const size_t p1 = std::min(plan.passes.size(), p0 + kMaxOuts / 2);
                     for (size_t p = p0; p < p1; ++p) {
                          begin_timed(kPauli);
-                         check(launch_pauli_sum(d_state_, prec_, n_qubits(), plan.passes[p], groups, terms, d_scratch_,
+                         check(launch_pauli_sum(d_state_, prec_, n_qubits(), plan.passes[p], terms, d_scratch_,
                                                 d_scratch_ + kReduceScratchDoubles + 2 * (p - p0), stream_),
                                "pauli_sum");
                          end_timed();
@@ -1415,16 +1414,13 @@ cplx Engine::expectation(const std::vector<uint64_t>& xm, const std::vector<uint
      return total;
 }
 
-Engine::ProgSlot& Engine::upload_pauli(const PauliPlan& plan, const PauliGroup*& groups, const PauliTerm*& terms)
+Engine::ProgSlot& Engine::upload_pauli(const PauliPlan& plan, const PauliTerm*& terms)
 {
-     const size_t gb = (plan.groups.size() * sizeof(PauliGroup) + 255) / 256 * 256;
-     const size_t need = gb + plan.terms.size() * sizeof(PauliTerm);
+     const size_t need = plan.terms.size() * sizeof(PauliTerm);
      ProgSlot& ps = program_slot(need);
-     std::memcpy(ps.h, plan.groups.data(), plan.groups.size() * sizeof(PauliGroup));
-     std::memcpy(ps.h + gb, plan.terms.data(), plan.terms.size() * sizeof(PauliTerm));
+     std::memcpy(ps.h, plan.terms.data(), need);
      check(hipMemcpyAsync(ps.d, ps.h, need, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync(pauli)");
-     groups = reinterpret_cast<const PauliGroup*>(ps.d);
-     terms = reinterpret_cast<const PauliTerm*>(ps.d + gb);
+     terms = reinterpret_cast<const PauliTerm*>(ps.d);
      return ps;
 }
 
@@ -1463,16 +1459,15 @@ void Engine::apply_pauli_sum(const std::vector<uint64_t>& xm, const std::vector<
           PauliPlan plan = plan_pauli(list, n_qubits(), true);
           list = std::move(plan.others);
           if (!plan.passes.empty()) {
-               const PauliGroup* groups = nullptr;
                const PauliTerm* terms = nullptr;
-               ProgSlot& ps = upload_pauli(plan, groups, terms);
+               ProgSlot& ps = upload_pauli(plan, terms);
                for (const auto& p: plan.passes) {
                     PauliApply a;
                     a.src = d_state_;
                     a.dst = d_tmp_;
-                    a.accumulate = written;
+                    if (written) a.add = d_tmp_;
                     begin_timed(kPauli);
-                    check(launch_pauli_apply(a, prec_, n_qubits(), p, groups, terms, stream_), "pauli_apply");
+                    check(launch_pauli_apply(a, prec_, n_qubits(), p, terms, stream_), "pauli_apply");
                     end_timed();
                     written = true;
                }
@@ -1537,12 +1532,81 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
      const size_t bytes = n_amps_ * amp_bytes(prec_);
      struct Buf {
           void* p = nullptr;
-          explicit Buf(size_t n) { check(hipMalloc(&p, n), "hipMalloc(time evolution)"); }
+          explicit Buf(size_t n)
+          {
+               if (n) check(hipMalloc(&p, n), "hipMalloc(time evolution)");
+          }
           ~Buf()
           {
                if (p) (void)hipFree(p);
           }
      };
+     PauliPlan plan;
+     if (n_qubits() >= kPauliMinQubits && !X.empty()) {
+          std::vector<PauliTermIn> list;
+          for (size_t j = 0; j < X.size(); ++j) list.push_back({X[j], Z[j], C[j]});
+          plan = plan_pauli(list, n_qubits(), true);
+     }
+     bool hermitian = true;
+     for (const auto& c: coeff) hermitian = hermitian && c.imag() == 0.0;
+     const double reach = std::abs(t) * l1;
+     if (hermitian && !plan.passes.empty() && plan.others.empty() && reach > 0 && reach <= 1e6) {
+          // Real coefficients: H / l1 has its spectrum in [-1, 1], and
+          // exp(-i z x) = J_0(z) + 2 sum_k (-i)^k J_k(z) T_k(x) with z = t l1
+          // takes about z + 20 products with H, where steps of a Taylor
+          // series take about 14 z.  T_{k+1} = 2 x T_k - T_{k-1} overwrites
+          // T_{k-1}: two vectors and the sum.
+          Buf t1(bytes), w_own(cmask ? bytes : 0), out_own(cmask ? bytes : 0);
+          if (!cmask) ensure_tmp(n_amps_);
+          void* const w = cmask ? w_own.p : d_state_;  // T_0, destroyed
+          void* const out = cmask ? out_own.p : d_tmp_;
+          if (cmask) {
+               check(launch_copy(w, d_state_, prec_, n_amps_, stream_), "copy");
+               check(launch_normalize(w, prec_, n_amps_, cmask, cmask, 1.0, stream_), "select");
+               check(launch_pauli_accumulate(d_state_, w, prec_, n_amps_, 0, 0, -1.0, 0.0, stream_), "subtract");
+          }
+          const std::vector<double> bes = bessel_series(reach);
+          const PauliTerm* terms = nullptr;
+          ProgSlot& ps = upload_pauli(plan, terms);
+          void* cur = w;
+          void* next = t1.p;
+          // (at least one product, so that the sum is formed)
+          for (size_t k = 1; k < std::max<size_t>(bes.size(), 2); ++k) {
+               for (size_t p = 0; p < plan.passes.size(); ++p) {
+                    PauliApply q;
+                    q.src = cur;
+                    q.dst = next;
+                    q.fr = (k == 1 ? 1.0 : 2.0) / l1;
+                    if (p > 0) {
+                         q.add = next;
+                    }
+                    else if (k > 1) {
+                         q.add = next;  // T_{k-2}
+                         q.g = -1.0;
+                    }
+                    if (p + 1 == plan.passes.size()) {
+                         q.o_src = k == 1 ? w : out;
+                         q.o_dst = out;
+                         q.h = k == 1 ? bes[0] : 1.0;
+                         // 2 J_k(z) (-i sign t)^k
+                         const cplx c = 2.0 * (k < bes.size() ? bes[k] : 0.0) * (t < 0 ? ipow(static_cast<int>(k & 3)) : ipow(static_cast<int>((4 - (k & 3)) & 3)));
+                         q.cr = c.real();
+                         q.ci = c.imag();
+                    }
+                    check(launch_pauli_apply(q, prec_, n_qubits(), plan.passes[p], terms, stream_), "pauli_apply");
+               }
+               std::swap(cur, next);
+          }
+          program_done(ps);
+          if (c0 != cplx(0, 0)) {
+               const cplx ph = std::exp(cplx(0, -t) * c0);
+               check(launch_scale(out, prec_, n_amps_, ph.real(), ph.imag(), stream_), "phase");
+          }
+          if (cmask) check(launch_pauli_accumulate(d_state_, out, prec_, n_amps_, 0, 0, 1.0, 0.0, stream_), "add");
+          else commit_tmp();
+          check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+          return;
+     }
      // w: the controlled part of the state, evolved step by step
      Buf w(bytes), out(bytes), a(bytes), b(bytes);
      check(launch_copy(w.p, d_state_, prec_, n_amps_, stream_), "copy");
@@ -1556,27 +1620,19 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
      constexpr int kMaxTerms = 64;
      void* pw = w.p;
      void* po = out.p;
-     PauliPlan plan;
-     if (n_qubits() >= kPauliMinQubits) {
-          std::vector<PauliTermIn> list;
-          for (size_t j = 0; j < X.size(); ++j) list.push_back({X[j], Z[j], C[j]});
-          plan = plan_pauli(list, n_qubits(), true);
-     }
      if (steps && !plan.passes.empty() && plan.others.empty()) {
           // Term k of a step is one pass over the state per plan pass; the
-          // last one also adds it to the sum and takes its norm, on which the
-          // following terms decide on the device whether they are still
-          // needed.  The host queues as many terms as could be: with norm
-          // bound (tau l1)^k / k! |psi| they are below the limit from there on.
+          // last one also adds it to the sum.  The host queues as many terms
+          // as could be needed: bounded by (tau l1)^k / k! |psi|, they are
+          // below the limit from there on.  The norms of the terms close to
+          // that, and of a few early ones, are taken, and the terms after them
+          // decide on the device whether they are still needed.
           double* const outs = d_scratch_ + kReduceScratchDoubles;
           check(launch_masked_norm(pw, prec_, n_qubits(), 0, 0, d_scratch_, outs, stream_), "norm");
           read_out(h_out_, 1);
-          bool hermitian = true;
-          for (const auto& c: coeff) hermitian = hermitian && c.imag() == 0.0;
           const double xl = std::abs(tau) * l1;
-          const PauliGroup* groups = nullptr;
           const PauliTerm* terms = nullptr;
-          ProgSlot& ps = upload_pauli(plan, groups, terms);
+          ProgSlot& ps = upload_pauli(plan, terms);
           for (uint64_t s = 0; s < steps; ++s) {
                // (a step of a sum that is not Hermitian grows the norm by at most e^xl)
                const double log_norm = 0.5 * std::log(h_out_[0]) + (hermitian ? 0.1 : xl * static_cast<double>(s + 1));
@@ -1588,27 +1644,30 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
                     }
                void* src = pw;
                void* dst = a.p;
+               const double* seen = nullptr;  // the last norm taken
                for (int k = 1; k <= last; ++k) {
+                    const bool take = k < last && (k + 4 >= last || k == 2 || k == 4 || k == 8);
                     // dst = (-i tau / k) H src; out (+)= dst
                     for (size_t p = 0; p < plan.passes.size(); ++p) {
                          PauliApply q;
                          q.src = src;
                          q.dst = dst;
-                         q.accumulate = p > 0;
+                         if (p > 0) q.add = dst;
                          q.fr = 0;
                          q.fi = -tau / k;
-                         if (k > 1) {
-                              q.skip = outs + (k - 1);
-                              q.skip_below = 1e-24;
-                         }
+                         q.skip = seen;
+                         q.skip_below = 1e-24;
                          if (p + 1 == plan.passes.size()) {
                               q.o_src = k == 1 ? pw : po;
                               q.o_dst = po;
-                              q.scratch = d_scratch_;
-                              q.norm = outs + k;
+                              if (take) {
+                                   q.scratch = d_scratch_;
+                                   q.norm = outs + k;
+                              }
                          }
-                         check(launch_pauli_apply(q, prec_, n_qubits(), plan.passes[p], groups, terms, stream_), "pauli_apply");
+                         check(launch_pauli_apply(q, prec_, n_qubits(), plan.passes[p], terms, stream_), "pauli_apply");
                     }
+                    if (take) seen = outs + k;
                     src = dst;
                     dst = dst == a.p ? b.p : a.p;
                }

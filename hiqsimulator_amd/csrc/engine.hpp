@@ -208,7 +208,7 @@ private:
      ProgSlot& program_slot(size_t bytes);
      // Uploads the plan of a Pauli sum into a staging slot; program_done()
      // after the launches that use it.
-     ProgSlot& upload_pauli(const PauliPlan& plan, const PauliGroup*& groups, const PauliTerm*& terms);
+     ProgSlot& upload_pauli(const PauliPlan& plan, const PauliTerm*& terms);
      void program_done(ProgSlot& ps);
      void release_buffer(void*& p);
      void collect_retired();

@@ -60,41 +60,74 @@ struct TileAt {
      }
 };
 
-// w[k] = sum over the group's terms of c (-1)^{|i & z|} for amplitude k.  The
-// sign splits into the tile's (uniform), the thread's and the amplitude
-// number's (uniform, as a factor +-1).
-template <int A>
-__device__ __forceinline__ void weights(double (&w)[A], const PauliTerm* __restrict__ terms, const PauliGroup& g,
-                                        uint64_t base, uint32_t tid)
+// The parity of k & zk as a factor +-1 (uniform).
+__device__ __forceinline__ double amp_sign(int k, uint32_t zk)
 {
+     return __hiloint2double(0x3ff00000 | static_cast<int>(__popc(static_cast<uint32_t>(k) & zk) << 31), 0);
+}
+
+// Runs the records of a pass on one tile: done(t, w) for every group, t its
+// last record and w[k] = sum over its terms of c (-1)^{|i & z|} for amplitude
+// k.  The sign splits into the tile's (uniform), the thread's and the
+// amplitude number's (uniform).
+template <int A, typename Done>
+__device__ __forceinline__ void run_terms(const PauliTerm* __restrict__ terms, const uint32_t count, const uint64_t base,
+                                          const uint32_t tid, Done&& done)
+{
+     double w[A], v = 0;
 #pragma unroll
      for (int k = 0; k < A; ++k) w[k] = 0;
-     PauliTerm cur = load_words(terms + g.first);
-     for (uint32_t t = 0; t < g.count; ++t) {
+     PauliTerm cur = load_words(terms);
+     for (uint32_t t = 0; t < count; ++t) {
           asm volatile("" : "+s"(cur.z_tile));
           __builtin_amdgcn_sched_barrier(0);
-          const PauliTerm nxt = load_words(terms + g.first + t + 1);  // (one spare record at the end)
+          const PauliTerm nxt = load_words(terms + t + 1);  // (one spare record at the end)
           const uint32_t uni = static_cast<uint32_t>(__popcll(base & cur.z_out));
           const uint32_t sgn = (__popc(tid & cur.z_tile & (kPauliThreads - 1u)) + uni) << 31;
-          const double c = __hiloint2double(__double2hiint(cur.c) ^ static_cast<int>(sgn), __double2loint(cur.c));
-          const uint32_t zk = cur.z_tile >> kPauliThr;
+          v += __hiloint2double(__double2hiint(cur.c) ^ static_cast<int>(sgn), __double2loint(cur.c));
+          if (cur.z_tile & kPauliClassEnd) {
+               const uint32_t zk = (cur.z_tile & 0xffffu) >> kPauliThr;
 #pragma unroll
-          for (int k = 0; k < A; ++k) {
-               const double s = __hiloint2double(0x3ff00000 | static_cast<int>(__popc(static_cast<uint32_t>(k) & zk) << 31), 0);
-               w[k] = fma(c, s, w[k]);
+               for (int k = 0; k < A; ++k) w[k] = fma(v, amp_sign(k, zk), w[k]);
+               v = 0;
+               if (cur.z_tile & kPauliGroupEnd) {
+                    done(cur, w);
+#pragma unroll
+                    for (int k = 0; k < A; ++k) w[k] = 0;
+               }
           }
           cur = nxt;
      }
 }
 
+// sum_k w[k] Re or Im (conj(y_k) x_k), y the amplitude at i ^ x; KB >= 0: only
+// the amplitudes whose number has bit KB clear.
+template <int KB, typename V, int A>
+__device__ __forceinline__ double group_sum(const V (&x)[A], const double (&w)[A], const V* tile, uint32_t tid, uint32_t xm,
+                                            bool im)
+{
+     double s = 0;
+#pragma unroll
+     for (int k = 0; k < A; ++k) {
+          if (KB >= 0 && ((k >> (KB < 0 ? 0 : KB)) & 1)) continue;
+          const V y = tile[(k * kPauliThreads + tid) ^ xm];
+          const double yr = y.x, yi = y.y, xr = x[k].x, xi = x[k].y;
+          // uniform choice of the part
+          const double p = im ? xi : xr, q = im ? -xr : xi;
+          s = fma(w[k], fma(yr, p, yi * q), s);
+     }
+     return s;
+}
+
 template <typename R, int A>
 __global__ void __launch_bounds__(kPauliThreads)
-    k_pauli_sum(const VT<R>* __restrict__ psi, const PauliPass P, const PauliGroup* __restrict__ groups,
-                const PauliTerm* __restrict__ terms, const uint64_t ntiles, double* __restrict__ partials)
+    k_pauli_sum(const VT<R>* __restrict__ psi, const PauliPass P, const PauliTerm* __restrict__ terms,
+                const uint64_t ntiles, double* __restrict__ partials)
 {
      using V = VT<R>;
      __shared__ V tile[kPauliThreads * A];
      const uint32_t tid = threadIdx.x;
+     const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tid)));
      const TileAt<A> at(P, tid);
      double acc[2] = {0.0, 0.0};
      for (uint64_t tix = blockIdx.x; tix < ntiles; tix += gridDim.x) {
@@ -106,21 +139,30 @@ __global__ void __launch_bounds__(kPauliThreads)
 #pragma unroll
           for (int k = 0; k < A; ++k) tile[k * kPauliThreads + tid] = x[k];
           __syncthreads();
-          for (uint32_t g = 0; g < P.ngroups; ++g) {
-               const PauliGroup G = load_words(groups + P.group_first + g);
-               double w[A];
-               weights<A>(w, terms, G, base, tid);
+          run_terms<A>(terms + P.first, P.count, base, tid, [&](const PauliTerm& t, const double (&w)[A]) {
+               const bool im = t.z_tile & kPauliImag;
                double s = 0;
-#pragma unroll
-               for (int k = 0; k < A; ++k) {
-                    const V y = tile[(k * kPauliThreads + tid) ^ G.x];
-                    const double yr = y.x, yi = y.y, xr = x[k].x, xi = x[k].y;
-                    const double q = (G.kind & 1u) ? yr * xi - yi * xr : yr * xr + yi * xi;
-                    s = fma(w[k], q, s);
+               // the half that the highest bit of x selects (pauli_prog.cpp)
+               const uint32_t kx = t.x >> kPauliThr;
+               const uint32_t wx = t.x & ((1u << kPauliThr) - (1u << kPauliLane));
+               if (kx >= 4u) {
+                    if constexpr (A >= 8) s = group_sum<2>(x, w, tile, tid, t.x, im);
                }
-               if (G.kind & 2u) acc[1] += s;
+               else if (kx >= 2u) {
+                    if constexpr (A >= 4) s = group_sum<1>(x, w, tile, tid, t.x, im);
+               }
+               else if (kx) {
+                    if constexpr (A >= 2) s = group_sum<0>(x, w, tile, tid, t.x, im);
+               }
+               else if (wx) {
+                    if (!((wave >> (31 - __clz(static_cast<int>(wx)))) & 1u)) s = group_sum<-1>(x, w, tile, tid, t.x, im);
+               }
+               else {
+                    s = group_sum<-1>(x, w, tile, tid, t.x, im);
+               }
+               if (t.z_tile & kPauliOut1) acc[1] += s;
                else acc[0] += s;
-          }
+          });
      }
      // wave sums, then one partial a block
      __shared__ double red[2][kPauliThreads / 64];
@@ -165,18 +207,18 @@ template <typename R>
 struct ApplyArgs {
      const VT<R>* src;
      VT<R>* dst;
+     const VT<R>* add;
      const VT<R>* o_src;
      VT<R>* o_dst;
      const double* skip;
      double skip_below;
-     R fr, fi;
-     int accumulate;
+     R fr, fi, g, h, cr, ci;
 };
 
 template <typename R, int A>
 __global__ void __launch_bounds__(kPauliThreads)
-    k_pauli_apply(const ApplyArgs<R> a, const PauliPass P, const PauliGroup* __restrict__ groups,
-                  const PauliTerm* __restrict__ terms, const uint64_t ntiles, double* __restrict__ partials)
+    k_pauli_apply(const ApplyArgs<R> a, const PauliPass P, const PauliTerm* __restrict__ terms,
+                  const uint64_t ntiles, double* __restrict__ partials)
 {
      using V = VT<R>;
      if (a.skip && a.skip[0] < a.skip_below) return;  // the whole grid
@@ -196,43 +238,40 @@ __global__ void __launch_bounds__(kPauliThreads)
                o[k].x = o[k].y = 0;
           }
           __syncthreads();
-          for (uint32_t g = 0; g < P.ngroups; ++g) {
-               const PauliGroup G = load_words(groups + P.group_first + g);
-               double w[A];
-               weights<A>(w, terms, G, base, tid);
-               const bool im = G.kind & 1u;
+          run_terms<A>(terms + P.first, P.count, base, tid, [&](const PauliTerm& t, const double (&w)[A]) {
+               const bool im = t.z_tile & kPauliImag;
 #pragma unroll
                for (int k = 0; k < A; ++k) {
-                    const V y = tile[(k * kPauliThreads + tid) ^ G.x];
+                    const V y = tile[(k * kPauliThreads + tid) ^ t.x];
                     const R v = static_cast<R>(w[k]);
                     // times v, or times i v
                     o[k].x = fma(v, im ? -y.y : y.x, o[k].x);
                     o[k].y = fma(v, im ? y.x : y.y, o[k].y);
                }
-          }
+          });
 #pragma unroll
           for (int k = 0; k < A; ++k) {
                const uint64_t i = base + at.lane + at.reg[k];
                V b;
                b.x = fma(-a.fi, o[k].y, a.fr * o[k].x);
                b.y = fma(a.fi, o[k].x, a.fr * o[k].y);
-               if (a.accumulate) {
-                    const V d = a.dst[i];
-                    b.x += d.x;
-                    b.y += d.y;
+               if (a.add) {
+                    const V d = a.add[i];
+                    b.x = fma(a.g, d.x, b.x);
+                    b.y = fma(a.g, d.y, b.y);
                }
                a.dst[i] = b;
                if (a.o_dst) {
                     V s = a.o_src[i];
-                    s.x += b.x;
-                    s.y += b.y;
+                    s.x = fma(-a.ci, b.y, fma(a.cr, b.x, a.h * s.x));
+                    s.y = fma(a.ci, b.x, fma(a.cr, b.y, a.h * s.y));
                     a.o_dst[i] = s;
                     const double br = b.x, bi = b.y;
-                    norm += br * br + bi * bi;
+                    norm = fma(br, br, fma(bi, bi, norm));
                }
           }
      }
-     if (!a.o_dst) return;
+     if (!partials) return;
      for (int d = 32; d > 0; d >>= 1) norm += __shfl_xor(norm, d, 64);
      __shared__ double red[kPauliThreads / 64];
      if ((tid & 63) == 0) red[tid >> 6] = norm;
@@ -254,14 +293,14 @@ bool pass_fits(const PauliPass& p, int n)
 }
 
 template <typename R, int A>
-void sum_launch(const void* psi, const PauliPass& p, const PauliGroup* g, const PauliTerm* t, uint64_t ntiles, int grid,
+void sum_launch(const void* psi, const PauliPass& p, const PauliTerm* t, uint64_t ntiles, int grid,
                 double* scratch, hipStream_t s)
 {
-     hipLaunchKernelGGL((k_pauli_sum<R, A>), dim3(grid), dim3(kPauliThreads), 0, s, static_cast<const VT<R>*>(psi), p, g,
-                        t, ntiles, scratch);
+     hipLaunchKernelGGL((k_pauli_sum<R, A>), dim3(grid), dim3(kPauliThreads), 0, s, static_cast<const VT<R>*>(psi), p, t,
+                        ntiles, scratch);
 }
 template <typename R, int A>
-void apply_launch(const PauliApply& a, const PauliPass& p, const PauliGroup* g, const PauliTerm* t, uint64_t ntiles,
+void apply_launch(const PauliApply& a, const PauliPass& p, const PauliTerm* t, uint64_t ntiles,
                   int grid, hipStream_t s)
 {
      ApplyArgs<R> k{};
@@ -271,10 +310,14 @@ void apply_launch(const PauliApply& a, const PauliPass& p, const PauliGroup* g, 
      k.o_dst = static_cast<VT<R>*>(a.o_dst);
      k.skip = a.skip;
      k.skip_below = a.skip_below;
+     k.add = static_cast<const VT<R>*>(a.add);
      k.fr = static_cast<R>(a.fr);
      k.fi = static_cast<R>(a.fi);
-     k.accumulate = a.accumulate ? 1 : 0;
-     hipLaunchKernelGGL((k_pauli_apply<R, A>), dim3(grid), dim3(kPauliThreads), 0, s, k, p, g, t, ntiles, a.scratch);
+     k.g = static_cast<R>(a.g);
+     k.h = static_cast<R>(a.h);
+     k.cr = static_cast<R>(a.cr);
+     k.ci = static_cast<R>(a.ci);
+     hipLaunchKernelGGL((k_pauli_apply<R, A>), dim3(grid), dim3(kPauliThreads), 0, s, k, p, t, ntiles, a.norm ? a.scratch : nullptr);
 }
 
 // f<A>() for the amplitudes a thread of an n-qubit state's tile holds.
@@ -288,31 +331,31 @@ void apply_launch(const PauliApply& a, const PauliPass& p, const PauliGroup* g, 
 
 }  // namespace
 
-hipError_t launch_pauli_sum(const void* psi, Prec prec, int n, const PauliPass& pass, const PauliGroup* groups,
-                            const PauliTerm* terms, double* scratch, double* out, hipStream_t s)
+hipError_t launch_pauli_sum(const void* psi, Prec prec, int n, const PauliPass& pass, const PauliTerm* terms,
+                            double* scratch, double* out, hipStream_t s)
 {
      if (!pass_fits(pass, n)) return hipErrorInvalidValue;
      const uint64_t ntiles = 1ull << (n - pauli_tile_bits(n));
      const int grid = static_cast<int>(ntiles < kReduceBlocks ? ntiles : kReduceBlocks);
-     if (prec == Prec::C128) HQ_PAULI(double, (sum_launch<R, A>(psi, pass, groups, terms, ntiles, grid, scratch, s)))
-     else HQ_PAULI(float, (sum_launch<R, A>(psi, pass, groups, terms, ntiles, grid, scratch, s)))
+     if (prec == Prec::C128) HQ_PAULI(double, (sum_launch<R, A>(psi, pass, terms, ntiles, grid, scratch, s)))
+     else HQ_PAULI(float, (sum_launch<R, A>(psi, pass, terms, ntiles, grid, scratch, s)))
      const hipError_t e = hipGetLastError();
      if (e != hipSuccess) return e;
      hipLaunchKernelGGL(k_sum_partials, dim3(2), dim3(kBlock), 0, s, scratch, grid, out, nullptr, 0.0);
      return hipGetLastError();
 }
 
-hipError_t launch_pauli_apply(const PauliApply& a, Prec prec, int n, const PauliPass& pass, const PauliGroup* groups,
-                              const PauliTerm* terms, hipStream_t s)
+hipError_t launch_pauli_apply(const PauliApply& a, Prec prec, int n, const PauliPass& pass, const PauliTerm* terms,
+                              hipStream_t s)
 {
-     if (!pass_fits(pass, n) || a.src == a.dst || (a.o_dst && (!a.o_src || !a.scratch || !a.norm)))
+     if (!pass_fits(pass, n) || a.src == a.dst || (a.o_dst && !a.o_src) || (a.norm && (!a.o_dst || !a.scratch)))
           return hipErrorInvalidValue;
      const uint64_t ntiles = 1ull << (n - pauli_tile_bits(n));
      const int grid = static_cast<int>(ntiles < kReduceBlocks ? ntiles : kReduceBlocks);
-     if (prec == Prec::C128) HQ_PAULI(double, (apply_launch<R, A>(a, pass, groups, terms, ntiles, grid, s)))
-     else HQ_PAULI(float, (apply_launch<R, A>(a, pass, groups, terms, ntiles, grid, s)))
+     if (prec == Prec::C128) HQ_PAULI(double, (apply_launch<R, A>(a, pass, terms, ntiles, grid, s)))
+     else HQ_PAULI(float, (apply_launch<R, A>(a, pass, terms, ntiles, grid, s)))
      const hipError_t e = hipGetLastError();
-     if (e != hipSuccess || !a.o_dst) return e;
+     if (e != hipSuccess || !a.norm) return e;
      hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kBlock), 0, s, a.scratch, grid, a.norm, a.skip, a.skip_below);
      return hipGetLastError();
 }

@@ -1,8 +1,10 @@
 // Planning of Pauli sums.  See pauli_prog.hpp.
 #include "pauli_prog.hpp"
 
+#include <algorithm>
+#include <cmath>
 #include <map>
-#include <tuple>
+#include <utility>
 
 namespace hq {
 
@@ -88,21 +90,57 @@ PauliPlan plan_pauli(const std::vector<PauliTermIn>& in, int n, bool apply)
                for (uint64_t b = m & bits; b; b &= b - 1) t |= 1u << rank[__builtin_ctzll(b)];
                return t;
           };
-          pass.group_first = static_cast<uint32_t>(plan.groups.size());
+          pass.first = static_cast<uint32_t>(plan.terms.size());
           for (uint64_t x: here)
                for (uint32_t kind = 0; kind < 4; ++kind) {
                     const auto it = by.find({x, kind});
                     if (it == by.end()) continue;
-                    PauliGroup g{to_tile(x), kind, static_cast<uint32_t>(plan.terms.size()),
-                                 static_cast<uint32_t>(it->second.size())};
-                    for (const Z& z: it->second) plan.terms.push_back(PauliTerm{z.z & ~bits, to_tile(z.z), 0, z.c});
-                    plan.groups.push_back(g);
+                    auto& zs = it->second;
+                    auto cls = [&](const Z& z) { return to_tile(z.z) >> kPauliThr; };
+                    std::stable_sort(zs.begin(), zs.end(), [&](const Z& a, const Z& b) { return cls(a) < cls(b); });
+                    const uint32_t xt = to_tile(x);
+                    // Expectation: i and i ^ x contribute the same; where the
+                    // highest bit of x tells waves or amplitudes of a thread
+                    // apart, the kernel takes the one half, twice.
+                    const double f = !apply && (xt >> kPauliLane) ? 2.0 : 1.0;
+                    for (size_t i = 0; i < zs.size(); ++i) {
+                         PauliTerm t{};
+                         t.z_out = zs[i].z & ~bits;
+                         t.c = f * zs[i].c;
+                         t.z_tile = to_tile(zs[i].z) | ((kind & 1u) ? kPauliImag : 0u) | ((kind & 2u) ? kPauliOut1 : 0u);
+                         t.x = xt;
+                         const bool last = i + 1 == zs.size();
+                         if (last) t.z_tile |= kPauliGroupEnd;
+                         if (last || cls(zs[i]) != cls(zs[i + 1])) t.z_tile |= kPauliClassEnd;
+                         plan.terms.push_back(t);
+                    }
                }
-          pass.ngroups = static_cast<uint32_t>(plan.groups.size()) - pass.group_first;
+          pass.count = static_cast<uint32_t>(plan.terms.size()) - pass.first;
           plan.passes.push_back(pass);
      }
-     plan.terms.push_back(PauliTerm{0, 0, 0, 0.0});
+     plan.terms.push_back(PauliTerm{});
      return plan;
+}
+
+std::vector<double> bessel_series(double z)
+{
+     if (!(z > 1e-300)) return {1.0};
+     // far enough above the turning point k = z that J_k is below 1e-60 there
+     const int top = static_cast<int>(z + 24.0 * std::cbrt(z) + 60.0) | 1;
+     std::vector<long double> j(static_cast<size_t>(top) + 2, 0.0L);
+     j[static_cast<size_t>(top)] = 1e-300L;
+     long double even = 0.0L;
+     for (int k = top; k >= 1; --k) {
+          j[k - 1] = 2.0L * k / z * j[k] - j[k + 1];
+          if (std::fabs(j[k - 1]) > 1e250L)
+               for (int q = k - 1; q <= top; ++q) j[q] *= 1e-250L;
+     }
+     for (int k = 2; k <= top; k += 2) even += j[k];
+     const long double norm = 1.0L / (j[0] + 2.0L * even);
+     std::vector<double> out;
+     for (int k = 0; k <= top; ++k) out.push_back(static_cast<double>(j[k] * norm));
+     while (out.size() > 1 && std::fabs(out.back()) < 1e-17) out.pop_back();
+     return out;
 }
 
 }  // namespace hq

@@ -92,28 +92,38 @@ void run_case(int n, int nterms, int max_weight, bool complex_c, unsigned seed)
                     for (int r = 0; r < T; ++r) base |= static_cast<uint64_t>((rank >> r) & 1) << pos[r];
                     return base;
                };
-               CHECK(P.group_first + P.ngroups <= plan.groups.size());
+               CHECK(P.first + P.count < plan.terms.size());  // and the record read ahead
                for (uint64_t base = 0; base < psi.size(); ++base) {
                     if (base & bits) continue;
-                    for (uint32_t g = P.group_first; g < P.group_first + P.ngroups; ++g) {
-                         const PauliGroup& G = plan.groups[g];
-                         CHECK(G.first + G.count < plan.terms.size());  // and the record read ahead
-                         CHECK(!(G.x >> T));
+                    std::vector<double> w(size_t(1) << T, 0.0);
+                    uint32_t group = P.first;
+                    for (uint32_t i = P.first; i < P.first + P.count; ++i) {
+                         const PauliTerm& t = plan.terms[i];
+                         const uint32_t zt = t.z_tile & 0xffffu;
+                         CHECK(!(t.x >> T) && !(zt >> T) && t.x == plan.terms[group].x);
+                         for (uint32_t r = 0; r < (1u << T); ++r) w[r] += t.c * parity(base & t.z_out) * parity(r & zt);
+                         if (i > group && !(plan.terms[i - 1].z_tile & kPauliClassEnd))
+                              CHECK((plan.terms[i - 1].z_tile & 0xffffu) >> kPauliThr == zt >> kPauliThr);
+                         if (!(t.z_tile & kPauliGroupEnd)) continue;
+                         CHECK(t.z_tile & kPauliClassEnd);
+                         group = i + 1;
                          for (uint32_t r = 0; r < (1u << T); ++r) {
-                              double w = 0;
-                              for (uint32_t t = G.first; t < G.first + G.count; ++t)
-                                   w += plan.terms[t].c * parity(base & plan.terms[t].z_out) * parity(r & plan.terms[t].z_tile);
-                              const cplx x = psi[index(base, r)], y = psi[index(base, r ^ G.x)];
+                              const cplx x = psi[index(base, r)], y = psi[index(base, r ^ t.x)];
+                              const bool im = t.z_tile & kPauliImag;
                               if (apply) {
-                                   dst[index(base, r)] += (G.kind & 1 ? cplx(0, w) : cplx(w, 0)) * y;
+                                   dst[index(base, r)] += (im ? cplx(0, w[r]) : cplx(w[r], 0)) * y;
                               }
                               else {
+                                   // the half that the kernel takes
+                                   if ((t.x >> kPauliLane) && ((r >> (31 - __builtin_clz(t.x))) & 1)) continue;
                                    const cplx q = std::conj(y) * x;
-                                   const double v = w * (G.kind & 1 ? q.imag() : q.real());
-                                   got += G.kind & 2 ? lcplx(0, v) : lcplx(v, 0);
+                                   const double v = w[r] * (im ? q.imag() : q.real());
+                                   got += t.z_tile & kPauliOut1 ? lcplx(0, v) : lcplx(v, 0);
                               }
                          }
+                         w.assign(size_t(1) << T, 0.0);
                     }
+                    CHECK(group == P.first + P.count);
                }
           }
           double scale = 0;

@@ -95,6 +95,28 @@ def test_evolution_matches_expm(engine_mod, n):
         assert np.abs(sim.get_state() - ref).max() <= tol, precision
 
 
+@pytest.mark.parametrize("t,imag", [(-6.0, 0.0), (25.0, 0.0), (1e-9, 0.0), (0.4, 0.15)])
+def test_evolution_long_backward_and_not_hermitian(engine_mod, t, imag):
+    """Chebyshev series over long and negative times; a sum that is not Hermitian takes the Taylor steps."""
+    n = 10
+    terms = [([(i, "Z"), (i + 1, "Z")], 0.4 + 0.05 * i) for i in range(n - 1)] + [([(i, "X")], 0.3) for i in range(n)]
+    if imag:
+        terms.append(([(2, "Y"), (7, "X")], 1j * imag))
+    mats = []
+    for term, c in terms:
+        m = sp.identity(1, format="csr")
+        ops = dict(term)
+        for q in reversed(range(n)):
+            m = sp.kron(m, sp.csr_matrix(np.array(NMAT[ops[q]]) if q in ops else np.eye(2)), format="csr")
+        mats.append(c * m)
+    ham = sum(mats)
+    print("time evolution t=%g imag=%g" % (t, imag), flush=True)
+    sim = prepared(engine_mod, n, "c128", 3)
+    psi = sim.get_state()
+    sim.emulate_time_evolution(terms, t, list(range(n)), [])
+    assert np.abs(sim.get_state() - expm_multiply(-1j * t * ham, psi)).max() <= 1e-10
+
+
 def test_controlled_evolution_keeps_the_rest(engine_mod):
     n = 13
     rng = np.random.default_rng(4)
