@@ -100,11 +100,10 @@ __device__ __forceinline__ void run_terms(const PauliTerm* __restrict__ terms, c
      }
 }
 
-// sum_k w[k] Re or Im (conj(y_k) x_k), y the amplitude at i ^ x; KB >= 0: only
-// the amplitudes whose number has bit KB clear.
-template <int KB, typename V, int A>
-__device__ __forceinline__ double group_sum(const V (&x)[A], const double (&w)[A], const V* tile, uint32_t tid, uint32_t xm,
-                                            bool im)
+// sum_k w[k] Re (IM: Im) of conj(y_k) x_k, y the amplitude at i ^ x; KB >= 0:
+// only the amplitudes whose number has bit KB clear.
+template <int KB, bool IM, typename V, int A>
+__device__ __forceinline__ double group_part(const V (&x)[A], const double (&w)[A], const V* tile, uint32_t tid, uint32_t xm)
 {
      double s = 0;
 #pragma unroll
@@ -112,11 +111,15 @@ __device__ __forceinline__ double group_sum(const V (&x)[A], const double (&w)[A
           if (KB >= 0 && ((k >> (KB < 0 ? 0 : KB)) & 1)) continue;
           const V y = tile[(k * kPauliThreads + tid) ^ xm];
           const double yr = y.x, yi = y.y, xr = x[k].x, xi = x[k].y;
-          // uniform choice of the part
-          const double p = im ? xi : xr, q = im ? -xr : xi;
-          s = fma(w[k], fma(yr, p, yi * q), s);
+          s = fma(w[k], IM ? fma(yr, xi, -(yi * xr)) : fma(yr, xr, yi * xi), s);
      }
      return s;
+}
+template <int KB, typename V, int A>
+__device__ __forceinline__ double group_sum(const V (&x)[A], const double (&w)[A], const V* tile, uint32_t tid, uint32_t xm,
+                                            bool im)
+{
+     return im ? group_part<KB, true>(x, w, tile, tid, xm) : group_part<KB, false>(x, w, tile, tid, xm);
 }
 
 template <typename R, int A>
@@ -237,16 +240,36 @@ __global__ void __launch_bounds__(kPauliThreads)
                tile[k * kPauliThreads + tid] = o[k];
                o[k].x = o[k].y = 0;
           }
+          V d[A];  // what the result is added to, on its way meanwhile
+#pragma unroll
+          for (int k = 0; k < A; ++k) d[k].x = d[k].y = 0;
+          if (a.add) {
+#pragma unroll
+               for (int k = 0; k < A; ++k) d[k] = a.add[base + at.lane + at.reg[k]];
+          }
           __syncthreads();
           run_terms<A>(terms + P.first, P.count, base, tid, [&](const PauliTerm& t, const double (&w)[A]) {
-               const bool im = t.z_tile & kPauliImag;
+               // two one-sided ifs on a flag the compiler cannot relate: an
+               // if-else would keep the sums before and after both alive
+               uint32_t real = ~t.z_tile & kPauliImag;
+               asm volatile("" : "+s"(real));
+               if (real) {
 #pragma unroll
-               for (int k = 0; k < A; ++k) {
-                    const V y = tile[(k * kPauliThreads + tid) ^ t.x];
-                    const R v = static_cast<R>(w[k]);
-                    // times v, or times i v
-                    o[k].x = fma(v, im ? -y.y : y.x, o[k].x);
-                    o[k].y = fma(v, im ? y.x : y.y, o[k].y);
+                    for (int k = 0; k < A; ++k) {
+                         const V y = tile[(k * kPauliThreads + tid) ^ t.x];
+                         const R v = static_cast<R>(w[k]);
+                         o[k].x = fma(v, y.x, o[k].x);
+                         o[k].y = fma(v, y.y, o[k].y);
+                    }
+               }
+               if (t.z_tile & kPauliImag) {
+#pragma unroll
+                    for (int k = 0; k < A; ++k) {
+                         const V y = tile[(k * kPauliThreads + tid) ^ t.x];
+                         const R v = static_cast<R>(w[k]);
+                         o[k].x = fma(-v, y.y, o[k].x);
+                         o[k].y = fma(v, y.x, o[k].y);
+                    }
                }
           });
 #pragma unroll
@@ -255,11 +278,8 @@ __global__ void __launch_bounds__(kPauliThreads)
                V b;
                b.x = fma(-a.fi, o[k].y, a.fr * o[k].x);
                b.y = fma(a.fi, o[k].x, a.fr * o[k].y);
-               if (a.add) {
-                    const V d = a.add[i];
-                    b.x = fma(a.g, d.x, b.x);
-                    b.y = fma(a.g, d.y, b.y);
-               }
+               b.x = fma(a.g, d[k].x, b.x);
+               b.y = fma(a.g, d[k].y, b.y);
                a.dst[i] = b;
                if (a.o_dst) {
                     V s = a.o_src[i];
