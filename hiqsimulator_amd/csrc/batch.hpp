@@ -143,8 +143,9 @@ inline uint32_t sample_log_blocks(int n)
      const int lb = n - 8;
      return static_cast<uint32_t>(lb < 0 ? 0 : (lb > 15 ? 15 : lb));
 }
-// One workgroup per job; out[out_off + s] = outcome of shot s.
-hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, int njobs,
+// The jobs' block probabilities become running sums in place;
+// out[out_off + s] = outcome of shot s.  max_shots: the largest job's.
+hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, int njobs, uint32_t max_shots,
                          double* sums, uint64_t* out, hipStream_t s);
 
 // ---- tile programs: many fused ops in one HBM pass --------------------------

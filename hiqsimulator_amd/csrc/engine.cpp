@@ -1328,8 +1328,8 @@ void Engine::sample(uint32_t shots, uint64_t seed, uint64_t* out)
      check(launch_block_sums_multi(d_state_, prec_, reinterpret_cast<const BatchItem*>(d), 1,
                                    uint64_t(1) << lb, d_blocks_, stream_),
            "block_sums_multi");
-     check(launch_sample(d_state_, prec_, reinterpret_cast<const SampleJob*>(d + 256), 1, d_blocks_,
-                         d_samples_, stream_),
+     check(launch_sample(d_state_, prec_, reinterpret_cast<const SampleJob*>(d + 256), 1, shots, d_blocks_, d_samples_,
+                         stream_),
            "sample");
      end_timed();
      check(hipMemcpyAsync(out, d_samples_, shots * sizeof(uint64_t), hipMemcpyDeviceToHost, stream_),

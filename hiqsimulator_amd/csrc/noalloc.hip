@@ -111,7 +111,7 @@ void sample_noalloc(const void* d_state, int n_qubits, Prec prec, uint32_t shots
      // no clearing between calls.
      check(launch_block_sums_multi(d_state, prec, d_item, 1, uint64_t(1) << lb, sums, stream),
            "block_sums_multi");
-     check(launch_sample(d_state, prec, d_job, 1, sums, d_out, stream), "sample");
+     check(launch_sample(d_state, prec, d_job, 1, shots, sums, d_out, stream), "sample");
 }
 
 }  // namespace hq
