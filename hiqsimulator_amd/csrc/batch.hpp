@@ -147,6 +147,12 @@ inline uint32_t sample_log_blocks(int n)
 // out[out_off + s] = outcome of shot s.  max_shots: the largest job's.
 hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, int njobs, uint32_t max_shots,
                          double* sums, uint64_t* out, hipStream_t s);
+// The outcome at the point u of the running probability of one state: the
+// first index whose running sum reaches u.  sums: the probabilities of its
+// 2^log_blocks blocks of 2^log_block_amps amplitudes (they become running
+// sums); out = {index, bits of the sum of all}, device or pinned host memory.
+hipError_t launch_measure(const void* psi, Prec prec, double* sums, int log_blocks, int log_block_amps, double u,
+                          uint64_t* out, hipStream_t s);
 
 // ---- tile programs: many fused ops in one HBM pass --------------------------
 // A tile holds the 2^kTileBits amplitudes whose index bits outside

@@ -1070,12 +1070,8 @@ __device__ __forceinline__ void cdf_columns(double* __restrict__ base, uint32_t 
      __builtin_amdgcn_wave_barrier();
 }
 
-__global__ void __launch_bounds__(kSampleThreads)
-    k_sample_cdf(const SampleJob* __restrict__ jobs, double* __restrict__ sums)
+__device__ __forceinline__ void running_sums(double* __restrict__ cdf, const uint32_t nb)
 {
-     const SampleJob jb = jobs[blockIdx.x];
-     double* const cdf = sums + jb.sums_off;
-     const uint32_t nb = 1u << jb.log_blocks;
      const uint32_t per = nb > kSampleThreads ? nb / kSampleThreads : 1u;
      const uint32_t t = threadIdx.x, lane = t & 63;
      const uint32_t first = t * per;
@@ -1126,40 +1122,25 @@ __global__ void __launch_bounds__(kSampleThreads)
           }
 }
 
-// One wave per shot (four shots a workgroup; blockIdx.y = the job): u =
-// U[0,1) * total, the first block whose running sum exceeds u, and in it the
-// first amplitude whose running probability exceeds the rest.  Both searches
-// go 64 ways a step: the lanes look at the ends of 64 equal parts of the
-// running sums, then sum 64 equal parts of the block's amplitudes, take the
-// part the rest falls into, and so on down to one amplitude.  A single thread
-// that scanned the block for its shot took 4.2 ms for 1024 shots of a
-// 28-qubit complex64 state (8192 amplitudes a block), all loads in a chain;
-// this takes 0.02 ms.
-template <typename R>
-__global__ void __launch_bounds__(256)
-    k_sample_shots(const VT<R>* __restrict__ arena, const SampleJob* __restrict__ jobs,
-                   const double* __restrict__ sums, uint64_t* __restrict__ out)
+// One wave finds the outcome at the point u of the running probability: the
+// first block whose running sum exceeds u (Incl: reaches u), and in it the
+// first amplitude whose running probability exceeds (reaches) the rest.  Both
+// searches go 64 ways a step: the lanes look at the ends of 64 equal parts of
+// the running sums, then sum 64 equal parts of the block's amplitudes, take
+// the part the rest falls into, and so on down to one amplitude.
+template <typename R, bool Incl>
+__device__ __forceinline__ uint64_t find_outcome(const VT<R>* __restrict__ psi, const double* __restrict__ cdf,
+                                                 const uint32_t nb, const uint64_t K, const double u,
+                                                 const uint32_t lane)
 {
-     const SampleJob jb = jobs[blockIdx.y];
-     const uint32_t s = blockIdx.x * 4 + (threadIdx.x >> 6);
-     const uint32_t lane = threadIdx.x & 63;
-     if (s >= jb.shots) return;  // (whole waves; no barrier below)
-     const double* const cdf = sums + jb.sums_off;
-     const uint32_t nb = 1u << jb.log_blocks;
-     const double total = cdf[nb - 1];
-     const uint2 key = make_uint2(static_cast<uint32_t>(jb.seed), static_cast<uint32_t>(jb.seed >> 32));
-     const uint4 r = philox4x32_10(make_uint4(s, 0u, 0x5a3du, 0u), key);
-     const double u = uniform53(r.x, r.y) * total;
-     uint32_t lo = 0;  // first block with cdf > u (the last one if none)
+     uint32_t lo = 0;  // (the last block if no running sum does)
      for (uint32_t len = nb; len > 1;) {
           const uint32_t part = len > 64 ? len / 64 : 1, parts = len / part;
-          const bool over = lane < parts && cdf[lo + (lane + 1) * part - 1] > u;
-          const uint64_t m = __ballot(over);
+          const double c = lane < parts ? cdf[lo + (lane + 1) * part - 1] : 0.0;
+          const uint64_t m = __ballot(lane < parts && (Incl ? c >= u : c > u));
           lo += (m ? static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(m))) - 1 : parts - 1) * part;
           len = part;
      }
-     const uint64_t K = 1ull << jb.log_block_amps;
-     const VT<R>* const psi = arena + jb.state_off;
      double rem = u - (lo ? cdf[lo - 1] : 0.0);
      uint64_t at = static_cast<uint64_t>(lo) * K;
      for (uint64_t len = K; len > 1;) {
@@ -1181,7 +1162,7 @@ __global__ void __launch_bounds__(256)
           }
           // (p > 0: the running sums of two lanes are rounded apart, so one
           // over an empty part can be the larger)
-          const uint64_t m = __ballot(lane < parts && p > 0.0 && rem < run);
+          const uint64_t m = __ballot(lane < parts && p > 0.0 && (Incl ? rem <= run : rem < run));
           uint32_t f;
           if (m) {
                f = static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(m))) - 1;
@@ -1198,7 +1179,57 @@ __global__ void __launch_bounds__(256)
           at += f * part;
           len = part;
      }
+     return at;
+}
+
+__global__ void __launch_bounds__(kSampleThreads)
+    k_sample_cdf(const SampleJob* __restrict__ jobs, double* __restrict__ sums)
+{
+     const SampleJob jb = jobs[blockIdx.x];
+     running_sums(sums + jb.sums_off, 1u << jb.log_blocks);
+}
+
+// One wave per shot, four shots a workgroup; blockIdx.y = the job.  A single
+// thread that scanned the block for its shot took 4.2 ms for 1024 shots of a
+// 28-qubit complex64 state (8192 amplitudes a block, all loads in a chain);
+// this takes 0.02 ms.
+template <typename R>
+__global__ void __launch_bounds__(256)
+    k_sample_shots(const VT<R>* __restrict__ arena, const SampleJob* __restrict__ jobs,
+                   const double* __restrict__ sums, uint64_t* __restrict__ out)
+{
+     const SampleJob jb = jobs[blockIdx.y];
+     const uint32_t s = blockIdx.x * 4 + (threadIdx.x >> 6);
+     const uint32_t lane = threadIdx.x & 63;
+     if (s >= jb.shots) return;  // (whole waves; no barrier below)
+     const double* const cdf = sums + jb.sums_off;
+     const uint32_t nb = 1u << jb.log_blocks;
+     const uint2 key = make_uint2(static_cast<uint32_t>(jb.seed), static_cast<uint32_t>(jb.seed >> 32));
+     const uint4 r = philox4x32_10(make_uint4(s, 0u, 0x5a3du, 0u), key);
+     const double u = uniform53(r.x, r.y) * cdf[nb - 1];
+     const uint64_t at = find_outcome<R, false>(arena + jb.state_off, cdf, nb, 1ull << jb.log_block_amps, u, lane);
      if (lane == 0) out[jb.out_off + s] = at;
+}
+
+// A measurement's outcome: the running sums, then the search, in one
+// workgroup.  out[0] = the index, out[1] = the sum of all probabilities (as
+// bits), straight into host memory.  Copying the sums and the chosen block to
+// the host and scanning them there took 45 us of a measurement of 16 qubits
+// and two more round trips; this takes 5 us.
+template <typename R>
+__global__ void __launch_bounds__(kSampleThreads)
+    k_measure(const VT<R>* __restrict__ psi, double* __restrict__ sums, const int log_blocks,
+              const int log_block_amps, const double u, uint64_t* __restrict__ out)
+{
+     const uint32_t nb = 1u << log_blocks;
+     running_sums(sums, nb);
+     __syncthreads();
+     if (threadIdx.x >= 64) return;
+     const uint64_t at = find_outcome<R, true>(psi, sums, nb, 1ull << log_block_amps, u, threadIdx.x);
+     if (threadIdx.x == 0) {
+          out[0] = at;
+          out[1] = static_cast<uint64_t>(__double_as_longlong(sums[nb - 1]));
+     }
 }
 
 template <typename R>
@@ -1429,6 +1460,19 @@ hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, in
      else
           hipLaunchKernelGGL((k_sample_shots<float>), grid, dim3(256), 0, s, static_cast<const float2*>(arena), jobs,
                              sums, out);
+     return hipGetLastError();
+}
+
+hipError_t launch_measure(const void* psi, Prec prec, double* sums, int log_blocks, int log_block_amps, double u,
+                          uint64_t* out, hipStream_t s)
+{
+     if (log_blocks < 0 || log_blocks > 15 || log_block_amps < 0 || log_block_amps > 40) return hipErrorInvalidValue;
+     if (prec == Prec::C128)
+          hipLaunchKernelGGL((k_measure<double>), dim3(1), dim3(kSampleThreads), 0, s, static_cast<const double2*>(psi),
+                             sums, log_blocks, log_block_amps, u, out);
+     else
+          hipLaunchKernelGGL((k_measure<float>), dim3(1), dim3(kSampleThreads), 0, s, static_cast<const float2*>(psi),
+                             sums, log_blocks, log_block_amps, u, out);
      return hipGetLastError();
 }
 

@@ -19,6 +19,10 @@ namespace {
 constexpr double kMaxFloatError = 1e-12;  // SimulatorMPI.cpp:75
 constexpr uint64_t kMaxBlocks = uint64_t(1) << 15;  // SimulatorMPI.cpp:903
 constexpr int kMaxOuts = 256;                        // batched reduction outputs
+// States of up to this many amplitudes lose a qubit without a wait between its
+// probabilities and the removal: below it the waits are most of the time (16
+// qubits: 21 us a qubit, 15 us now), above it the passes are.
+constexpr uint64_t kTakeBitMax = uint64_t(1) << 20;
 
 void check(hipError_t e, const char* what)
 {
@@ -70,14 +74,12 @@ Engine::Engine(uint64_t seed, int64_t max_local, int64_t max_cluster, Prec prec,
      check(hipMalloc(reinterpret_cast<void**>(&d_scratch_),
                      (kReduceScratchDoubles + 2 * kMaxOuts) * sizeof(double)),
            "hipMalloc(scratch)");
+     check(init_reduce_scratch(d_scratch_, stream_), "hipMemsetAsync(scratch)");
      check(hipHostMalloc(reinterpret_cast<void**>(&h_out_), 2 * kMaxOuts * sizeof(double),
                          hipHostMallocDefault),
            "hipHostMalloc(out)");
      check(hipMalloc(reinterpret_cast<void**>(&d_blocks_), kMaxBlocks * sizeof(double)),
            "hipMalloc(blocks)");
-     check(hipHostMalloc(reinterpret_cast<void**>(&h_blocks_), kMaxBlocks * sizeof(double),
-                         hipHostMallocDefault),
-           "hipHostMalloc(blocks)");
      // The empty register is the one-amplitude state [1] (SimulatorMPI.cpp:96-98).
      ensure_state(1);
      check(launch_fill(d_state_, prec_, 1, 1.0, 0.0, stream_), "fill");
@@ -105,8 +107,6 @@ Engine::~Engine()
      if (d_scratch_) (void)hipFree(d_scratch_);
      if (h_out_) (void)hipHostFree(h_out_);
      if (d_blocks_) (void)hipFree(d_blocks_);
-     if (h_blocks_) (void)hipHostFree(h_blocks_);
-     if (h_stage_) (void)hipHostFree(h_stage_);
      if (d_samples_) (void)hipFree(d_samples_);
      for (auto& ps: prog_) {
           if (ps.ev) (void)hipEventDestroy(ps.ev);
@@ -220,13 +220,7 @@ const void* Engine::upload_matrix(const Mat& m, const void* desc, size_t desc_by
      return d;
 }
 
-void Engine::read_out(double* host, size_t count)
-{
-     check(hipMemcpyAsync(host, d_scratch_ + kReduceScratchDoubles, count * sizeof(double),
-                          hipMemcpyDeviceToHost, stream_),
-           "hipMemcpyAsync(out)");
-     check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-}
+void Engine::wait_out() { check(hipStreamSynchronize(stream_), "hipStreamSynchronize"); }
 
 // ---------------------------------------------------------------------------
 // Timing
@@ -356,23 +350,34 @@ void Engine::deallocate_qubit(int64_t id)
      DeviceScope ds(device_);
      const size_t pos = find_sure(id);
      settle();
-     begin_timed(kReduce);
-     check(launch_two_bucket(d_state_, prec_, n_qubits(), static_cast<int>(pos), d_scratch_,
-                             d_scratch_ + kReduceScratchDoubles, stream_),
-           "two_bucket");
+     // A small state loses its qubit in the same breath, before the host knows
+     // which half it keeps or that the qubit is entangled (the state itself
+     // stays as it is until then): two waits' worth of latency in one.
+     const bool small = n_amps_ <= kTakeBitMax && n_amps_ / 2 <= cap_tmp_;
+     if (small) ensure_tmp(n_amps_ / 2);
+     begin_timed(small ? kRemoveBit : kReduce);
+     if (small)
+          check(launch_take_bit(d_tmp_, d_state_, prec_, n_qubits(), static_cast<int>(pos), kMaxFloatError, d_scratch_,
+                                d_scratch_ + kReduceScratchDoubles, h_out_, stream_),
+                "take_bit");
+     else
+          check(launch_two_bucket(d_state_, prec_, n_qubits(), static_cast<int>(pos), d_scratch_, h_out_, stream_),
+                "two_bucket");
      end_timed();
-     read_out(h_out_, 2);
+     wait_out();
      const double s0 = h_out_[0], s1 = h_out_[1];
      if (!((s0 > kMaxFloatError) ^ (s1 > kMaxFloatError)))
           throw std::runtime_error("DeallocateLocalQubit(): qubit " + std::to_string(id)
                                    + " is entangled");
      const int keep = s0 > kMaxFloatError ? 0 : 1;
-     ensure_tmp(n_amps_ / 2);
-     begin_timed(kRemoveBit);
-     check(launch_remove_bit(d_tmp_, d_state_, prec_, n_amps_, static_cast<int>(pos), keep,
-                             stream_),
-           "remove_bit");
-     end_timed();
+     if (!small) {
+          ensure_tmp(n_amps_ / 2);
+          begin_timed(kRemoveBit);
+          check(launch_remove_bit(d_tmp_, d_state_, prec_, n_amps_, static_cast<int>(pos), keep,
+                                  stream_),
+                "remove_bit");
+          end_timed();
+     }
      swap_tmp();
      n_amps_ /= 2;
      locals_.erase(locals_.begin() + static_cast<long>(pos));
@@ -661,87 +666,52 @@ void Engine::mask_of(const std::vector<int64_t>& ids, const std::vector<uint8_t>
 double Engine::masked_norm(uint64_t msk, uint64_t val)
 {
      begin_timed(kReduce);
-     check(launch_masked_norm(d_state_, prec_, n_qubits(), msk, val, d_scratch_,
-                              d_scratch_ + kReduceScratchDoubles, stream_),
-           "masked_norm");
+     check(launch_masked_norm(d_state_, prec_, n_qubits(), msk, val, d_scratch_, h_out_, stream_), "masked_norm");
      end_timed();
-     read_out(h_out_, 1);
+     wait_out();
      return h_out_[0];
-}
-
-void Engine::normalize(double norm, uint64_t msk, uint64_t val)
-{
-     const double f = 1.0 / std::sqrt(norm);
-     begin_timed(kNormalize);
-     check(launch_normalize(d_state_, prec_, n_amps_, msk, val, f, stream_), "normalize");
-     end_timed();
 }
 
 std::vector<uint8_t> Engine::measure(const std::vector<int64_t>& ids)
 {
      DeviceScope ds(device_);
      settle();
-     const uint64_t nb = std::min<uint64_t>(n_amps_, kMaxBlocks);
-     const uint64_t K = n_amps_ / nb;
-     begin_timed(kReduce);
-     check(launch_block_sums(d_state_, prec_, n_amps_, nb, d_blocks_, stream_), "block_sums");
-     end_timed();
-     check(hipMemcpyAsync(h_blocks_, d_blocks_, nb * sizeof(double), hipMemcpyDeviceToHost,
-                          stream_),
-           "hipMemcpyAsync(blocks)");
-     check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-     std::partial_sum(h_blocks_, h_blocks_ + nb, h_blocks_);
+     const int lb = static_cast<int>(sample_log_blocks(n_qubits()));
      const double u = dist_(rng_);
-     uint64_t b = 0;
-     for (; b < nb; ++b)
-          if (u <= h_blocks_[b]) break;
-     if (b == nb) {
+     uint64_t found[2];
+     begin_timed(kReduce);
+     check(launch_block_sums(d_state_, prec_, n_amps_, uint64_t(1) << lb, d_blocks_, stream_), "block_sums");
+     check(launch_measure(d_state_, prec_, d_blocks_, lb, n_qubits() - lb, u, reinterpret_cast<uint64_t*>(h_out_),
+                          stream_),
+           "measure");
+     end_timed();
+     wait_out();
+     std::memcpy(found, h_out_, sizeof(found));
+     double total;
+     std::memcpy(&total, &found[1], sizeof(total));
+     if (!(u <= total)) {
           std::ostringstream os;
-          os << "MeasureQubits(): Random number " << u << " > norm partial sum "
-             << h_blocks_[nb - 1];
+          os << "MeasureQubits(): Random number " << u << " > norm partial sum " << total;
           throw std::runtime_error(os.str());
-     }
-     // In-block scan in index order, starting from the previous prefix
-     // (SimulatorMPI.cpp:943-961).
-     const size_t ab = amp_bytes(prec_);
-     if (K * ab > stage_bytes_) {
-          if (h_stage_) check(hipHostFree(h_stage_), "hipHostFree");
-          h_stage_ = nullptr;
-          check(hipHostMalloc(reinterpret_cast<void**>(&h_stage_), K * ab, hipHostMallocDefault),
-                "hipHostMalloc(stage)");
-          stage_bytes_ = K * ab;
-     }
-     check(hipMemcpyAsync(h_stage_, static_cast<char*>(d_state_) + b * K * ab, K * ab,
-                          hipMemcpyDeviceToHost, stream_),
-           "hipMemcpyAsync(block)");
-     check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-     double shift = b > 0 ? h_blocks_[b - 1] : 0.0;
-     uint64_t k = b * K;
-     for (uint64_t j = 0; j < K; ++j, ++k) {
-          double re, im;
-          if (prec_ == Prec::C128) {
-               re = reinterpret_cast<const double*>(h_stage_)[2 * j];
-               im = reinterpret_cast<const double*>(h_stage_)[2 * j + 1];
-          }
-          else {
-               re = reinterpret_cast<const float*>(h_stage_)[2 * j];
-               im = reinterpret_cast<const float*>(h_stage_)[2 * j + 1];
-          }
-          shift += re * re + im * im;
-          if (shift >= u) break;
      }
      std::vector<uint8_t> res(ids.size(), 0);
      uint64_t msk = 0, val = 0;
      for (size_t i = 0; i < ids.size(); ++i) {
           const size_t p = find_sure(ids[i]);
           msk |= uint64_t(1) << p;
-          if ((k >> p) & 1) {
+          if ((found[0] >> p) & 1) {
                val |= uint64_t(1) << p;
                res[i] = 1;
           }
      }
-     const double norm = masked_norm(msk, val);
-     normalize(norm, msk, val);
+     // The norm of what is kept stays on the device.
+     double* const norm = d_scratch_ + kReduceScratchDoubles;
+     begin_timed(kReduce);
+     check(launch_masked_norm(d_state_, prec_, n_qubits(), msk, val, d_scratch_, norm, stream_), "masked_norm");
+     end_timed();
+     begin_timed(kNormalize);
+     check(launch_normalize(d_state_, prec_, n_amps_, msk, val, 1.0, norm, stream_), "normalize");
+     end_timed();
      return res;
 }
 
@@ -774,7 +744,7 @@ cplx Engine::get_amplitude(const std::vector<uint8_t>& bits, const std::vector<i
               "qubits.");
      settle();
      const size_t ab = amp_bytes(prec_);
-     char buf[16];
+     char* const buf = reinterpret_cast<char*>(h_out_);
      check(hipMemcpyAsync(buf, static_cast<char*>(d_state_) + num * ab, ab, hipMemcpyDeviceToHost,
                           stream_),
            "hipMemcpyAsync(amplitude)");
@@ -800,7 +770,9 @@ void Engine::collapse(const std::vector<int64_t>& ids, const std::vector<uint8_t
      const double norm = masked_norm(msk, val);
      if (norm < 1.e-12)
           throw std::runtime_error("collapseWaveFunction(): Invalid collapse! Probability is ~0.");
-     normalize(norm, msk, val);
+     begin_timed(kNormalize);
+     check(launch_normalize(d_state_, prec_, n_amps_, msk, val, 1.0 / std::sqrt(norm), nullptr, stream_), "normalize");
+     end_timed();
 }
 
 double Engine::entropy()
@@ -808,11 +780,9 @@ double Engine::entropy()
      DeviceScope ds(device_);
      settle();
      begin_timed(kReduce);
-     check(launch_entropy(d_state_, prec_, n_amps_, d_scratch_, d_scratch_ + kReduceScratchDoubles,
-                          stream_),
-           "entropy");
+     check(launch_entropy(d_state_, prec_, n_amps_, d_scratch_, h_out_, stream_), "entropy");
      end_timed();
-     read_out(h_out_, 1);
+     wait_out();
      return -h_out_[0];
 }
 
@@ -1050,11 +1020,10 @@ void Engine::compare_snapshot(double out[5])
           throw std::runtime_error("compare_snapshot(): no snapshot of the current size");
      settle();
      begin_timed(kReduce);
-     check(launch_compare(d_state_, d_snap_, prec_, n_amps_, d_scratch_,
-                          d_scratch_ + kReduceScratchDoubles, stream_),
+     check(launch_compare(d_state_, d_snap_, prec_, n_amps_, d_scratch_, h_out_, stream_),
            "compare");
      end_timed();
-     read_out(h_out_, 5);
+     wait_out();
      for (int i = 0; i < 5; ++i) out[i] = h_out_[i];
 }
 
@@ -1389,11 +1358,11 @@ cplx Engine::expectation(const std::vector<uint64_t>& xm, const std::vector<uint
                     for (size_t p = p0; p < p1; ++p) {
                          begin_timed(kPauli);
                          check(launch_pauli_sum(d_state_, prec_, n_qubits(), plan.passes[p], terms, d_scratch_,
-                                                d_scratch_ + kReduceScratchDoubles + 2 * (p - p0), stream_),
+                                                h_out_ + 2 * (p - p0), stream_),
                                "pauli_sum");
                          end_timed();
                     }
-                    read_out(h_out_, 2 * (p1 - p0));
+                    wait_out();
                     for (size_t p = 0; p < p1 - p0; ++p) total += cplx(h_out_[2 * p], h_out_[2 * p + 1]);
                }
                program_done(ps);
@@ -1401,14 +1370,20 @@ cplx Engine::expectation(const std::vector<uint64_t>& xm, const std::vector<uint
      }
      for (size_t t0 = 0; t0 < list.size(); t0 += kMaxOuts / 2) {
           const size_t t1 = std::min(list.size(), t0 + kMaxOuts / 2);
-          for (size_t t = t0; t < t1; ++t) {
+          for (size_t t = t0; t < t1; t += kPauliMasks) {
+               PauliMasks masks{};
+               const int count = static_cast<int>(std::min<size_t>(kPauliMasks, t1 - t));
+               for (int j = 0; j < count; ++j) {
+                    masks.x[j] = list[t + j].x;
+                    masks.z[j] = list[t + j].z;
+               }
                begin_timed(kPauli);
-               check(launch_pauli_expectation(d_state_, prec_, n_amps_, list[t].x, list[t].z, d_scratch_,
-                                              d_scratch_ + kReduceScratchDoubles + 2 * (t - t0), stream_),
+               check(launch_pauli_expectation(d_state_, prec_, n_amps_, masks, count, d_scratch_, h_out_ + 2 * (t - t0),
+                                              stream_),
                      "pauli_expectation");
                end_timed();
           }
-          read_out(h_out_, 2 * (t1 - t0));
+          wait_out();
           for (size_t t = t0; t < t1; ++t) total += list[t].c * cplx(h_out_[2 * (t - t0)], h_out_[2 * (t - t0) + 1]);
      }
      return total;
@@ -1562,7 +1537,7 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
           void* const out = cmask ? out_own.p : d_tmp_;
           if (cmask) {
                check(launch_copy(w, d_state_, prec_, n_amps_, stream_), "copy");
-               check(launch_normalize(w, prec_, n_amps_, cmask, cmask, 1.0, stream_), "select");
+               check(launch_normalize(w, prec_, n_amps_, cmask, cmask, 1.0, nullptr, stream_), "select");
                check(launch_pauli_accumulate(d_state_, w, prec_, n_amps_, 0, 0, -1.0, 0.0, stream_), "subtract");
           }
           const std::vector<double> bes = bessel_series(reach);
@@ -1611,7 +1586,7 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
      Buf w(bytes), out(bytes), a(bytes), b(bytes);
      check(launch_copy(w.p, d_state_, prec_, n_amps_, stream_), "copy");
      if (cmask) {
-          check(launch_normalize(w.p, prec_, n_amps_, cmask, cmask, 1.0, stream_), "select");
+          check(launch_normalize(w.p, prec_, n_amps_, cmask, cmask, 1.0, nullptr, stream_), "select");
           // the state keeps only its uncontrolled part until w comes back
           check(launch_pauli_accumulate(d_state_, w.p, prec_, n_amps_, 0, 0, -1.0, 0.0, stream_), "subtract");
      }
@@ -1628,8 +1603,8 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
           // that, and of a few early ones, are taken, and the terms after them
           // decide on the device whether they are still needed.
           double* const outs = d_scratch_ + kReduceScratchDoubles;
-          check(launch_masked_norm(pw, prec_, n_qubits(), 0, 0, d_scratch_, outs, stream_), "norm");
-          read_out(h_out_, 1);
+          check(launch_masked_norm(pw, prec_, n_qubits(), 0, 0, d_scratch_, h_out_, stream_), "norm");
+          wait_out();
           const double xl = std::abs(tau) * l1;
           const PauliTerm* terms = nullptr;
           ProgSlot& ps = upload_pauli(plan, terms);
@@ -1691,10 +1666,8 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
                                "pauli_accumulate");
                     }
                     check(launch_pauli_accumulate(po, pb, prec_, n_amps_, 0, 0, 1.0, 0.0, stream_), "accumulate");
-                    check(launch_masked_norm(pb, prec_, n_qubits(), 0, 0, d_scratch_, d_scratch_ + kReduceScratchDoubles,
-                                             stream_),
-                          "norm");
-                    read_out(h_out_, 1);
+                    check(launch_masked_norm(pb, prec_, n_qubits(), 0, 0, d_scratch_, h_out_, stream_), "norm");
+                    wait_out();
                     std::swap(pa, pb);
                     if (h_out_[0] < 1e-24) break;
                }

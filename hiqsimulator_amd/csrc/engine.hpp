@@ -227,11 +227,10 @@ private:
      double masked_norm(uint64_t msk, uint64_t val);
      void mask_of(const std::vector<int64_t>& ids, const std::vector<uint8_t>& bits,
                   uint64_t& msk, uint64_t& val) const;
-     void normalize(double norm, uint64_t msk, uint64_t val);
      int n_qubits() const { return static_cast<int>(locals_.size()); }
      void begin_timed(int cls);
      void end_timed();
-     void read_out(double* host, size_t count);
+     void wait_out();  // for reductions that write h_out_
 
      Prec prec_;
      int device_;
@@ -265,11 +264,8 @@ private:
      int ring_next_ = 0;
 
      double* d_scratch_ = nullptr;  // reductions + outputs
-     double* h_out_ = nullptr;      // pinned, 16 doubles
+     double* h_out_ = nullptr;      // pinned: reductions write their results here
      double* d_blocks_ = nullptr;   // measurement block sums (2^15)
-     double* h_blocks_ = nullptr;   // pinned
-     char* h_stage_ = nullptr;      // pinned staging for block scans
-     size_t stage_bytes_ = 0;
      uint64_t* d_samples_ = nullptr;  // sample outcomes
      size_t samples_cap_ = 0;
      // Tile-program staging ring: pinned host image and device copy of

@@ -97,23 +97,41 @@ hipError_t launch_fill(void* psi, Prec prec, uint64_t n, double vre, double vim,
 // dst[i] = src[i], n amplitudes (plain streaming copy).
 hipError_t launch_copy(void* dst, const void* src, Prec prec, uint64_t n, hipStream_t s);
 
-// (i & msk) == val ? psi[i] * f : 0 (SimulatorMPI.cpp:872-895).
+// (i & msk) == val ? psi[i] * f : 0 (SimulatorMPI.cpp:872-895); with `norm`
+// (device memory), 1 / sqrt(*norm) in place of f.
 hipError_t launch_normalize(void* psi, Prec prec, uint64_t n, uint64_t msk, uint64_t val,
-                            double f, hipStream_t s);
+                            double f, const double* norm, hipStream_t s);
 
 // dst[j] = src[insert_bit(j, pos) | keep << pos], j < n/2 (bit removal,
 // SimulatorMPI.cpp:305-321).
 hipError_t launch_remove_bit(void* dst, const void* src, Prec prec, uint64_t n_src, int pos,
                              int keep, hipStream_t s);
+// launch_two_bucket, then launch_remove_bit of the half that its result asks
+// for (bit 0 if its probability is above eps), with no wait in between; the
+// two probabilities also go to `report` (pinned host memory).  buckets: two
+// doubles of device memory.
+hipError_t launch_take_bit(void* dst, const void* src, Prec prec, int n_qubits, int pos, double eps, double* scratch,
+                           double* buckets, double* report, hipStream_t s);
 
 // dst[j] = src[i(j)] with bit p of j = bit src_pos[p] of i, for p < n_qubits.
 hipError_t launch_permute(void* dst, const void* src, Prec prec, int n_qubits,
                           const uint8_t* src_pos, hipStream_t s);
 
-// ---- reductions (FP64 accumulation; results land in device `out`) --------
-// Number of FP64 slots of scratch the reductions need.
+// ---- reductions (FP64 accumulation; results land in `out`: device memory, or
+// pinned host memory that is read after the stream has been waited for) -----
 constexpr int kReduceBlocks = 1024;
-constexpr size_t kReduceScratchDoubles = 5 * kReduceBlocks + 16;
+// Strings of one launch_pauli_expectation.
+constexpr int kPauliMasks = 8;
+struct PauliMasks {
+     uint64_t x[kPauliMasks], z[kPauliMasks];
+};
+// FP64 slots of scratch that the reductions need: partial sums of two outputs
+// per string, then a counter (cleared once by init_reduce_scratch, and zero
+// again after each reduction).  Reductions that share a scratch run on one
+// stream.
+constexpr size_t kReducePartials = 2 * kPauliMasks * kReduceBlocks;
+constexpr size_t kReduceScratchDoubles = kReducePartials + 2;
+hipError_t init_reduce_scratch(double* scratch, hipStream_t s);
 
 // out[0] = sum |psi[i]|^2 over i with (i & msk) == val.
 hipError_t launch_masked_norm(const void* psi, Prec prec, int n_qubits, uint64_t msk,
@@ -124,11 +142,10 @@ hipError_t launch_two_bucket(const void* psi, Prec prec, int n_qubits, int pos,
 // out[0] = sum p log2 p over p = |psi[i]|^2 > 0 (SimulatorMPI.cpp:681-694).
 hipError_t launch_entropy(const void* psi, Prec prec, uint64_t n, double* scratch,
                           double* out, hipStream_t s);
-// out[0..1] = sum_i conj(psi[i ^ x]) * phase(i) * psi[i],
-// phase(i) = i^{popcount(x & z)} * (-1)^{popcount(i & z)}.
-hipError_t launch_pauli_expectation(const void* psi, Prec prec, uint64_t n, uint64_t xmask,
-                                    uint64_t zmask, double* scratch, double* out,
-                                    hipStream_t s);
+// out[2t..2t+1] = sum_i conj(psi[i ^ x_t]) (-1)^{popcount(i & z_t)} psi[i] for
+// nterms <= kPauliMasks strings.
+hipError_t launch_pauli_expectation(const void* psi, Prec prec, uint64_t n, const PauliMasks& masks, int nterms,
+                                    double* scratch, double* out, hipStream_t s);
 // out[b] = sum_{j < K} |psi[b*K + j]|^2 for b < nb, K = n / nb.
 hipError_t launch_block_sums(const void* psi, Prec prec, uint64_t n, uint64_t nb, double* out,
                              hipStream_t s);

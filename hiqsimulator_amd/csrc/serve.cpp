@@ -90,6 +90,7 @@ Server::Server(Prec prec, int device, uint64_t state_bytes, uint64_t matrix_byte
      check(hipMalloc(&d_mats_, mat_entries * ab), "hipMalloc(matrices)");
      check(hipMalloc(reinterpret_cast<void**>(&d_scratch_), kReduceScratchDoubles * sizeof(double)),
            "hipMalloc(scratch)");
+     check(init_reduce_scratch(d_scratch_, stream_), "hipMemsetAsync(scratch)");
      state_pool_ = RangeAlloc(state_cap_amps_);
      mat_pool_ = RangeAlloc(mat_entries);
      mat_cap_entries_ = mat_entries;
@@ -677,9 +678,13 @@ std::vector<int64_t> Server::step(bool block)
           if (r.kind != ServeKind::Expectation) continue;
           const void* psi = static_cast<const char*>(d_states_) + r.state_off * ab;
           double* out = reinterpret_cast<double*>(slot.d_out + fo.second);
-          for (size_t t = 0; t < r.xmask.size(); ++t) {
-               check(launch_pauli_expectation(psi, prec_, uint64_t(1) << r.n, r.xmask[t], r.zmask[t],
-                                              d_scratch_, out + 2 * t, stream_),
+          for (size_t t = 0; t < r.xmask.size(); t += kPauliMasks) {
+               PauliMasks masks{};
+               const int count = static_cast<int>(std::min<size_t>(kPauliMasks, r.xmask.size() - t));
+               std::copy_n(r.xmask.begin() + static_cast<long>(t), count, masks.x);
+               std::copy_n(r.zmask.begin() + static_cast<long>(t), count, masks.z);
+               check(launch_pauli_expectation(psi, prec_, uint64_t(1) << r.n, masks, count, d_scratch_, out + 2 * t,
+                                              stream_),
                      "launch_pauli_expectation");
                ++stats_.launches;
           }
