@@ -70,6 +70,55 @@ __global__ void __launch_bounds__(BS)
      }
 }
 
+// Small states: one thread per output amplitude, with the matrix staged in LDS
+// by the whole workgroup.  The direct form gives a group to one thread, which
+// then walks the matrix by a chain of uniform loads: 13.5 us for a k = 4 pass
+// over 6 qubits, 2.5 us here.  Each output is summed in the same order.
+constexpr int kSmallBlock = 256;
+template <int K, typename R>
+__global__ void __launch_bounds__(kSmallBlock)
+    k_dense_small(typename C2<R>::T* __restrict__ psi, const typename C2<R>::T* __restrict__ mat, const DenseDesc d,
+                  const uint64_t ngroups)
+{
+     using V = typename C2<R>::T;
+     constexpr int D = 1 << K;
+     __shared__ V lm[D * D];  // [column][row]
+     const uint64_t o = static_cast<uint64_t>(blockIdx.x) * kSmallBlock + threadIdx.x;
+     const uint64_t g = o >> K;
+     const int row = static_cast<int>(o & (D - 1));
+     const bool live = g < ngroups;
+     V* const p = psi + (insert_zeros(live ? g : 0, d.ins) | d.ctrlmask);
+     V v[D];
+#pragma unroll
+     for (int j = 0; j < D; ++j) {
+          uint64_t off = 0;
+#pragma unroll
+          for (int l = 0; l < K; ++l)
+               if ((j >> l) & 1) off += 1ull << d.pos[l];
+          v[j] = p[off];
+     }
+     for (int e = threadIdx.x; e < D * D; e += kSmallBlock) lm[(e & (D - 1)) * D + (e >> K)] = mat[e];
+     __syncthreads();  // (for the matrix; a group is in one wave, which stores after all its loads)
+     R re = 0, im = 0;
+#pragma unroll
+     for (int j = 0; j < D; ++j) {
+          const V m = lm[j * D + row];
+          re = fma(m.x, v[j].x, re);
+          re = fma(-m.y, v[j].y, re);
+          im = fma(m.x, v[j].y, im);
+          im = fma(m.y, v[j].x, im);
+     }
+     if (!live) return;
+     uint64_t off = 0;
+#pragma unroll
+     for (int l = 0; l < K; ++l)
+          if ((row >> l) & 1) off += 1ull << d.pos[l];
+     V out;
+     out.x = re;
+     out.y = im;
+     p[off] = out;
+}
+
 // Wave-tile description (built on the host).  The tile index r of an
 // amplitude is its index bits at the tile positions V = (targets) + (the six
 // lowest non-inserted positions), in ascending bit order; V always holds
@@ -774,6 +823,14 @@ hipError_t dense_direct_launch(void* psi, const void* mat, const DenseDesc& d, u
      return hipGetLastError();
 }
 
+// Up to this many (log2) amplitudes under the controls a pass of k >= 2 takes
+// the small form.  Pass times with both timing events, which take 6.6 us of
+// them, direct or tile form against the small form: complex128 k = 4, 2^18
+// 25.4 / 8.7 us, 2^19 26.1 / 13.5; complex64 k = 4, 2^19 17.6 / 11.4, 2^20
+// 18.5 / 19.1; k = 3, 2^18 11.2 / 7.5 and 9.1 / 6.9, 2^19 12.2 / 10.7 and
+// 9.2 / 9.3; k = 2, 2^18 7.8 / 7.1 and 7.0 / 6.9, 2^19 9.2 / 9.7.
+constexpr int small_log(int k) { return k == 4 ? 19 : 18; }
+
 template <int K, typename R>
 hipError_t dense_k(void* psi, int n, const void* mat, const DenseDesc& d, hipStream_t s)
 {
@@ -783,6 +840,12 @@ hipError_t dense_k(void* psi, int n, const void* mat, const DenseDesc& d, hipStr
      const uint64_t ngroups = 1ull << (n - nins);
      uint64_t ins_mask = 0, tmask = 0;
      for (int i = 0; i < nins; ++i) ins_mask |= 1ull << d.ins.p[i];
+     if (K >= 2 && ngroups <= (1ull << small_log(K)) >> K) {
+          const unsigned blocks = static_cast<unsigned>(((ngroups << K) + kSmallBlock - 1) / kSmallBlock);
+          hipLaunchKernelGGL((k_dense_small<K, R>), dim3(blocks), dim3(kSmallBlock), 0, s, static_cast<V*>(psi),
+                             static_cast<const V*>(mat), d, ngroups);
+          return hipGetLastError();
+     }
      int min_t = 64;
      for (int l = 0; l < K; ++l) {
           tmask |= 1ull << d.pos[l];
