@@ -184,15 +184,13 @@ void Engine::commit_tmp()
      }
 }
 
-const void* Engine::upload_matrix(const Mat& m, const void* desc, size_t desc_bytes)
+int Engine::stage_matrix(const Mat& m, size_t& bytes)
 {
-     if (desc_bytes > kSlotBytes - kMatBytes) throw std::runtime_error("upload_matrix(): descriptor too large");
      const int slot = ring_next_;
      ring_next_ = (ring_next_ + 1) % kRing;
      if (ring_used_[slot]) check(hipEventSynchronize(ring_ev_[slot]), "hipEventSynchronize");
      char* h = h_ring_ + slot * kSlotBytes;
      const size_t n = m.dim * m.dim;
-     size_t bytes;
      if (prec_ == Prec::C128) {
           auto* o = reinterpret_cast<double*>(h);
           for (size_t i = 0; i < n; ++i) {
@@ -209,14 +207,28 @@ const void* Engine::upload_matrix(const Mat& m, const void* desc, size_t desc_by
           }
           bytes = n * 8;
      }
+     return slot;
+}
+
+void Engine::slot_queued(int slot)
+{
+     check(hipEventRecord(ring_ev_[slot], stream_), "hipEventRecord");
+     ring_used_[slot] = true;
+}
+
+const void* Engine::upload_matrix(const Mat& m, const void* desc, size_t desc_bytes)
+{
+     if (desc_bytes > kSlotBytes - kMatBytes) throw std::runtime_error("upload_matrix(): descriptor too large");
+     size_t bytes = 0;
+     const int slot = stage_matrix(m, bytes);
+     char* h = h_ring_ + slot * kSlotBytes;
      if (desc_bytes) {
           std::memcpy(h + kMatBytes, desc, desc_bytes);
           bytes = kMatBytes + desc_bytes;
      }
      char* d = d_ring_ + slot * kSlotBytes;
      check(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync(matrix)");
-     check(hipEventRecord(ring_ev_[slot], stream_), "hipEventRecord");
-     ring_used_[slot] = true;
+     slot_queued(slot);
      return d;
 }
 
@@ -565,10 +577,15 @@ void Engine::dense_or_diag(const Mat& m, const std::vector<uint32_t>& pos, uint6
           end_timed();
      }
      else if (!dense5_as_tile(m, pos, ctrlmask)) {
-          const void* dm = upload_matrix(m);
+          // A pass of a few workgroups reads its matrix from host memory.
+          const bool from_host = dense_matrix_from_host(n_qubits(), d);
+          size_t bytes = 0;
+          const int slot = from_host ? stage_matrix(m, bytes) : 0;
+          const void* dm = from_host ? h_ring_ + slot * kSlotBytes : upload_matrix(m);
           begin_timed(kDense1 + d.k - 1);
           check(launch_dense(d_state_, prec_, n_qubits(), dm, d, stream_), "dense pass");
           end_timed();
+          if (from_host) slot_queued(slot);
      }
 }
 

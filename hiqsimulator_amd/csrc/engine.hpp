@@ -220,6 +220,8 @@ private:
      void ensure_state(uint64_t n_amps);
      void ensure_tmp(uint64_t n_amps);
      void swap_tmp();
+     int stage_matrix(const Mat& m, size_t& bytes);  // fills a slot of the host ring
+     void slot_queued(int slot);                      // the work that reads it is on the stream
      const void* upload_matrix(const Mat& m, const void* desc = nullptr, size_t desc_bytes = 0);
      void dense_or_diag(const Mat& m, const std::vector<uint32_t>& pos, uint64_t ctrlmask,
                         bool diag);

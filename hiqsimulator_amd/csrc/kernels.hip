@@ -1016,6 +1016,12 @@ int tile_threads_for(Prec p, int kmax)
      return nt ? nt : (p == Prec::C64 || kmax >= 5 ? 256 : 512);
 }
 
+// Up to four workgroups of the small form.
+bool dense_matrix_from_host(int n_qubits, const DenseDesc& d)
+{
+     return d.k >= 2 && d.ins.n <= n_qubits && n_qubits - d.ins.n + d.k <= 10;
+}
+
 hipError_t launch_dense(void* psi, Prec prec, int n_qubits, const void* mat, const DenseDesc& d,
                         hipStream_t s)
 {

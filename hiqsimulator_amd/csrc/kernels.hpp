@@ -37,6 +37,9 @@ struct DenseDesc {
 // (2^k)^2 complex values in the state's precision, row-major.
 hipError_t launch_dense(void* psi, Prec prec, int n_qubits, const void* mat,
                         const DenseDesc& d, hipStream_t s);
+// True where the pass reads each matrix entry at most a few times: `mat` may
+// then be pinned host memory, which saves its copy.
+bool dense_matrix_from_host(int n_qubits, const DenseDesc& d);
 
 // The dense pass takes its direct form (instead of the LDS tile form) when
 // every target bit is at or above this position: `tile_high_target` for
