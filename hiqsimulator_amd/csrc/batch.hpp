@@ -150,9 +150,10 @@ hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, in
 // The outcome at the point u of the running probability of one state: the
 // first index whose running sum reaches u.  sums: the probabilities of its
 // 2^log_blocks blocks of 2^log_block_amps amplitudes (they become running
-// sums); out = {index, bits of the sum of all}, device or pinned host memory.
+// sums); out = {index, bits of the sum of all}, device or pinned host memory;
+// *flag becomes seq once they are there.
 hipError_t launch_measure(const void* psi, Prec prec, double* sums, int log_blocks, int log_block_amps, double u,
-                          uint64_t* out, hipStream_t s);
+                          uint64_t* out, uint64_t* flag, uint64_t seq, hipStream_t s);
 
 // ---- tile programs: many fused ops in one HBM pass --------------------------
 // A tile holds the 2^kTileBits amplitudes whose index bits outside

@@ -1219,7 +1219,8 @@ __global__ void __launch_bounds__(256)
 template <typename R>
 __global__ void __launch_bounds__(kSampleThreads)
     k_measure(const VT<R>* __restrict__ psi, double* __restrict__ sums, const int log_blocks,
-              const int log_block_amps, const double u, uint64_t* __restrict__ out)
+              const int log_block_amps, const double u, uint64_t* __restrict__ out, uint64_t* __restrict__ flag,
+              const uint64_t seq)
 {
      const uint32_t nb = 1u << log_blocks;
      running_sums(sums, nb);
@@ -1227,8 +1228,11 @@ __global__ void __launch_bounds__(kSampleThreads)
      if (threadIdx.x >= 64) return;
      const uint64_t at = find_outcome<R, true>(psi, sums, nb, 1ull << log_block_amps, u, threadIdx.x);
      if (threadIdx.x == 0) {
-          out[0] = at;
-          out[1] = static_cast<uint64_t>(__double_as_longlong(sums[nb - 1]));
+          __hip_atomic_store(out, at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          __hip_atomic_store(out + 1, static_cast<uint64_t>(__double_as_longlong(sums[nb - 1])), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_SYSTEM);
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          __hip_atomic_store(flag, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
      }
 }
 
@@ -1464,15 +1468,15 @@ hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, in
 }
 
 hipError_t launch_measure(const void* psi, Prec prec, double* sums, int log_blocks, int log_block_amps, double u,
-                          uint64_t* out, hipStream_t s)
+                          uint64_t* out, uint64_t* flag, uint64_t seq, hipStream_t s)
 {
      if (log_blocks < 0 || log_blocks > 15 || log_block_amps < 0 || log_block_amps > 40) return hipErrorInvalidValue;
      if (prec == Prec::C128)
           hipLaunchKernelGGL((k_measure<double>), dim3(1), dim3(kSampleThreads), 0, s, static_cast<const double2*>(psi),
-                             sums, log_blocks, log_block_amps, u, out);
+                             sums, log_blocks, log_block_amps, u, out, flag, seq);
      else
           hipLaunchKernelGGL((k_measure<float>), dim3(1), dim3(kSampleThreads), 0, s, static_cast<const float2*>(psi),
-                             sums, log_blocks, log_block_amps, u, out);
+                             sums, log_blocks, log_block_amps, u, out, flag, seq);
      return hipGetLastError();
 }
 

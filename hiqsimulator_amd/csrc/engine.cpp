@@ -6,6 +6,7 @@
 #include "sched.hpp"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -21,7 +22,7 @@ constexpr uint64_t kMaxBlocks = uint64_t(1) << 15;  // SimulatorMPI.cpp:903
 constexpr int kMaxOuts = 256;                        // batched reduction outputs
 // States of up to this many amplitudes lose a qubit without a wait between its
 // probabilities and the removal: below it the waits are most of the time (16
-// qubits: 21 us a qubit, 15 us now), above it the passes are.
+// qubits: 21 us a qubit, 10 us now), above it the passes are.
 constexpr uint64_t kTakeBitMax = uint64_t(1) << 20;
 
 void check(hipError_t e, const char* what)
@@ -75,9 +76,11 @@ Engine::Engine(uint64_t seed, int64_t max_local, int64_t max_cluster, Prec prec,
                      (kReduceScratchDoubles + 2 * kMaxOuts) * sizeof(double)),
            "hipMalloc(scratch)");
      check(init_reduce_scratch(d_scratch_, stream_), "hipMemsetAsync(scratch)");
-     check(hipHostMalloc(reinterpret_cast<void**>(&h_out_), 2 * kMaxOuts * sizeof(double),
+     check(hipHostMalloc(reinterpret_cast<void**>(&h_out_), (2 * kMaxOuts + 8) * sizeof(double),
                          hipHostMallocDefault),
            "hipHostMalloc(out)");
+     h_flag_ = reinterpret_cast<uint64_t*>(h_out_ + 2 * kMaxOuts);
+     *h_flag_ = 0;
      check(hipMalloc(reinterpret_cast<void**>(&d_blocks_), kMaxBlocks * sizeof(double)),
            "hipMalloc(blocks)");
      // The empty register is the one-amplitude state [1] (SimulatorMPI.cpp:96-98).
@@ -232,6 +235,23 @@ const void* Engine::upload_matrix(const Mat& m, const void* desc, size_t desc_by
      return d;
 }
 
+OutTo Engine::out_here() { return OutTo(h_out_, h_flag_, ++out_seq_); }
+
+// The results of the last out_here().  A wait for the stream takes a packet of
+// its own behind the kernel and some 5 us more than the results do, so short
+// waits watch the flag; long ones, and streams that fail, go to the runtime.
+void Engine::wait_flag()
+{
+     const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+     do {
+          for (int i = 0; i < 64; ++i) {
+               if (__atomic_load_n(h_flag_, __ATOMIC_ACQUIRE) == out_seq_) return;
+               __builtin_ia32_pause();
+          }
+     } while (std::chrono::steady_clock::now() < until);
+     wait_out();
+}
+
 void Engine::wait_out() { check(hipStreamSynchronize(stream_), "hipStreamSynchronize"); }
 
 // ---------------------------------------------------------------------------
@@ -370,13 +390,13 @@ void Engine::deallocate_qubit(int64_t id)
      begin_timed(small ? kRemoveBit : kReduce);
      if (small)
           check(launch_take_bit(d_tmp_, d_state_, prec_, n_qubits(), static_cast<int>(pos), kMaxFloatError, d_scratch_,
-                                d_scratch_ + kReduceScratchDoubles, h_out_, stream_),
+                                d_scratch_ + kReduceScratchDoubles, out_here(), stream_),
                 "take_bit");
      else
-          check(launch_two_bucket(d_state_, prec_, n_qubits(), static_cast<int>(pos), d_scratch_, h_out_, stream_),
+          check(launch_two_bucket(d_state_, prec_, n_qubits(), static_cast<int>(pos), d_scratch_, out_here(), stream_),
                 "two_bucket");
      end_timed();
-     wait_out();
+     wait_flag();
      const double s0 = h_out_[0], s1 = h_out_[1];
      if (!((s0 > kMaxFloatError) ^ (s1 > kMaxFloatError)))
           throw std::runtime_error("DeallocateLocalQubit(): qubit " + std::to_string(id)
@@ -683,9 +703,9 @@ void Engine::mask_of(const std::vector<int64_t>& ids, const std::vector<uint8_t>
 double Engine::masked_norm(uint64_t msk, uint64_t val)
 {
      begin_timed(kReduce);
-     check(launch_masked_norm(d_state_, prec_, n_qubits(), msk, val, d_scratch_, h_out_, stream_), "masked_norm");
+     check(launch_masked_norm(d_state_, prec_, n_qubits(), msk, val, d_scratch_, out_here(), stream_), "masked_norm");
      end_timed();
-     wait_out();
+     wait_flag();
      return h_out_[0];
 }
 
@@ -699,10 +719,10 @@ std::vector<uint8_t> Engine::measure(const std::vector<int64_t>& ids)
      begin_timed(kReduce);
      check(launch_block_sums(d_state_, prec_, n_amps_, uint64_t(1) << lb, d_blocks_, stream_), "block_sums");
      check(launch_measure(d_state_, prec_, d_blocks_, lb, n_qubits() - lb, u, reinterpret_cast<uint64_t*>(h_out_),
-                          stream_),
+                          h_flag_, ++out_seq_, stream_),
            "measure");
      end_timed();
-     wait_out();
+     wait_flag();
      std::memcpy(found, h_out_, sizeof(found));
      double total;
      std::memcpy(&total, &found[1], sizeof(total));
@@ -760,20 +780,9 @@ cplx Engine::get_amplitude(const std::vector<uint8_t>& bits, const std::vector<i
               "GetAmplitude(): the second argument must be a permutation of all allocated "
               "qubits.");
      settle();
-     const size_t ab = amp_bytes(prec_);
-     char* const buf = reinterpret_cast<char*>(h_out_);
-     check(hipMemcpyAsync(buf, static_cast<char*>(d_state_) + num * ab, ab, hipMemcpyDeviceToHost,
-                          stream_),
-           "hipMemcpyAsync(amplitude)");
-     check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-     if (prec_ == Prec::C128) {
-          double v[2];
-          std::memcpy(v, buf, 16);
-          return cplx(v[0], v[1]);
-     }
-     float v[2];
-     std::memcpy(v, buf, 8);
-     return cplx(v[0], v[1]);
+     check(launch_fetch(d_state_, prec_, num, out_here(), stream_), "fetch");
+     wait_flag();
+     return cplx(h_out_[0], h_out_[1]);
 }
 
 void Engine::collapse(const std::vector<int64_t>& ids, const std::vector<uint8_t>& values)
@@ -797,9 +806,9 @@ double Engine::entropy()
      DeviceScope ds(device_);
      settle();
      begin_timed(kReduce);
-     check(launch_entropy(d_state_, prec_, n_amps_, d_scratch_, h_out_, stream_), "entropy");
+     check(launch_entropy(d_state_, prec_, n_amps_, d_scratch_, out_here(), stream_), "entropy");
      end_timed();
-     wait_out();
+     wait_flag();
      return -h_out_[0];
 }
 

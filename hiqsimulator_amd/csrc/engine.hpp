@@ -232,7 +232,10 @@ private:
      int n_qubits() const { return static_cast<int>(locals_.size()); }
      void begin_timed(int cls);
      void end_timed();
-     void wait_out();  // for reductions that write h_out_
+     // Results into h_out_, announced by h_flag_: one at a time, then wait_flag.
+     OutTo out_here();
+     void wait_flag();
+     void wait_out();  // for everything on the stream
 
      Prec prec_;
      int device_;
@@ -267,6 +270,8 @@ private:
 
      double* d_scratch_ = nullptr;  // reductions + outputs
      double* h_out_ = nullptr;      // pinned: reductions write their results here
+     uint64_t* h_flag_ = nullptr;   // pinned, behind h_out_
+     uint64_t out_seq_ = 0;
      double* d_blocks_ = nullptr;   // measurement block sums (2^15)
      uint64_t* d_samples_ = nullptr;  // sample outcomes
      size_t samples_cap_ = 0;

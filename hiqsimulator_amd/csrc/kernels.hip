@@ -245,6 +245,26 @@ __global__ void __launch_bounds__(kBlock)
           dst[i] = src[i];
 }
 
+// Results of one thread: written past all caches, the flag after they are out.
+template <int N>
+__device__ __forceinline__ void put_out(const OutTo& to, const double (&v)[N], const int n = N)
+{
+#pragma unroll
+     for (int o = 0; o < N; ++o)
+          if (o < n) __hip_atomic_store(to.out + o, v[o], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+     if (to.flag) {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          __hip_atomic_store(to.flag, to.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+     }
+}
+
+template <typename R>
+__global__ void k_fetch(const typename C2<R>::T* __restrict__ psi, const uint64_t index, const OutTo to)
+{
+     const double v[2] = {static_cast<double>(psi[index].x), static_cast<double>(psi[index].y)};
+     put_out(to, v);
+}
+
 // norm: if given, the factor is 1 / sqrt(*norm) instead of f.  Amplitudes that
 // the mask drops are not read: keeping half of 2^28 complex128 amplitudes took
 // 1.34 ms with all of them read, 1.05 ms now, a quarter 0.86 ms.
@@ -287,15 +307,13 @@ template <typename R>
 __global__ void __launch_bounds__(kBlock)
     k_remove_bit(typename C2<R>::T* __restrict__ dst, const typename C2<R>::T* __restrict__ src,
                  const uint64_t n_dst, const int pos, uint64_t keep, const double* __restrict__ buckets,
-                 const double eps, double* __restrict__ report)
+                 const double eps, const OutTo report)
 {
      if (buckets) {
           const double s0 = buckets[0], s1 = buckets[1];
           keep = s0 > eps ? 0 : 1;
-          if (blockIdx.x == 0 && threadIdx.x == 0) {
-               report[0] = s0;
-               report[1] = s1;
-          }
+          const double both[2] = {s0, s1};
+          if (blockIdx.x == 0 && threadIdx.x == 0) put_out(report, both);
      }
      const uint64_t lo_mask = (1ull << pos) - 1ull;
      const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
@@ -313,7 +331,7 @@ constexpr int kTakeBitAmps = 4 * kTakeBitThreads;
 template <typename R>
 __global__ void __launch_bounds__(kTakeBitThreads)
     k_take_bit(typename C2<R>::T* __restrict__ dst, const typename C2<R>::T* __restrict__ src, const int n,
-               const int pos, const double eps, double* __restrict__ report)
+               const int pos, const double eps, const OutTo report)
 {
      using V = typename C2<R>::T;
      V a[4];
@@ -339,10 +357,7 @@ __global__ void __launch_bounds__(kTakeBitThreads)
           s[0] += red[0][w];
           s[1] += red[1][w];
      }
-     if (threadIdx.x == 0) {
-          report[0] = s[0];
-          report[1] = s[1];
-     }
+     if (threadIdx.x == 0) put_out(report, s);
      const int keep = s[0] > eps ? 0 : 1;
 #pragma unroll
      for (int u = 0; u < 4; ++u) {
@@ -473,7 +488,8 @@ __global__ void __launch_bounds__(kBlock)
 // all.  Deterministic for a given size: the order of the sums does not depend
 // on which block that is.  One launch, and the result may go straight to
 // pinned host memory: with a second kernel for the last sum and a copy of the
-// result, a probability of a 6-qubit state took 21 us, 13 us now.
+// result, a probability of a 6-qubit state took 21 us, 13 us now and 9 us with a
+// flag that the host watches.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double wave_sum(double v)
 {
@@ -506,7 +522,7 @@ __device__ __forceinline__ void block_sum(double (&acc)[NOUT], double (&red)[NOU
 // sums go to out.
 template <int NOUT>
 __device__ __forceinline__ void reduce_out(double (&acc)[NOUT], double* __restrict__ partials,
-                                           uint32_t* __restrict__ counter, double* __restrict__ out,
+                                           uint32_t* __restrict__ counter, const OutTo& out,
                                            const int nout = NOUT)
 {
      __shared__ double red[NOUT][kBlock / 64];
@@ -515,9 +531,7 @@ __device__ __forceinline__ void reduce_out(double (&acc)[NOUT], double* __restri
      block_sum<NOUT>(acc, red);
      if (threadIdx.x == 0) {
           if (nblocks == 1) {
-#pragma unroll
-               for (int o = 0; o < NOUT; ++o)
-                    if (o < nout) out[o] = acc[o];
+               put_out(out, acc, nout);
                last = false;
           }
           else {
@@ -548,9 +562,7 @@ __device__ __forceinline__ void reduce_out(double (&acc)[NOUT], double* __restri
      }
      block_sum<NOUT>(acc, red);
      if (threadIdx.x == 0) {
-#pragma unroll
-          for (int o = 0; o < NOUT; ++o)
-               if (o < nout) out[o] = acc[o];
+          put_out(out, acc, nout);
           __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
      }
 }
@@ -587,7 +599,7 @@ template <typename R>
 __global__ void __launch_bounds__(kBlock)
     k_masked_norm(const typename C2<R>::T* __restrict__ psi, const uint64_t count,
                   const InsertSet ins, const uint64_t val, double* __restrict__ partials,
-                  uint32_t* __restrict__ counter, double* __restrict__ out)
+                  uint32_t* __restrict__ counter, const OutTo out)
 {
      double acc[1] = {0.0};
      for_each_amp(psi, count, [&](uint64_t t) { return insert_zeros(t, ins) | val; },
@@ -598,7 +610,7 @@ __global__ void __launch_bounds__(kBlock)
 template <typename R>
 __global__ void __launch_bounds__(kBlock)
     k_two_bucket(const typename C2<R>::T* __restrict__ psi, const uint64_t n, const int pos,
-                 double* __restrict__ partials, uint32_t* __restrict__ counter, double* __restrict__ out)
+                 double* __restrict__ partials, uint32_t* __restrict__ counter, const OutTo out)
 {
      double acc[2] = {0.0, 0.0};
      for_each_amp(psi, n, [](uint64_t i) { return i; },
@@ -613,7 +625,7 @@ __global__ void __launch_bounds__(kBlock)
 template <typename R>
 __global__ void __launch_bounds__(kBlock)
     k_entropy(const typename C2<R>::T* __restrict__ psi, const uint64_t n,
-              double* __restrict__ partials, uint32_t* __restrict__ counter, double* __restrict__ out)
+              double* __restrict__ partials, uint32_t* __restrict__ counter, const OutTo out)
 {
      double acc[1] = {0.0};
      for_each_amp(psi, n, [](uint64_t i) { return i; },
@@ -631,7 +643,7 @@ __global__ void __launch_bounds__(kBlock)
 template <typename R>
 __global__ void __launch_bounds__(kBlock)
     k_pauli_exp(const typename C2<R>::T* __restrict__ psi, const uint64_t n, const PauliMasks masks, const int nterms,
-                double* __restrict__ partials, uint32_t* __restrict__ counter, double* __restrict__ out)
+                double* __restrict__ partials, uint32_t* __restrict__ counter, const OutTo out)
 {
      using V = typename C2<R>::T;
      double acc[2 * kPauliMasks] = {};
@@ -1096,7 +1108,7 @@ hipError_t launch_normalize(void* psi, Prec prec, uint64_t n, uint64_t msk, uint
 
 namespace {
 hipError_t remove_bit(void* dst, const void* src, Prec prec, uint64_t n_src, int pos, int keep, const double* buckets,
-                      double eps, double* report, hipStream_t s)
+                      double eps, const OutTo& report, hipStream_t s)
 {
      const uint64_t n_dst = n_src / 2;
      const unsigned grid = grid_for(n_dst, kBlock * 4);
@@ -1119,7 +1131,7 @@ hipError_t launch_remove_bit(void* dst, const void* src, Prec prec, uint64_t n_s
 }
 
 hipError_t launch_take_bit(void* dst, const void* src, Prec prec, int n_qubits, int pos, double eps, double* scratch,
-                           double* buckets, double* report, hipStream_t s)
+                           double* buckets, const OutTo& report, hipStream_t s)
 {
      if (pos < 0 || pos >= n_qubits) return hipErrorInvalidValue;
      const uint64_t n = 1ull << n_qubits;
@@ -1229,13 +1241,22 @@ hipError_t launch_pauli_accumulate(void* dst, const void* src, Prec prec, uint64
      return hipGetLastError();
 }
 
+hipError_t launch_fetch(const void* psi, Prec prec, uint64_t index, const OutTo& out, hipStream_t s)
+{
+     if (prec == Prec::C128)
+          hipLaunchKernelGGL((k_fetch<double>), dim3(1), dim3(1), 0, s, static_cast<const double2*>(psi), index, out);
+     else
+          hipLaunchKernelGGL((k_fetch<float>), dim3(1), dim3(1), 0, s, static_cast<const float2*>(psi), index, out);
+     return hipGetLastError();
+}
+
 hipError_t init_reduce_scratch(double* scratch, hipStream_t s)
 {
      return hipMemsetAsync(scratch + kReducePartials, 0, (kReduceScratchDoubles - kReducePartials) * sizeof(double), s);
 }
 
 hipError_t launch_masked_norm(const void* psi, Prec prec, int n_qubits, uint64_t msk, uint64_t val,
-                         double* scratch, double* out, hipStream_t s)
+                         double* scratch, const OutTo& out, hipStream_t s)
 {
      const InsertSet ins = ctrl_insert_set(msk);
      if (ins.n > n_qubits) return hipErrorInvalidValue;
@@ -1253,7 +1274,7 @@ hipError_t launch_masked_norm(const void* psi, Prec prec, int n_qubits, uint64_t
 }
 
 hipError_t launch_two_bucket(const void* psi, Prec prec, int n_qubits, int pos, double* scratch,
-                        double* out, hipStream_t s)
+                        const OutTo& out, hipStream_t s)
 {
      const uint64_t n = 1ull << n_qubits;
      const int grid = reduce_grid(n);
@@ -1268,7 +1289,7 @@ hipError_t launch_two_bucket(const void* psi, Prec prec, int n_qubits, int pos, 
      return hipGetLastError();
 }
 
-hipError_t launch_entropy(const void* psi, Prec prec, uint64_t n, double* scratch, double* out,
+hipError_t launch_entropy(const void* psi, Prec prec, uint64_t n, double* scratch, const OutTo& out,
                      hipStream_t s)
 {
      const int grid = reduce_grid(n);
@@ -1284,7 +1305,7 @@ hipError_t launch_entropy(const void* psi, Prec prec, uint64_t n, double* scratc
 }
 
 hipError_t launch_pauli_expectation(const void* psi, Prec prec, uint64_t n, const PauliMasks& masks, int nterms,
-                                    double* scratch, double* out, hipStream_t s)
+                                    double* scratch, const OutTo& out, hipStream_t s)
 {
      if (nterms < 1 || nterms > kPauliMasks) return hipErrorInvalidValue;
      const int grid = reduce_grid(n);

@@ -109,12 +109,23 @@ hipError_t launch_normalize(void* psi, Prec prec, uint64_t n, uint64_t msk, uint
 // SimulatorMPI.cpp:305-321).
 hipError_t launch_remove_bit(void* dst, const void* src, Prec prec, uint64_t n_src, int pos,
                              int keep, hipStream_t s);
+// Where results go, and optionally a flag in pinned host memory that becomes
+// `seq` once they are there: a host that spins on it sees them some 5 us before
+// a wait for the stream returns.
+struct OutTo {
+     double* out;
+     uint64_t* flag = nullptr;
+     uint64_t seq = 0;
+     OutTo(double* o) : out(o) {}
+     OutTo(double* o, uint64_t* f, uint64_t s) : out(o), flag(f), seq(s) {}
+};
+
 // launch_two_bucket, then launch_remove_bit of the half that its result asks
 // for (bit 0 if its probability is above eps), with no wait in between; the
 // two probabilities also go to `report` (pinned host memory).  buckets: two
 // doubles of device memory.
 hipError_t launch_take_bit(void* dst, const void* src, Prec prec, int n_qubits, int pos, double eps, double* scratch,
-                           double* buckets, double* report, hipStream_t s);
+                           double* buckets, const OutTo& report, hipStream_t s);
 
 // dst[j] = src[i(j)] with bit p of j = bit src_pos[p] of i, for p < n_qubits.
 hipError_t launch_permute(void* dst, const void* src, Prec prec, int n_qubits,
@@ -138,20 +149,23 @@ hipError_t init_reduce_scratch(double* scratch, hipStream_t s);
 
 // out[0] = sum |psi[i]|^2 over i with (i & msk) == val.
 hipError_t launch_masked_norm(const void* psi, Prec prec, int n_qubits, uint64_t msk,
-                              uint64_t val, double* scratch, double* out, hipStream_t s);
+                              uint64_t val, double* scratch, const OutTo& out, hipStream_t s);
 // out[0] = sum over i with bit pos == 0, out[1] = with bit pos == 1.
 hipError_t launch_two_bucket(const void* psi, Prec prec, int n_qubits, int pos,
-                             double* scratch, double* out, hipStream_t s);
+                             double* scratch, const OutTo& out, hipStream_t s);
 // out[0] = sum p log2 p over p = |psi[i]|^2 > 0 (SimulatorMPI.cpp:681-694).
 hipError_t launch_entropy(const void* psi, Prec prec, uint64_t n, double* scratch,
-                          double* out, hipStream_t s);
+                          const OutTo& out, hipStream_t s);
 // out[2t..2t+1] = sum_i conj(psi[i ^ x_t]) (-1)^{popcount(i & z_t)} psi[i] for
 // nterms <= kPauliMasks strings.
 hipError_t launch_pauli_expectation(const void* psi, Prec prec, uint64_t n, const PauliMasks& masks, int nterms,
-                                    double* scratch, double* out, hipStream_t s);
+                                    double* scratch, const OutTo& out, hipStream_t s);
 // out[b] = sum_{j < K} |psi[b*K + j]|^2 for b < nb, K = n / nb.
 hipError_t launch_block_sums(const void* psi, Prec prec, uint64_t n, uint64_t nb, double* out,
                              hipStream_t s);
+
+// One amplitude: its two parts, as doubles.
+hipError_t launch_fetch(const void* psi, Prec prec, uint64_t index, const OutTo& out, hipStream_t s);
 
 // psi[i] = complex Gaussian N(0,1) + i N(0,1) from Philox4x32-10 keyed by
 // `seed` with counter i (not normalised).
