@@ -52,7 +52,8 @@ def build(verbose=False):
     os.makedirs(BUILD, exist_ok=True)
     objs = []
     cmds = []
-    for src in ("kernels.hip", "batch_kernels.hip", "gate_kernels.hip", "pauli_kernels.hip", "noalloc.hip", "engine.cpp",
+    for src in ("kernels.hip", "batch_kernels.hip", "gate_kernels.hip", "pauli_kernels.hip", "readback.hip",
+                "noalloc.hip", "engine.cpp",
                 "gate_prog.cpp", "pauli_prog.cpp", "batch.cpp", "serve.cpp",
                 "capi.cpp", "sched.cpp"):
         obj = os.path.join(BUILD, src.replace(".", "_") + ".o")

@@ -962,17 +962,7 @@ void Engine::get_state_c128(std::complex<double>* out)
 {
      DeviceScope ds(device_);
      settle();
-     if (prec_ == Prec::C128) {
-          check(hipMemcpyAsync(out, d_state_, n_amps_ * 16, hipMemcpyDeviceToHost, stream_),
-                "hipMemcpyAsync(state)");
-          check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-          return;
-     }
-     std::vector<std::complex<float>> tmp(n_amps_);
-     check(hipMemcpyAsync(tmp.data(), d_state_, n_amps_ * 8, hipMemcpyDeviceToHost, stream_),
-           "hipMemcpyAsync(state)");
-     check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-     for (uint64_t i = 0; i < n_amps_; ++i) out[i] = std::complex<double>(tmp[i]);
+     readback_.read(d_state_, prec_, n_amps_, out, stream_);
 }
 
 void Engine::set_state_c128(const std::complex<double>* in, uint64_t n)

@@ -18,6 +18,7 @@
 #include <string>
 #include <vector>
 
+#include "readback.hpp"
 #include "fusion.hpp"
 #include "kernels.hpp"
 #include "pauli_prog.hpp"
@@ -270,6 +271,7 @@ private:
 
      double* d_scratch_ = nullptr;  // reductions + outputs
      double* h_out_ = nullptr;      // pinned: reductions write their results here
+     Readback readback_;
      uint64_t* h_flag_ = nullptr;   // pinned, behind h_out_
      uint64_t out_seq_ = 0;
      double* d_blocks_ = nullptr;   // measurement block sums (2^15)

@@ -88,3 +88,16 @@ def test_lists_of_strings(engine_mod, n, terms, precision):
         spec.append(([(q, ops[q]) for q in range(n)], c))
     got = sim.get_expectation_value(spec, list(range(n)))
     assert abs(got - total) <= terms * 8 * (eps(n, precision) + 2.0 ** -48)
+
+
+@pytest.mark.parametrize("precision", ["c128", "c64"])
+@pytest.mark.parametrize("n", [0, 1, 9, 10, 11, 15, 16, 17, 18])
+def test_state_comes_back(engine_mod, n, precision):
+    """One workgroup up to 2^10 amplitudes, chunks of 2^16 in two buffers above."""
+    print("readback n=%d %s" % (n, precision), flush=True)
+    if n == 0:
+        assert np.array_equal(engine_mod.SimulatorMPI(1, 4, 4, precision).get_state(), [1.0])
+        return
+    sim, psi = prepared(engine_mod, n, precision, 80 + n)
+    assert np.array_equal(sim.get_state(), psi)
+    assert np.array_equal(sim.get_state(), psi)
