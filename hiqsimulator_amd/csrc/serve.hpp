@@ -173,7 +173,10 @@ private:
      std::deque<int64_t> waiting_;
      std::vector<int64_t> active_;
      Slot slots_[kServeSlots];
-     static constexpr int kPlanners = 2;
+     // Planning is most of the host's work: a burst of 24 requests of 12 to 24
+     // qubits in complex64 took 13.5 ms with 2 threads, 9.7 ms with 4 and 10.5
+     // ms with 8.
+     static constexpr int kPlanners = 4;
      std::vector<std::thread> planners_;
      std::mutex qmu_;
      std::condition_variable qcv_;
