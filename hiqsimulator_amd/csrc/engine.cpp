@@ -1561,8 +1561,17 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
           ProgSlot& ps = upload_pauli(plan, terms);
           void* cur = w;
           void* next = t1.p;
-          // (at least one product, so that the sum is formed)
-          for (size_t k = 1; k < std::max<size_t>(bes.size(), 2); ++k) {
+          // (at least one product, so that the sum is formed.)  The sum takes
+          // two polynomials at a time, the one a product reads and the one it
+          // makes: every second product neither reads nor writes it.
+          const size_t last = std::max<size_t>(bes.size(), 2) - 1;
+          // J_0(z), 2 J_k(z) (-i sign t)^k
+          auto weight = [&](size_t k) {
+               if (k == 0) return cplx(bes[0], 0);
+               const int e = static_cast<int>(k & 3);
+               return 2.0 * (k < bes.size() ? bes[k] : 0.0) * ipow(t < 0 ? e : (4 - e) & 3);
+          };
+          for (size_t k = 1; k <= last; ++k) {
                for (size_t p = 0; p < plan.passes.size(); ++p) {
                     PauliApply q;
                     q.src = cur;
@@ -1575,14 +1584,14 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
                          q.add = next;  // T_{k-2}
                          q.g = -1.0;
                     }
-                    if (p + 1 == plan.passes.size()) {
-                         q.o_src = k == 1 ? w : out;
+                    if (p + 1 == plan.passes.size() && (k % 2 == 1 || k == last)) {
+                         q.o_src = k == 1 ? nullptr : out;
                          q.o_dst = out;
-                         q.h = k == 1 ? bes[0] : 1.0;
-                         // 2 J_k(z) (-i sign t)^k
-                         const cplx c = 2.0 * (k < bes.size() ? bes[k] : 0.0) * (t < 0 ? ipow(static_cast<int>(k & 3)) : ipow(static_cast<int>((4 - (k & 3)) & 3)));
+                         const cplx c = weight(k), e = k % 2 == 1 ? weight(k - 1) : cplx(0, 0);
                          q.cr = c.real();
                          q.ci = c.imag();
+                         q.er = e.real();
+                         q.ei = e.imag();
                     }
                     check(launch_pauli_apply(q, prec_, n_qubits(), plan.passes[p], terms, stream_), "pauli_apply");
                }

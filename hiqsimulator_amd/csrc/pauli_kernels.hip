@@ -215,7 +215,7 @@ struct ApplyArgs {
      VT<R>* o_dst;
      const double* skip;
      double skip_below;
-     R fr, fi, g, h, cr, ci;
+     R fr, fi, g, h, cr, ci, er, ei;
 };
 
 template <typename R, int A>
@@ -282,9 +282,17 @@ __global__ void __launch_bounds__(kPauliThreads)
                b.y = fma(a.g, d[k].y, b.y);
                a.dst[i] = b;
                if (a.o_dst) {
-                    V s = a.o_src[i];
-                    s.x = fma(-a.ci, b.y, fma(a.cr, b.x, a.h * s.x));
-                    s.y = fma(a.ci, b.x, fma(a.cr, b.y, a.h * s.y));
+                    const V e = tile[k * kPauliThreads + tid];
+                    V s;
+                    s.x = fma(-a.ei, e.y, a.er * e.x);
+                    s.y = fma(a.ei, e.x, a.er * e.y);
+                    if (a.o_src) {
+                         const V t = a.o_src[i];
+                         s.x = fma(a.h, t.x, s.x);
+                         s.y = fma(a.h, t.y, s.y);
+                    }
+                    s.x = fma(-a.ci, b.y, fma(a.cr, b.x, s.x));
+                    s.y = fma(a.ci, b.x, fma(a.cr, b.y, s.y));
                     a.o_dst[i] = s;
                     const double br = b.x, bi = b.y;
                     norm = fma(br, br, fma(bi, bi, norm));
@@ -337,6 +345,8 @@ void apply_launch(const PauliApply& a, const PauliPass& p, const PauliTerm* t, u
      k.h = static_cast<R>(a.h);
      k.cr = static_cast<R>(a.cr);
      k.ci = static_cast<R>(a.ci);
+     k.er = static_cast<R>(a.er);
+     k.ei = static_cast<R>(a.ei);
      hipLaunchKernelGGL((k_pauli_apply<R, A>), dim3(grid), dim3(kPauliThreads), 0, s, k, p, t, ntiles, a.norm ? a.scratch : nullptr);
 }
 
@@ -368,7 +378,7 @@ hipError_t launch_pauli_sum(const void* psi, Prec prec, int n, const PauliPass& 
 hipError_t launch_pauli_apply(const PauliApply& a, Prec prec, int n, const PauliPass& pass, const PauliTerm* terms,
                               hipStream_t s)
 {
-     if (!pass_fits(pass, n) || a.src == a.dst || (a.o_dst && !a.o_src) || (a.norm && (!a.o_dst || !a.scratch)))
+     if (!pass_fits(pass, n) || a.src == a.dst || (a.norm && (!a.o_dst || !a.scratch)))
           return hipErrorInvalidValue;
      const uint64_t ntiles = 1ull << (n - pauli_tile_bits(n));
      const int grid = static_cast<int>(ntiles < kReduceBlocks ? ntiles : kReduceBlocks);

@@ -76,8 +76,8 @@ hipError_t launch_pauli_sum(const void* psi, Prec prec, int n, const PauliPass& 
                             double* scratch, double* out, hipStream_t s);
 
 // dst = f * (the pass's share of the sum applied to src) + g * add (add may be
-// dst; dst != src).  With o_dst: o_dst = h * o_src + c * dst afterwards (o_src
-// may be o_dst), and with norm: norm[0] = |dst|^2 (through scratch).  With
+// dst; dst != src).  With o_dst: o_dst = h * o_src + e * src + c * dst
+// afterwards (o_src may be o_dst, or null for zero), and with norm: norm[0] = |dst|^2 (through scratch).  With
 // skip: nothing is done when skip[0] < skip_below, and norm[0] = skip[0].
 struct PauliApply {
      const void* src = nullptr;
@@ -87,7 +87,7 @@ struct PauliApply {
      double g = 1;
      const void* o_src = nullptr;
      void* o_dst = nullptr;
-     double h = 1, cr = 1, ci = 0;
+     double h = 1, cr = 1, ci = 0, er = 0, ei = 0;
      const double* skip = nullptr;
      double skip_below = 0;
      double* scratch = nullptr;
