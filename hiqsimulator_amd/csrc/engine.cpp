@@ -450,11 +450,21 @@ void Engine::permute_qubits(const std::vector<int64_t>& ids)
      if (seen != (ids.empty() ? 0 : ((uint64_t(1) << ids.size()) - 1)))
           throw std::runtime_error("permute_qubits(): ids must be a permutation of the qubits");
      if (identity) return;
-     settle();
-     ensure_tmp(n_amps_);
-     begin_timed(kPermute);
-     check(launch_permute(d_tmp_, d_state_, prec_, n_qubits(), src.data(), stream_), "permute");
-     end_timed();
+     // Gates that are still queued run first; the last of their passes stores
+     // the state permuted when it can.
+     bool permuted = false;
+     if (!queue_.empty()) {
+          ensure_tmp(n_amps_);
+          int passes = 0;
+          (void)gate_items(queue_, 0, passes, src.data(), &permuted);
+     }
+     if (!permuted) {
+          settle();
+          ensure_tmp(n_amps_);
+          begin_timed(kPermute);
+          check(launch_permute(d_tmp_, d_state_, prec_, n_qubits(), src.data(), stream_), "permute");
+          end_timed();
+     }
      commit_tmp();
      locals_ = ids;
 }
@@ -1143,7 +1153,7 @@ void Engine::program_done(ProgSlot& ps)
      ps.busy = true;
 }
 
-bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes)
+bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, const uint8_t* src_pos, bool* permuted)
 {
      passes = 0;
      const int n = n_qubits();
@@ -1161,7 +1171,9 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes)
           std::vector<char> ops;
           while (gp.size() < group && planner.remaining().size() > keep && planner.next(plan)) {
                gp.emplace_back();
-               compile_gate_pass(units, plan, n, prec_, gp.back(), stages, ops);
+               // the last pass may store the state permuted
+               const bool perm = src_pos && planner.remaining().empty() && widen_for_permutation(units, plan, n, prec_, src_pos);
+               compile_gate_pass(units, plan, n, prec_, gp.back(), stages, ops, perm ? src_pos : nullptr);
           }
           for (const auto& p: gp) check_gate_pass(p, stages, ops, prec_, n);
           const size_t stage_bytes = (stages.size() * sizeof(GateStage) + 255) / 256 * 256;
@@ -1173,9 +1185,10 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes)
           for (const auto& p: gp) {
                begin_timed(kTile);
                check(launch_gate_pass(d_state_, prec_, n, p, reinterpret_cast<const GateStage*>(ps.d), ps.d + stage_bytes,
-                                      stream_),
+                                      stream_, p.permuted ? d_tmp_ : d_state_),
                      "gate pass");
                end_timed();
+               if (p.permuted) *permuted = true;
                ++passes;
           }
           program_done(ps);

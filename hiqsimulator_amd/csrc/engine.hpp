@@ -202,7 +202,10 @@ private:
      // The same by gate programs (gate_prog.hpp), for states of at least
      // gate_min_qubits and lists whose gates mix at most two qubits each;
      // false (and nothing done) for others.
-     bool gate_items(std::vector<PosGate>& items, size_t keep, int& passes);
+     // src_pos: the last pass also permutes the index bits (launch_permute) into
+     // d_tmp_ if it can; *permuted tells.
+     bool gate_items(std::vector<PosGate>& items, size_t keep, int& passes, const uint8_t* src_pos = nullptr,
+                     bool* permuted = nullptr);
      // A free staging slot of at least `bytes`; waits for the launches of
      // kProgSlots groups ago.
      struct ProgSlot;

@@ -531,9 +531,10 @@ __device__ __forceinline__ uint64_t reg_index(int k, const uint8_t (&pos)[kGateM
 // moves real and imaginary parts separately; tied to the loads' registers the
 // whole array ends up twice in the register file, and spills.
 template <typename R>
-__device__ __forceinline__ void gate_program(VT<R>* __restrict__ psi, const GatePass& P,
+__device__ __forceinline__ void gate_program(VT<R>* psi, const GatePass& P,
                                              const GateStage* __restrict__ stages,
-                                             const GateOp<R>* __restrict__ ops, const uint64_t tix, char* lds)
+                                             const GateOp<R>* __restrict__ ops, const uint64_t tix, char* lds,
+                                             VT<R>* dst)
 {
      using V = VT<R>;
      constexpr int E = Shape<R>::E, A = 1 << E, H = Shape<R>::T - kGateLow;
@@ -563,7 +564,13 @@ __device__ __forceinline__ void gate_program(VT<R>* __restrict__ psi, const Gate
           slot = to;
           run_ops<R>(x, ops + st.op_first, st.nops, base, tid);
      } while (++s < P.nstages);
-     V* const p = psi + base + thread_index(fresh(tid), P.out_thr);
+     uint64_t to = base;
+     if (P.permuted) {
+          to = 0;
+#pragma unroll
+          for (int j = 0; j < kGateMaxBase; ++j) to |= ((tix >> j) & 1) << P.base_out[j];
+     }
+     V* const p = dst + to + thread_index(fresh(tid), P.out_thr);
 #pragma unroll
      for (int k = 0; k < A; ++k) {
           st_nt(p + reg_index(k, P.out_reg), copy_amp(x[k]));
@@ -573,20 +580,22 @@ __device__ __forceinline__ void gate_program(VT<R>* __restrict__ psi, const Gate
 
 template <typename R>
 __global__ void __launch_bounds__(kGateThreads) __attribute__((amdgpu_waves_per_eu(4)))
-    k_gate_pass(VT<R>* __restrict__ psi, const GatePass P, const GateStage* __restrict__ stages,
-                const GateOp<R>* __restrict__ ops, const int swz, const uint64_t nblocks)
+    k_gate_pass(VT<R>* psi, const GatePass P, const GateStage* __restrict__ stages,
+                const GateOp<R>* __restrict__ ops, const int swz, const uint64_t nblocks, VT<R>* dst)
 {
      __shared__ __align__(16) char lds[sizeof(R) << Shape<R>::T];
      const uint64_t b = block_linear();
      if (b >= nblocks) return;  // padding of the 2-D grid (whole block)
-     gate_program<R>(psi, P, stages + P.stage_first, ops, swizzle_block(b, swz), lds);
+     gate_program<R>(psi, P, stages + P.stage_first, ops, swizzle_block(b, swz), lds, dst);
 }
 
 }  // namespace
 
 hipError_t launch_gate_pass(void* psi, Prec prec, int n_qubits, const GatePass& pass, const GateStage* stages,
-                            const void* ops, hipStream_t s)
+                            const void* ops, hipStream_t s, void* dst)
 {
+     if (pass.permuted ? (!dst || dst == psi) : (dst && dst != psi)) return hipErrorInvalidValue;
+     if (!dst) dst = psi;
      const int T = gate_tile_bits(prec);
      if (n_qubits < T || n_qubits > 40 || pass.nstages < 1) return hipErrorInvalidValue;
      for (int j = 0; j < T - kGateLow; ++j)
@@ -598,11 +607,11 @@ hipError_t launch_gate_pass(void* psi, Prec prec, int n_qubits, const GatePass& 
      if (prec == Prec::C128)
           hipLaunchKernelGGL((k_gate_pass<double>), grid_2d(blocks), dim3(kGateThreads), 0, s,
                              static_cast<double2*>(psi), pass, stages, static_cast<const GateOp<double>*>(ops), swz,
-                             blocks);
+                             blocks, static_cast<double2*>(dst));
      else
           hipLaunchKernelGGL((k_gate_pass<float>), grid_2d(blocks), dim3(kGateThreads), 0, s,
                              static_cast<float2*>(psi), pass, stages, static_cast<const GateOp<float>*>(ops), swz,
-                             blocks);
+                             blocks, static_cast<float2*>(dst));
      return hipGetLastError();
 }
 

@@ -264,9 +264,9 @@ struct Layout {
 // The thread order of a stage whose register ranks are given.  The first five
 // (complex64: six) lane bits get ranks with independent low slot bits, so that
 // 32 lanes of 8 bytes or 64 of 4 hit distinct banks;
-// `io`: lanes 0..3 are ranks 0..3, so that the stage's grouping can be loaded
-// and stored in runs of 16 amplitudes.
-Layout make_layout(Prec prec, const std::vector<int>& reg, bool io)
+// `io`: lanes 0..3 are these ranks (0..3 to load), so that the stage's
+// grouping can be loaded or stored in runs of 16 amplitudes; null: any.
+Layout make_layout(Prec prec, const std::vector<int>& reg, const int* io)
 {
      Layout L{};
      bool in_reg[kGateMaxTile] = {};
@@ -278,24 +278,25 @@ Layout make_layout(Prec prec, const std::vector<int>& reg, bool io)
      const size_t want = prec == Prec::C128 ? 5 : 6;
      std::vector<int> lanes, rest;
      uint32_t basis[6] = {0, 0, 0, 0, 0, 0};  // basis[b]: vector with leading bit b
-     for (int r = 0; r < gate_tile_bits(prec); ++r) {
-          if (in_reg[r]) {
-               if (io && r < kGateLow) throw std::runtime_error("gate program: internal layout error");
-               continue;
-          }
+     std::vector<int> order;
+     for (int q = 0; io && q < kGateLow; ++q) {
+          if (in_reg[io[q]]) throw std::runtime_error("gate program: internal layout error");
+          order.push_back(io[q]);
+     }
+     for (int r = 0; r < gate_tile_bits(prec); ++r)
+          if (!in_reg[r] && std::find(order.begin(), order.end(), r) == order.end()) order.push_back(r);
+     const size_t runs = io ? kGateLow : 0;  // lanes that are given, independent or not
+     for (size_t q = 0; q < order.size(); ++q) {
+          const int r = order[q];
           uint32_t v = gate_slot(prec, r) & low;
           for (int b = 5; b >= 0; --b)
                if ((v >> b) & 1) {
                     if (!basis[b]) break;
                     v ^= basis[b];
                }
-          if (v && lanes.size() < want) {
-               basis[31 - __builtin_clz(v)] = v;
-               lanes.push_back(r);
-          }
-          else {
-               rest.push_back(r);
-          }
+          const bool lane = q < runs || (v && lanes.size() < want);
+          if (lane && v) basis[31 - __builtin_clz(v)] = v;
+          (lane ? lanes : rest).push_back(r);
      }
      lanes.insert(lanes.end(), rest.begin(), rest.end());
      if (lanes.size() != static_cast<size_t>(kGateThr)) throw std::runtime_error("gate program: internal layout error");
@@ -306,7 +307,7 @@ Layout make_layout(Prec prec, const std::vector<int>& reg, bool io)
 class Compiler {
 public:
      Compiler(const std::vector<GateUnit>& units, const GatePassPlan& plan, int n, Prec prec, GatePass& pass,
-              std::vector<GateStage>& stages, std::vector<char>& ops)
+              std::vector<GateStage>& stages, std::vector<char>& ops, const uint8_t* src_pos)
          : units_(units),
            plan_(plan),
            prec_(prec),
@@ -328,6 +329,14 @@ public:
           if (r != T_) throw std::runtime_error("gate program: internal tile error");
           for (int q = 0; q < kGateLow; ++q)
                if (pos_[q] != q) throw std::runtime_error("gate program: internal tile error");
+          for (int q = 0; q < kGateLow; ++q) {
+               in_lanes_[q] = q;
+               out_lanes_[q] = src_pos ? rank_[src_pos[q]] : q;
+               if (out_lanes_[q] < 0) throw std::runtime_error("gate program: internal tile error");
+          }
+          for (int p = 0; p < n; ++p) new_pos_[src_pos ? src_pos[p] : p] = static_cast<uint8_t>(p);
+          permuted_ = src_pos != nullptr;
+          n_ = n;
           if (ops_.size() >= ob_) ops_.resize(ops_.size() - ob_);  // the spare record moves to the end
      }
 
@@ -337,24 +346,40 @@ public:
           pass_.stage_first = static_cast<uint32_t>(stages_.size());
           for (int j = 0; j < T_ - kGateLow; ++j) pass_.hpos[j] = static_cast<uint8_t>(pos_[kGateLow + j]);
           const size_t ns = plan_.stages.size();
-          std::vector<int> top;
-          for (int r = T_ - E_; r < T_; ++r) top.push_back(r);
-          auto low = [](const std::vector<int>& reg) { return *std::min_element(reg.begin(), reg.end()) < kGateLow; };
           std::vector<std::vector<int>> regs;
-          for (size_t s = 0; s < ns; ++s) regs.push_back(reg_ranks(plan_.regs[s]));
-          // a first or last stage whose registers hold low ranks is loaded or
-          // stored through an empty stage
-          if (low(regs.front())) {
-               begin_stage(top, true);
+          for (size_t s = 0; s < ns; ++s)
+               regs.push_back(reg_ranks(plan_.regs[s], permuted_ && s + 1 == ns ? out_lanes_ : nullptr));
+          // a first or last stage whose registers hold ranks of the load's or
+          // the store's runs is loaded or stored through an empty stage, and
+          // so is a single stage whose runs are not the same ones
+          const bool in_empty = holds(regs.front(), in_lanes_);
+          if (in_empty) {
+               begin_stage(reg_ranks(0, nullptr), in_lanes_);
                set_io(pass_.in_thr, pass_.in_reg);
           }
+          bool stored = false;
           for (size_t s = 0; s < ns; ++s) {
-               begin_stage(regs[s], !low(regs[s]) && (s == 0 || s + 1 == ns));
+               const int* io = nullptr;
+               if (s == 0 && !in_empty) io = in_lanes_;
+               else if (s + 1 == ns && !holds(regs[s], out_lanes_)) io = out_lanes_;
+               begin_stage(regs[s], io);
                if (pass_stages() == 1) set_io(pass_.in_thr, pass_.in_reg);
                emit_stage(plan_.stages[s], s + 1 == ns);
+               stored = s + 1 == ns && io && std::equal(io, io + kGateLow, out_lanes_);
           }
-          if (low(regs.back())) begin_stage(top, true);
+          if (!stored) begin_stage(reg_ranks(0, permuted_ ? out_lanes_ : nullptr), out_lanes_);
           set_io(pass_.out_thr, pass_.out_reg);
+          if (permuted_) {
+               for (int j = 0; j < kGateThr; ++j) pass_.out_thr[j] = new_pos_[pass_.out_thr[j]];
+               for (int b = 0; b < E_; ++b) pass_.out_reg[b] = new_pos_[pass_.out_reg[b]];
+               int j = 0;
+               for (int p = 0; p < n_; ++p)
+                    if (!((plan_.bits >> p) & 1)) {
+                         if (j >= kGateMaxBase) throw std::runtime_error("gate program: internal tile error");
+                         pass_.base_out[j++] = new_pos_[p];
+                    }
+               pass_.permuted = 1;
+          }
           if (pass_stages() > kGateMaxStages) throw std::runtime_error("gate program: too many stages");
           pass_.nstages = static_cast<uint8_t>(pass_stages());
           ops_.resize(ops_.size() + ob_, 0);  // the spare record
@@ -385,8 +410,15 @@ private:
 
      size_t pass_stages() const { return stages_.size() - pass_.stage_first; }
 
-     // Register ranks of a stage, filled up from the top ranks.
-     std::vector<int> reg_ranks(uint64_t bits) const
+     static bool holds(const std::vector<int>& reg, const int* lanes)
+     {
+          return std::any_of(lanes, lanes + kGateLow,
+                             [&](int r) { return std::find(reg.begin(), reg.end(), r) != reg.end(); });
+     }
+
+     // Register ranks of a stage, filled up from the top ranks (that are not
+     // among `avoid`).
+     std::vector<int> reg_ranks(uint64_t bits, const int* avoid) const
      {
           std::vector<int> reg;
           for (uint64_t m = bits; m; m &= m - 1) {
@@ -396,12 +428,14 @@ private:
           }
           if (reg.size() > static_cast<size_t>(E_)) throw std::runtime_error("gate program: internal stage error");
           for (int r = T_ - 1; r >= 0 && reg.size() < static_cast<size_t>(E_); --r)
-               if (std::find(reg.begin(), reg.end(), r) == reg.end()) reg.push_back(r);
+               if (std::find(reg.begin(), reg.end(), r) == reg.end() &&
+                   !(avoid && std::find(avoid, avoid + kGateLow, r) != avoid + kGateLow))
+                    reg.push_back(r);
           std::sort(reg.begin(), reg.end());
           return reg;
      }
 
-     void begin_stage(const std::vector<int>& reg, bool io)
+     void begin_stage(const std::vector<int>& reg, const int* io)
      {
           lay_ = make_layout(prec_, reg, io);
           const uint32_t sb = gate_slot_bytes(prec_);
@@ -770,6 +804,10 @@ private:
      std::vector<GateStage>& stages_;
      std::vector<char>& ops_;
      int rank_[64], pos_[kGateMaxTile];
+     int in_lanes_[kGateLow], out_lanes_[kGateLow];  // ranks of the load's and the store's runs
+     uint8_t new_pos_[64] = {};                      // of an index bit, after the permutation
+     bool permuted_ = false;
+     int n_ = 0;
      int tbit_[64], rbit_[64];
      Layout lay_{};
      size_t nops_ = 0;
@@ -783,9 +821,24 @@ private:
 }  // namespace
 
 void compile_gate_pass(const std::vector<GateUnit>& units, const GatePassPlan& plan, int n, Prec prec, GatePass& pass,
-                       std::vector<GateStage>& stages, std::vector<char>& ops)
+                       std::vector<GateStage>& stages, std::vector<char>& ops, const uint8_t* src_pos)
 {
-     Compiler(units, plan, n, prec, pass, stages, ops).run();
+     Compiler(units, plan, n, prec, pass, stages, ops, src_pos).run();
+}
+
+bool widen_for_permutation(const std::vector<GateUnit>& units, GatePassPlan& plan, int n, Prec prec,
+                           const uint8_t* src_pos)
+{
+     uint64_t bits = (uint64_t(1) << kGateLow) - 1;
+     for (const auto& st: plan.stages)
+          for (int i: st) bits |= units[i].a;
+     for (int q = 0; q < kGateLow; ++q) bits |= uint64_t(1) << src_pos[q];
+     const int T = gate_tile_bits(prec);
+     if (popc(bits) > T) return false;
+     for (uint64_t m = plan.bits & ~bits; m && popc(bits) < T; m &= m - 1) bits |= low_bit(m);
+     for (int p = 0; p < n && popc(bits) < T; ++p) bits |= uint64_t(1) << p;
+     plan.bits = bits;
+     return true;
 }
 
 void check_gate_pass(const GatePass& pass, const std::vector<GateStage>& stages, const std::vector<char>& ops,
@@ -807,7 +860,13 @@ void check_gate_pass(const GatePass& pass, const std::vector<GateStage>& stages,
           uint64_t got = 0;
           for (int j = 0; j < kGateThr; ++j) got |= uint64_t(1) << thr[j];
           for (int b = 0; b < E; ++b) got |= uint64_t(1) << reg[b];
-          if (got != bits) fail();
+          uint64_t want = bits;
+          if (io && pass.permuted) {  // every bit of the new index once
+               if (n - T > kGateMaxBase) fail();
+               for (int j = 0; j < n - T; ++j) got |= uint64_t(1) << pass.base_out[j];
+               want = (uint64_t(1) << n) - 1;
+          }
+          if (got != want) fail();
      }
      for (int s = 0; s < pass.nstages; ++s) {
           const GateStage& st = stages[pass.stage_first + s];

@@ -97,6 +97,7 @@ void interpret(State& psi, int n, const GatePass& P, const std::vector<GateStage
           return s / gate_slot_bytes(prec);
      };
      std::vector<cplx> x(size_t(kGateThreads) * A), lds(size_t(1) << T);
+     State other(P.permuted ? psi.size() : 0, cplx(NAN, NAN));  // where a permuted pass stores
      for (uint64_t tix = 0; tix < (uint64_t(1) << (n - T)); ++tix) {
           uint64_t base = tix << kGateLow;
           for (int j = 0; j < T - kGateLow; ++j) {
@@ -214,9 +215,14 @@ void interpret(State& psi, int n, const GatePass& P, const std::vector<GateStage
                     }
                }
           }
+          const uint64_t to = P.permuted ? bits(static_cast<uint32_t>(tix), P.base_out, n - T) : base;
           for (uint32_t t = 0; t < kGateThreads; ++t)
-               for (uint32_t k = 0; k < A; ++k) psi.at(base + bits(t, P.out_thr, kGateThr) + bits(k, P.out_reg, E)) = x[t * A + k];
+               for (uint32_t k = 0; k < A; ++k)
+                    (P.permuted ? other : psi).at(to + bits(t, P.out_thr, kGateThr) + bits(k, P.out_reg, E)) = x[t * A + k];
+          // runs of 16 amplitudes are loaded and stored by 16 lanes
+          for (int j = 0; j < kGateLow; ++j) CHECK(P.in_thr[j] == j && P.out_thr[j] == j);
      }
+     if (P.permuted) psi.swap(other);
 }
 
 struct Maker {
@@ -305,7 +311,10 @@ struct Maker {
      }
 };
 
-void run_case(int n, int ngates, int span, int first, Prec prec, unsigned seed, size_t min_passes = 1)
+// permute: the last pass also takes the bits of the index to other places, if
+// it can; returns whether it did.
+bool run_case(int n, int ngates, int span, int first, Prec prec, unsigned seed, size_t min_passes = 1,
+              bool permute = false)
 {
      Maker mk{std::mt19937(seed), n};
      mk.first = first;
@@ -328,14 +337,32 @@ void run_case(int n, int ngates, int span, int first, Prec prec, unsigned seed, 
      std::vector<char> ops;
      std::vector<GatePass> passes;
      std::vector<int> seen(units.size(), 0);
+     std::vector<uint8_t> src_pos;
+     bool permuted = false;
+     if (permute) {
+          for (int q: mk.qubits(n, n)) src_pos.push_back(static_cast<uint8_t>(q));
+          CHECK(src_pos.size() == static_cast<size_t>(n));
+     }
      while (planner.next(plan)) {
+          const uint64_t tile = plan.bits;
+          permuted = permute && planner.remaining().empty() && widen_for_permutation(units, plan, n, prec, src_pos.data());
+          if (!permuted) CHECK(plan.bits == tile);
           for (size_t s = 0; s < plan.stages.size(); ++s) {
                CHECK(!(plan.regs[s] & ~plan.bits));
                for (int i: plan.stages[s]) ++seen[i];
           }
           GatePass p;
-          compile_gate_pass(units, plan, n, prec, p, stages, ops);
+          compile_gate_pass(units, plan, n, prec, p, stages, ops, permuted ? src_pos.data() : nullptr);
           passes.push_back(p);
+     }
+     if (permuted) {
+          State moved(ref.size());
+          for (uint64_t i = 0; i < ref.size(); ++i) {
+               uint64_t from = 0;
+               for (int p = 0; p < n; ++p) from |= ((i >> p) & 1) << src_pos[p];
+               moved[i] = ref[from];
+          }
+          ref.swap(moved);
      }
      for (int c: seen) CHECK(c == 1);
      CHECK(passes.size() >= min_passes);
@@ -357,6 +384,7 @@ void run_case(int n, int ngates, int span, int first, Prec prec, unsigned seed, 
                        static_cast<int>(prec), seed, err, norm);
           std::exit(1);
      }
+     return permuted;
 }
 
 }  // namespace
@@ -372,6 +400,17 @@ int main()
                for (int f: {0, 4, n - 5}) run_case(n, 60, 5, f, prec, seed++);  // few qubits: long stages
           }
           run_case(18, 80, 18, 0, prec, seed++, 2);
+     }
+     // the last pass permutes
+     seed = 1000;
+     for (Prec prec: {Prec::C128, Prec::C64}) {
+          const int T = gate_tile_bits(prec);
+          for (int r = 0; r < 8; ++r) CHECK(run_case(T, 1 + 9 * r, T, 0, prec, seed++, 1, true));  // one tile: always
+          int did = 0;
+          for (int n: {T + 1, 17, 18})
+               for (int r = 0; r < 8; ++r) did += run_case(n, 1 + 12 * r, n, 0, prec, seed++, 1, true);
+          for (int f: {0, 4, 12}) did += run_case(17, 60, 5, f, prec, seed++, 1, true);
+          CHECK(did >= 8 && did < 27);  // both outcomes
      }
      // more gates than one stage or one pass holds
      {

@@ -87,3 +87,33 @@ def test_long_gate_list_on_few_qubits(engine_mod, oracle_mod):
     sim.allocate_qureg(list(range(n)), 0)
     assert sim.apply_tiled(gates, 4) >= 1
     assert np.abs(sim.get_state() - oracle_state(oracle_mod, n, gates)).max() <= 1e-12
+
+
+@pytest.mark.parametrize("n", [13, 14, 15, 18, 21])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_last_pass_permutes(engine_mod, oracle_mod, n, pinned):
+    """Permutations right behind queued gates: the last pass stores the state
+    permuted where its tile has room, and a pass of its own does where not."""
+    rng = np.random.default_rng(n)
+    parts = [gates_of(n, c, 60 + n + c) for c in (3, 16, 40)]
+    perms = [[int(q) for q in rng.permutation(n)] for _ in range(3)]
+    perms[1] = perms[1][:4] + sorted(perms[1][4:])
+    ref = oracle_state(oracle_mod, n, [g for part in parts for g in part])
+    # ids are qubits: the state's bit p holds qubit perms[-1][p]
+    i, src = np.arange(1 << n), np.zeros(1 << n, dtype=np.int64)
+    for p, q in enumerate(perms[-1]):
+        src |= ((i >> p) & 1) << q
+    ref = ref[src]
+    for prec in ("c128", "c64"):
+        print("permuting passes n=%d %s pinned=%d" % (n, prec, pinned), flush=True)
+        sim = engine_mod.SimulatorMPI(1, n, 5, prec)
+        sim.allocate_qureg(list(range(n)), 0)
+        view = sim.state_dlpack() if pinned else None  # results go back into the viewed buffer
+        for gates, order in zip(parts, perms):
+            apply_circuit_inorder(sim, gates, 5)
+            sim.permute_qubits(order)
+        sim.synchronize()
+        psi = sim.get_state()
+        tol = 1e-12 if prec == "c128" else 8 * 2.0 ** -23 * sum(map(len, parts)) * np.abs(ref).max()
+        assert np.abs(psi - ref).max() <= tol
+        del view
