@@ -1,7 +1,11 @@
 // gfx950 kernels of the planned Pauli sums (pauli_prog.hpp).
 //
 // Bound: HBM for a few groups a pass (one read of the state; apply: a read
-// and one or two writes more), vector issue beyond about twenty terms.
+// and one or two writes more), vector issue and LDS beyond about twenty terms.
+// Before, every term was a pass of its own.  Expectation of 101 terms (26
+// qubits, complex128): 101 passes of 0.2 ms, 3 of 0.36 ms now, 0.17 ms of each
+// for the read; evolution under 39 terms (20 qubits): 2883 passes, 57 of 13.9
+// us now.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -26,11 +30,11 @@ __device__ __forceinline__ T load_words(const T* __restrict__ p)
 }
 
 // Where a tile lies and where a thread's amplitudes lie in it: amplitude k of
-// thread t is tile rank index k * 512 + t.
-template <int A>
+// thread t is tile rank index k * 2^THR + t.
+template <int A, int THR>
 struct TileAt {
      static constexpr int KB = A == 8 ? 3 : (A == 4 ? 2 : (A == 2 ? 1 : 0));
-     static constexpr int H = kPauliThr + KB - kPauliLow;
+     static constexpr int H = THR + KB - kPauliLow;
      uint64_t lane;   // index bits of the thread
      uint64_t reg[A]; // index bits of the amplitude number (uniform)
 
@@ -38,13 +42,13 @@ struct TileAt {
      {
           lane = tid & ((1u << kPauliLow) - 1u);
 #pragma unroll
-          for (int j = 0; j < kPauliThr - kPauliLow; ++j)
+          for (int j = 0; j < THR - kPauliLow; ++j)
                lane |= static_cast<uint64_t>((tid >> (kPauliLow + j)) & 1u) << P.hpos[j];
 #pragma unroll
           for (int k = 0; k < A; ++k) {
                uint64_t o = 0;
 #pragma unroll
-               for (int j = 0; j < KB; ++j) o |= static_cast<uint64_t>((k >> j) & 1) << P.hpos[kPauliThr - kPauliLow + j];
+               for (int j = 0; j < KB; ++j) o |= static_cast<uint64_t>((k >> j) & 1) << P.hpos[THR - kPauliLow + j];
                reg[k] = o;
           }
      }
@@ -69,8 +73,10 @@ __device__ __forceinline__ double amp_sign(int k, uint32_t zk)
 // Runs the records of a pass on one tile: done(t, w) for every group, t its
 // last record and w[k] = sum over its terms of c (-1)^{|i & z|} for amplitude
 // k.  The sign splits into the tile's (uniform), the thread's and the
-// amplitude number's (uniform).
-template <int A, typename Done>
+// amplitude number's (uniform).  Classes (terms that share the amplitude
+// number's part) are those of kPauliThr thread bits, which is right for more
+// of them, too.
+template <int A, int THR, typename Done>
 __device__ __forceinline__ void run_terms(const PauliTerm* __restrict__ terms, const uint32_t count, const uint64_t base,
                                           const uint32_t tid, Done&& done)
 {
@@ -83,10 +89,10 @@ __device__ __forceinline__ void run_terms(const PauliTerm* __restrict__ terms, c
           __builtin_amdgcn_sched_barrier(0);
           const PauliTerm nxt = load_words(terms + t + 1);  // (one spare record at the end)
           const uint32_t uni = static_cast<uint32_t>(__popcll(base & cur.z_out));
-          const uint32_t sgn = (__popc(tid & cur.z_tile & (kPauliThreads - 1u)) + uni) << 31;
+          const uint32_t sgn = (__popc(tid & cur.z_tile & ((1u << THR) - 1u)) + uni) << 31;
           v += __hiloint2double(__double2hiint(cur.c) ^ static_cast<int>(sgn), __double2loint(cur.c));
           if (cur.z_tile & kPauliClassEnd) {
-               const uint32_t zk = (cur.z_tile & 0xffffu) >> kPauliThr;
+               const uint32_t zk = (cur.z_tile & 0xffffu) >> THR;
 #pragma unroll
                for (int k = 0; k < A; ++k) w[k] = fma(v, amp_sign(k, zk), w[k]);
                v = 0;
@@ -131,7 +137,7 @@ __global__ void __launch_bounds__(kPauliThreads)
      __shared__ V tile[kPauliThreads * A];
      const uint32_t tid = threadIdx.x;
      const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tid)));
-     const TileAt<A> at(P, tid);
+     const TileAt<A, kPauliThr> at(P, tid);
      double acc[2] = {0.0, 0.0};
      for (uint64_t tix = blockIdx.x; tix < ntiles; tix += gridDim.x) {
           const uint64_t base = at.base(P, tix);
@@ -142,7 +148,7 @@ __global__ void __launch_bounds__(kPauliThreads)
 #pragma unroll
           for (int k = 0; k < A; ++k) tile[k * kPauliThreads + tid] = x[k];
           __syncthreads();
-          run_terms<A>(terms + P.first, P.count, base, tid, [&](const PauliTerm& t, const double (&w)[A]) {
+          run_terms<A, kPauliThr>(terms + P.first, P.count, base, tid, [&](const PauliTerm& t, const double (&w)[A]) {
                const bool im = t.z_tile & kPauliImag;
                double s = 0;
                // the half that the highest bit of x selects (pauli_prog.cpp)
@@ -218,16 +224,17 @@ struct ApplyArgs {
      R fr, fi, g, h, cr, ci, er, ei;
 };
 
-template <typename R, int A>
-__global__ void __launch_bounds__(kPauliThreads)
+template <typename R, int A, int THR>
+__global__ void __launch_bounds__(1 << THR)
     k_pauli_apply(const ApplyArgs<R> a, const PauliPass P, const PauliTerm* __restrict__ terms,
                   const uint64_t ntiles, double* __restrict__ partials)
 {
      using V = VT<R>;
+     constexpr int kThreads = 1 << THR;
      if (a.skip && a.skip[0] < a.skip_below) return;  // the whole grid
-     __shared__ V tile[kPauliThreads * A];
+     __shared__ V tile[kThreads * A];
      const uint32_t tid = threadIdx.x;
-     const TileAt<A> at(P, tid);
+     const TileAt<A, THR> at(P, tid);
      double norm = 0;
      for (uint64_t tix = blockIdx.x; tix < ntiles; tix += gridDim.x) {
           const uint64_t base = at.base(P, tix);
@@ -237,7 +244,7 @@ __global__ void __launch_bounds__(kPauliThreads)
           __syncthreads();  // the previous tile has been read
 #pragma unroll
           for (int k = 0; k < A; ++k) {
-               tile[k * kPauliThreads + tid] = o[k];
+               tile[k * kThreads + tid] = o[k];
                o[k].x = o[k].y = 0;
           }
           V d[A];  // what the result is added to, on its way meanwhile
@@ -248,7 +255,7 @@ __global__ void __launch_bounds__(kPauliThreads)
                for (int k = 0; k < A; ++k) d[k] = a.add[base + at.lane + at.reg[k]];
           }
           __syncthreads();
-          run_terms<A>(terms + P.first, P.count, base, tid, [&](const PauliTerm& t, const double (&w)[A]) {
+          run_terms<A, THR>(terms + P.first, P.count, base, tid, [&](const PauliTerm& t, const double (&w)[A]) {
                // two one-sided ifs on a flag the compiler cannot relate: an
                // if-else would keep the sums before and after both alive
                uint32_t real = ~t.z_tile & kPauliImag;
@@ -256,7 +263,7 @@ __global__ void __launch_bounds__(kPauliThreads)
                if (real) {
 #pragma unroll
                     for (int k = 0; k < A; ++k) {
-                         const V y = tile[(k * kPauliThreads + tid) ^ t.x];
+                         const V y = tile[(k * kThreads + tid) ^ t.x];
                          const R v = static_cast<R>(w[k]);
                          o[k].x = fma(v, y.x, o[k].x);
                          o[k].y = fma(v, y.y, o[k].y);
@@ -265,7 +272,7 @@ __global__ void __launch_bounds__(kPauliThreads)
                if (t.z_tile & kPauliImag) {
 #pragma unroll
                     for (int k = 0; k < A; ++k) {
-                         const V y = tile[(k * kPauliThreads + tid) ^ t.x];
+                         const V y = tile[(k * kThreads + tid) ^ t.x];
                          const R v = static_cast<R>(w[k]);
                          o[k].x = fma(-v, y.y, o[k].x);
                          o[k].y = fma(v, y.x, o[k].y);
@@ -282,7 +289,7 @@ __global__ void __launch_bounds__(kPauliThreads)
                b.y = fma(a.g, d[k].y, b.y);
                a.dst[i] = b;
                if (a.o_dst) {
-                    const V e = tile[k * kPauliThreads + tid];
+                    const V e = tile[k * kThreads + tid];
                     V s;
                     s.x = fma(-a.ei, e.y, a.er * e.x);
                     s.y = fma(a.ei, e.x, a.er * e.y);
@@ -301,12 +308,12 @@ __global__ void __launch_bounds__(kPauliThreads)
      }
      if (!partials) return;
      for (int d = 32; d > 0; d >>= 1) norm += __shfl_xor(norm, d, 64);
-     __shared__ double red[kPauliThreads / 64];
+     __shared__ double red[kThreads / 64];
      if ((tid & 63) == 0) red[tid >> 6] = norm;
      __syncthreads();
      if (tid == 0) {
           double v = 0;
-          for (int i = 0; i < kPauliThreads / 64; ++i) v += red[i];
+          for (int i = 0; i < kThreads / 64; ++i) v += red[i];
           partials[blockIdx.x] = v;
      }
 }
@@ -347,7 +354,18 @@ void apply_launch(const PauliApply& a, const PauliPass& p, const PauliTerm* t, u
      k.ci = static_cast<R>(a.ci);
      k.er = static_cast<R>(a.er);
      k.ei = static_cast<R>(a.ei);
-     hipLaunchKernelGGL((k_pauli_apply<R, A>), dim3(grid), dim3(kPauliThreads), 0, s, k, p, t, ntiles, a.norm ? a.scratch : nullptr);
+     // One workgroup a CU at most: twice the threads, half the amplitudes each,
+     // hide more of each other's latency (20 qubits, complex128: 14.8 us a pass
+     // with 512 threads, 13.9 us with 1024).  With more tiles two workgroups of
+     // 512 share a CU and overlap.
+     if constexpr (A > 1)
+          if (ntiles <= 256) {
+               hipLaunchKernelGGL((k_pauli_apply<R, A / 2, kPauliThr + 1>), dim3(grid), dim3(2 * kPauliThreads), 0, s, k, p,
+                                  t, ntiles, a.norm ? a.scratch : nullptr);
+               return;
+          }
+     hipLaunchKernelGGL((k_pauli_apply<R, A, kPauliThr>), dim3(grid), dim3(kPauliThreads), 0, s, k, p, t, ntiles,
+                        a.norm ? a.scratch : nullptr);
 }
 
 // f<A>() for the amplitudes a thread of an n-qubit state's tile holds.
