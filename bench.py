@@ -699,8 +699,8 @@ def main():
     dense_ms_step = sum(ms for name, (c, ms) in times.items() if name.startswith("dense")) / args.steps
     del sim
 
-    # The same gates with tile passes (the cluster scheduler targeting the
-    # LDS tile): fewer HBM passes, each applying several fused ops.  Run on a
+    # The same gates through apply_tiled: fewer HBM passes, each applying many
+    # gates to tiles of the state.  Run on a
     # fresh state without the permutations; compared with the fused passes'
     # kernel time of the run above.
     tile = None
@@ -723,7 +723,8 @@ def main():
         tile_ms = ttot / tcnt if tcnt else float("nan")
         # Algorithmic flops of the ops (8 * 2^k per amplitude per op; ops of
         # 3+ qubits run on the matrix cores when tile_mfma is on), from the
-        # same tile plan apply_tiled makes on this fresh state.
+        # tile plan of this fresh state.  A list that runs gate by gate takes
+        # other passes than that plan: it has no such ops.
         pass_of, op_of, _ = hq._cppsim_amd.plan_tile_passes([g[1] for g in gates], [g[2] for g in gates], n, tw)
         support = {}
         for gi, (p, o) in enumerate(zip(pass_of, op_of)):
@@ -732,16 +733,17 @@ def main():
                 m |= 1 << q
             support[(p, o)] = support.get((p, o), 0) | m
         widths = [bin(m).count("1") for m in support.values()]
-        mfma_flop = sum(8.0 * 2 ** w * 2 ** n for w in widths if w >= 3)
+        fused = tp == max(pass_of) + 1
+        mfma_flop = sum(8.0 * 2 ** w * 2 ** n for w in widths if w >= 3) if fused else None
         tile = {"hbm_passes_per_circuit": tp, "fused_passes_per_circuit": n_pass,
                 "ms_per_circuit": round(el_t / args.steps * 1e3, 2),
                 "fused_pass_kernel_ms_per_circuit": round(dense_ms_step, 2),
                 "speedup_vs_fused_kernels": round(dense_ms_step / (el_t / args.steps * 1e3), 3),
                 "tile_pass_avg_ms": round(tile_ms, 4),
                 "tile_pass_hbm_gbs": round(32.0 * 2 ** n / (tile_ms * 1e-3) / 1e9, 1),
-                "op_width": tw, "ops_per_circuit": len(widths),
+                "op_width": tw if fused else None, "ops_per_circuit": len(widths) if fused else None,
                 "mfma_flop_per_circuit": mfma_flop,
-                "mfma_tflops": round(mfma_flop / (tile_ms * 1e-3 * tp) / 1e12, 2) if tp else None,
+                "mfma_tflops": round(mfma_flop / (tile_ms * 1e-3 * tp) / 1e12, 2) if fused and tp else None,
                 "final_norm": ts.get_probability([], [])}
         del ts
         log("tile passes: %s" % tile)
