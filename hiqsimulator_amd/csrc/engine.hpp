@@ -63,9 +63,8 @@ public:
      // the reference does.  In kPassDeferred mode (the default) the gates of
      // a cluster of at most 5 qubits with its controls, on a state of 12 or
      // more qubits, are queued instead (unfused, on bit positions); queued
-     // gates run as tile passes (several clusters per HBM pass, planned with
-     // the tile as the local set and fused per tile op) once kQueueHigh of
-     // them wait, and all of them before any call that reads the state,
+     // gates run as gate or tile passes (several clusters per HBM pass, as
+     // apply_tiled) once kQueueHigh of them wait, and all of them before any call that reads the state,
      // changes the qubit set or order, or synchronizes.  The width check (at
      // most 5 qubits) still raises here.
      void run();
@@ -149,16 +148,18 @@ public:
      // Pauli sum (masks over ids, as above).  The reference's engine calls
      // this for ProjectQ's TimeEvolution gate (_simulator_mpi.py:469-475)
      // but its C++ never defines it.  Identity terms become a phase; the
-     // rest is a Taylor series in s = ceil(|t| sum|c|) steps, each summed
-     // until a term's norm drops below 1e-12 (at most 64 terms).
+     // rest is a Chebyshev series for real coefficients and planned sums
+     // (pauli_prog.hpp), else a Taylor series in s = ceil(|t| sum|c|) steps,
+     // each summed until a term's norm drops below 1e-12 (at most 64 terms).
      void time_evolution(const std::vector<uint64_t>& xm, const std::vector<uint64_t>& zm,
                          const std::vector<cplx>& coeff, double t, const std::vector<int64_t>& ids,
                          const std::vector<int64_t>& ctrls);
 
      // Applies a gate list (ids as in apply_gate; matrices 2^t x 2^t with t
-     // targets) with tile passes: each HBM pass loads tiles of index bits
-     // {0..5} + 6 planned bits into LDS and applies every op of its plan
-     // there (ops of at most op_width qubits, fused in FP64 on the host).
+     // targets) as gate programs where they can be (gate_items), otherwise
+     // with tile passes: each HBM pass loads tiles of index bits {0..5} + 6
+     // planned bits into LDS and applies every op of its plan there (ops of
+     // at most op_width qubits, fused in FP64 on the host).
      // Pending gates are run first.  Below 12 qubits the ops run as plain
      // fused passes.  Returns the number of HBM passes.
      struct Gate {
@@ -190,9 +191,9 @@ private:
           Mat m;
           std::vector<int64_t> t, c;
      };
-     // Runs every queued cluster (tile passes).
+     // Runs every queued cluster.
      void settle() { drain_queue(0); }
-     // Applies queued clusters as tile passes until at most `keep` remain.
+     // Applies queued clusters as gate or tile passes until at most `keep` remain.
      void drain_queue(size_t keep);
      // Plans `items` into tile passes and launches them while more than
      // `keep` items are left unplanned; the launched items are removed from

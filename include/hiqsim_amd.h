@@ -72,10 +72,9 @@ int hiqsim_run(hiqsim_t* h);
  *     reference's Run() (SimulatorMPI.cpp:441-541);
  *   HIQSIM_PASS_DEFERRED (1, the default): on a state of 12 or more qubits
  *     the gates of a cluster of at most 5 qubits with its controls are
- *     queued (unfused); queued gates run as tile passes, several clusters
- *     per HBM pass, planned with the LDS tile as the local set and fused per
- *     tile op (as hiqsim_apply_tiled), once 512 of them wait (down to 256)
- *     and before any call that reads the state, changes the qubit set or the
+ *     queued (unfused); queued gates run as gate or tile passes, several
+ *     clusters per HBM pass (as hiqsim_apply_tiled), once 512 of them wait
+ *     (down to 256) and before any call that reads the state, changes the qubit set or the
  *     qubit order, or synchronizes.  Results equal the reference's within
  *     floating-point rounding.
  * get: *mode, and *queued = gates waiting (queued may be NULL). */
@@ -203,8 +202,10 @@ int hiqsim_apply_pauli_sum(hiqsim_t* h, const uint64_t* xmask, const uint64_t* z
  * TimeEvolution gate, never defined in the reference's C++): psi <- exp(-i
  * time H) psi on the subspace where every ctrls qubit is 1, H the Pauli sum
  * as above (Hermitian for a unitary result).  Identity terms become a phase;
- * the rest is a Taylor series in ceil(|time| sum|coeff|) steps, each summed
- * until a term's norm is below 1e-12. */
+ * the rest is a Chebyshev series in H / sum|coeff| to 1e-17 for real
+ * coefficients (on 9 or more qubits, X parts within 12 index bits, |time|
+ * sum|coeff| up to 1e6), otherwise a Taylor series in ceil(|time| sum|coeff|)
+ * steps, each summed until a term's norm is below 1e-12. */
 int hiqsim_emulate_time_evolution(hiqsim_t* h, const uint64_t* xmask, const uint64_t* zmask,
                                   const double* coeff, size_t nterms, double time, const int64_t* ids,
                                   size_t nids, const int64_t* ctrls, size_t nctrls);
@@ -259,11 +260,14 @@ int hiqsim_plan_clusters(const int64_t* gate_ids, const size_t* gate_off, const 
 /* Applies a gate list with tile passes (no reference counterpart; the
  * reference applies one fused cluster per state pass, SimulatorMPI::Run,
  * SimulatorMPI.cpp:441-541).  Gates as in hiqsim_batch_add_circuit but on
- * the handle's qubit ids.  Each HBM pass loads tiles of index bits {0..5}
- * plus 6 planned bits into LDS and applies there every op its plan holds
- * (ops of at most op_width qubits, fused in FP64); the plan is the cluster
- * scheduler's rule with the tile as the local set.  Pending gates are run
- * first.  *npasses = HBM passes used. */
+ * the handle's qubit ids.  From 13 qubits on in complex128 and 21 in
+ * complex64, lists whose gates mix at most two qubits each (controls and
+ * block-diagonal targets do not count) run gate by gate on tiles of 2^13 or
+ * 2^14 amplitudes in registers.  Otherwise each HBM pass loads tiles of index
+ * bits {0..5} plus 6 planned bits into LDS and applies there every op its plan
+ * holds (ops of at most op_width qubits, fused in FP64); the plan is the
+ * cluster scheduler's rule with the tile as the local set.  Pending gates are
+ * run first.  *npasses = HBM passes used. */
 int hiqsim_apply_tiled(hiqsim_t* h, size_t ngates, const double* mats, const int64_t* tgt_ids,
                        const size_t* tgt_off, const int64_t* ctrl_ids, const size_t* ctrl_off,
                        int op_width, int* npasses);
