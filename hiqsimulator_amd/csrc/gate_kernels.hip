@@ -267,32 +267,78 @@ __device__ __forceinline__ void op_two(V (&x)[A], const GateOp<R>* __restrict__ 
      }
 }
 
-// The two doubles a list record holds at the start of its coefficients.
-template <typename R>
-__device__ __forceinline__ double2 list_factor(const GateOp<R>& o)
+// An opcode whose value the compiler takes as unknown at each use.
+__device__ __forceinline__ uint32_t opaque_code(uint32_t c)
 {
-     double2 f;
-     __builtin_memcpy(&f, o.c, sizeof(f));
-     return f;
+     asm volatile("" : "+s"(c));
+     return c;
+}
+
+// What a list needs of a record: its conditions and the two doubles at the
+// start of its coefficients.  The scalar unit moves every word of a record
+// that is loaded ahead, and has as much to do here as the vector unit.
+struct ListRecord {
+     uint32_t tcond;
+     uint64_t omask, oval;
+     double fx, fy;
+};
+template <typename R>
+__device__ __forceinline__ ListRecord load_list_record(const GateOp<R>* __restrict__ p)
+{
+     const uint32_t* const q = reinterpret_cast<const uint32_t*>(p);
+     uint32_t w[9];
+#pragma unroll
+     for (int i = 0; i < 9; ++i) w[i] = q[i + 1];
+     ListRecord r;
+     r.tcond = w[0];
+     __builtin_memcpy(&r.omask, w + 1, 8);
+     __builtin_memcpy(&r.oval, w + 3, 8);
+     __builtin_memcpy(&r.fx, w + 5, 8);
+     __builtin_memcpy(&r.fy, w + 7, 8);
+     return r;
 }
 
 // The product of the factors of ops[0..count) whose conditions hold for this
-// thread's tile and index.  In FP64 for either type: a list multiplies one
-// amplitude by many factors, and their rounded moduli would add up.
+// thread's tile and index; with tables > 0, the list begins with those.  In
+// FP64 for either type: a list multiplies one amplitude by many factors, and
+// their rounded moduli would add up.
 template <typename V, typename R>
 __device__ __forceinline__ V factor_product(const GateOp<R>* __restrict__ ops, uint32_t count, uint64_t base,
-                                            uint32_t tid)
+                                            uint64_t tix, uint32_t tid, uint32_t tables)
 {
      double2 f = make_double2(1, 0);
-     GateOp<R> cur = load_record(ops);
+     if (tables) {
+          const double* t = reinterpret_cast<const double*>(ops);
+          const uint32_t lane = tid & (kGateTableLanes - 1u);
+          const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tid / kGateTableLanes)));
+          f.x = t[2 * lane];
+          f.y = t[2 * lane + 1];
+          t += 2 * kGateTableLanes;
+          cmul(f, t[2 * wave], t[2 * wave + 1]);
+          t += 2 * kGateTableWaves;
+          uint32_t left = static_cast<uint32_t>(tix);  // (n <= 40: 27 bits at most)
+          for (uint32_t g = 1; g < tables; ++g) {
+               const uint32_t i = left & ((1u << kGateTableBits) - 1u);
+               cmul(f, t[2 * i], t[2 * i + 1]);
+               t += 2 << kGateTableBits;
+               left >>= kGateTableBits;
+          }
+          const uint32_t skip = static_cast<uint32_t>((gate_table_entries(static_cast<int>(tables) - 1) * 16 + sizeof(GateOp<R>) - 1) / sizeof(GateOp<R>));
+          ops += skip;
+          count -= skip;
+     }
+     ListRecord cur = load_list_record(ops);  // (a list is never the last record)
+#pragma unroll 2
      for (uint32_t e = 0; e < count; ++e) {
           asm volatile("" : "+s"(cur.tcond));
           __builtin_amdgcn_sched_barrier(0);
-          const GateOp<R> nxt = load_record(ops + e + 1);  // (a list is never the last record)
+          const ListRecord nxt = load_list_record(ops + e + 1);
           if ((base & cur.omask) == cur.oval) {  // uniform
-               const bool on = (tid & (cur.tcond & 0xffffu)) == (cur.tcond >> 16);
-               const double2 u = list_factor(cur);
-               cmul(f, on ? u.x : 1.0, on ? u.y : 0.0);
+               if (cur.tcond == 0) cmul(f, cur.fx, cur.fy);
+               if (opaque_code(cur.tcond) != 0) {
+                    const bool on = (tid & (cur.tcond & 0xffffu)) == (cur.tcond >> 16);
+                    cmul(f, on ? cur.fx : 1.0, on ? cur.fy : 0.0);
+               }
           }
           cur = nxt;
      }
@@ -308,13 +354,6 @@ __device__ __forceinline__ void pin(V (&x)[A])
 {
 #pragma unroll
      for (int k = 0; k < A; ++k) asm volatile("" : "+v"(x[k].x), "+v"(x[k].y));
-}
-
-// An opcode whose value the compiler takes as unknown at each use.
-__device__ __forceinline__ uint32_t opaque_code(uint32_t c)
-{
-     asm volatile("" : "+s"(c));
-     return c;
 }
 
 #define HQ_IN(LO, HI) if (opaque_code(code) - static_cast<uint32_t>(LO) < static_cast<uint32_t>((HI) - (LO)))
@@ -389,7 +428,7 @@ __device__ __forceinline__ void run_layer(V (&x)[A], const GateOp<R>& o, const G
 // which takes their registers twice and spills.
 template <typename R, typename V, int A>
 __device__ __forceinline__ void run_ops(V (&x)[A], const GateOp<R>* __restrict__ ops, const uint32_t nops,
-                                        const uint64_t base, const uint32_t tid)
+                                        const uint64_t base, const uint64_t tix, const uint32_t tid)
 {
      constexpr int E = Shape<R>::E;
      if (nops == 0) return;
@@ -427,7 +466,7 @@ __device__ __forceinline__ void run_ops(V (&x)[A], const GateOp<R>* __restrict__
                     HQ_AT(kGatePT) { op_phase_tested(x, cur.c[0], cur.c[1], rm, rv); }
                     HQ_IN(kGatePA, kGateG2)
                     {
-                         const V f = factor_product<V, R>(list, count, base, tid);
+                         const V f = factor_product<V, R>(list, count, base, tix, tid, rm);
                          HQ_BITS(kGatePA, op_phase<B>(x, f.x, f.y))
                          HQ_AT(kGatePL) { op_phase<-1>(x, f.x, f.y); }
                     }
@@ -566,7 +605,7 @@ __device__ __forceinline__ void gate_program(VT<R>* psi, const GatePass& P,
           const uint32_t to = thread_slot(tid, st.thr_lds);
           if (s > 0) regroup<R>(x, lds, slot, to, load_record(stages + s - 1).reg_lds, st.reg_lds);
           slot = to;
-          run_ops<R>(x, ops + st.op_first, st.nops, base, tid);
+          run_ops<R>(x, ops + st.op_first, st.nops, base, tix, tid);
      } while (++s < P.nstages);
      uint64_t to = base;
      if (P.permuted) {

@@ -336,6 +336,7 @@ public:
           }
           for (int p = 0; p < n; ++p) new_pos_[src_pos ? src_pos[p] : p] = static_cast<uint8_t>(p);
           permuted_ = src_pos != nullptr;
+          for (int p = 0, j = 0; p < n; ++p) outer_[p] = rank_[p] < 0 ? j++ : -1;
           n_ = n;
           if (ops_.size() >= ob_) ops_.resize(ops_.size() - ob_);  // the spare record moves to the end
      }
@@ -657,18 +658,65 @@ private:
      {
           put_phases(kGatePA + static_cast<uint32_t>(b), ph_[b]);
      }
-     // A list of conditional factors, in as many ops as it takes.
+     // A list of conditional factors, in as many ops as it takes; the first one
+     // begins with tables of the factors that depend on the lane, on the wave or
+     // on five bits of the tile number alone, when there are four or more of them.
      void put_phases(uint32_t code, std::vector<Phase>& v)
      {
-          for (size_t i = 0; i < v.size();) {
-               const size_t k = std::min<size_t>(v.size() - i, kGateMaxList);
-               put(code, Cond(), nullptr, 0, static_cast<uint32_t>(k));
+          const int groups = gate_table_groups(prec_, n_);
+          const uint32_t lanes = kGateTableLanes - 1;
+          // the table of a condition (-1: none): its first entry, its size, and the bits and value asked there
+          struct Place {
+               int first = -1, size = 0;
+               uint64_t m = 0, on = 0;
+          };
+          auto place = [&](const Cond& c) {
+               Place r;
+               if (!c.om && !(c.tm & ~lanes)) r = {0, kGateTableLanes, c.tm, c.tv};
+               else if (!c.om && !(c.tm & lanes)) r = {kGateTableLanes, kGateTableWaves, c.tm / kGateTableLanes, c.tv / kGateTableLanes};
+               else if (!c.tm) {
+                    uint64_t m = 0, on = 0;
+                    for (uint64_t q = c.om; q; q &= q - 1) {
+                         const int p = __builtin_ctzll(q);
+                         m |= uint64_t(1) << outer_[p];
+                         on |= ((c.ov >> p) & 1) << outer_[p];
+                    }
+                    const int g = __builtin_ctzll(m) / kGateTableBits, at = g * kGateTableBits;
+                    if (m >> at >> kGateTableBits == 0)
+                         r = {kGateTableLanes + kGateTableWaves + (g << kGateTableBits), 1 << kGateTableBits, m >> at, on >> at};
+               }
+               return r;
+          };
+          auto tabled = [&](const Phase& p) { return place(p.c).first >= 0; };
+          const bool table = std::count_if(v.begin(), v.end(), tabled) >= 4;
+          std::vector<cplx> t(table ? gate_table_entries(groups) : 0, cplx(1.0, 0.0));
+          if (table) {
+               for (const auto& p: v) {
+                    const Place r = place(p.c);
+                    for (int i = 0; r.first >= 0 && i < r.size; ++i)
+                         if ((static_cast<uint64_t>(i) & r.m) == r.on) t[r.first + i] *= p.f;
+               }
+               v.erase(std::remove_if(v.begin(), v.end(), tabled), v.end());
+          }
+          const uint32_t block = prec_ == Prec::C128 ? gate_table_records<double>(groups) : gate_table_records<float>(groups);
+          for (size_t i = 0; i < v.size() || (table && i == 0);) {
+               const bool here = table && i == 0;
+               const size_t taken = here ? block : 0;
+               const size_t k = std::min<size_t>(v.size() - i, kGateMaxList - taken);
+               put(code, Cond(), nullptr, 0, static_cast<uint32_t>(taken + k), here ? 1u + static_cast<uint32_t>(groups) : 0u);
+               if (here) {
+                    const size_t at = ops_.size();
+                    ops_.resize(at + taken * ob_, 0);
+                    std::memcpy(ops_.data() + at, t.data(), t.size() * 16);
+                    nops_ += taken;
+               }
                for (size_t e = 0; e < k; ++e, ++i) {
                     const Cond& c = v[i].c;
                     put_raw(0, c.tm | c.tv << 16, c.om, c.ov, nullptr, 0);
                     const double f[2] = {v[i].f.real(), v[i].f.imag()};  // FP64 in either precision
                     std::memcpy(ops_.data() + ops_.size() - ob_ + offsetof(GateOp<float>, c), f, sizeof(f));
                }
+               if (here && k == 0) break;
           }
           v.clear();
      }
@@ -806,6 +854,7 @@ private:
      int rank_[64], pos_[kGateMaxTile];
      int in_lanes_[kGateLow], out_lanes_[kGateLow];  // ranks of the load's and the store's runs
      uint8_t new_pos_[64] = {};                      // of an index bit, after the permutation
+     int outer_[64];  // an index bit's place in the tile number
      bool permuted_ = false;
      int n_ = 0;
      int tbit_[64], rbit_[64];
@@ -896,7 +945,13 @@ void check_gate_pass(const GatePass& pass, const std::vector<GateStage>& stages,
                std::memcpy(&w, ops.data() + (st.op_first + p) * ob, 4);
                std::memcpy(&tc, ops.data() + (st.op_first + p) * ob + 4, 4);
                if ((w & 0xff) >= kGateCodes || ((w & 0xff) == kGateLayer && tc > 16)) fail();
-               p += 1 + ((w >> 8) & 0xff);
+               const uint32_t code = w & 0xff, count = (w >> 8) & 0xff;
+               if (code >= kGatePA && code < kGateG2 && (w >> 16)) {
+                    const int g = static_cast<int>(w >> 16) - 1;
+                    if (g != gate_table_groups(prec, n)) fail();
+                    if (count < (prec == Prec::C128 ? gate_table_records<double>(g) : gate_table_records<float>(g))) fail();
+               }
+               p += 1 + count;
                if (p > st.nops) fail();
           }
      }

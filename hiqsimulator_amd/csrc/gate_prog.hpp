@@ -89,6 +89,21 @@ enum GateKind : uint32_t {
 // Register pairs of kGateG2: (0,1) (0,2) (1,2) (0,3) (1,3) (2,3) (0,4) (1,4) (2,4) (3,4).
 constexpr uint32_t gate_pair(int b0, int b1) { return static_cast<uint32_t>(b1 * (b1 - 1) / 2 + b0); }
 constexpr uint32_t kGateMaxList = 255;  // `count` is a byte
+// A list (kGatePA, kGatePL) whose aux is 1 + g begins with tables in the place
+// of records: the products of its factors whose conditions are on lane bits
+// only, for each of the 64 lanes; on wave bits only, for each of the 8 waves;
+// and on bits 5 i .. 5 i + 4 of the tile number only, for each of their 32
+// values, i < g (g covers the whole number).  Pairs of doubles.  A factor from
+// a record takes some sixteen vector and thirty scalar instructions; a table
+// takes one load and one product.  Worth it from four such factors on: the QFT
+// of 29 qubits in complex64 took 12.7 ms with records, 10.7 ms with tables.
+constexpr int kGateTableLanes = 64, kGateTableWaves = kGateThreads / 64;
+constexpr int kGateTableBits = 5;
+constexpr int gate_table_groups(Prec p, int n) { return (n - gate_tile_bits(p) + kGateTableBits - 1) / kGateTableBits; }
+constexpr size_t gate_table_entries(int groups)
+{
+     return kGateTableLanes + kGateTableWaves + (static_cast<size_t>(groups) << kGateTableBits);
+}
 
 // One op.  But for layers it applies where (tile base index & omask) == oval,
 // (thread & tmask) == tval and, for the ops that say so, (amplitude &
@@ -103,6 +118,12 @@ struct GateOp {
 static_assert(sizeof(GateOp<double>) == 104 && sizeof(GateOp<float>) == 64 &&
                   offsetof(GateOp<double>, c) == offsetof(GateOp<float>, c),
               "record sizes");
+// Records that the tables take the place of.
+template <typename R>
+constexpr uint32_t gate_table_records(int groups)
+{
+     return static_cast<uint32_t>((gate_table_entries(groups) * 16 + sizeof(GateOp<R>) - 1) / sizeof(GateOp<R>));
+}
 inline size_t gate_op_bytes(Prec p) { return p == Prec::C128 ? sizeof(GateOp<double>) : sizeof(GateOp<float>); }
 
 // One stage: LDS byte offsets of the thread bits and the register bits (the

@@ -64,9 +64,22 @@ void apply(State& psi, const Gate& g)
 }
 
 template <typename R>
-cplx factor(const GateOp<R>* o, uint32_t count, uint64_t base, uint32_t tid)
+cplx factor(const GateOp<R>* o, uint32_t count, uint64_t base, uint64_t tix, uint32_t tid, uint32_t tables)
 {
      cplx f = 1;
+     if (tables) {  // products by lane, by wave and by five bits of the tile number, in the place of records
+          const uint32_t skip = gate_table_records<R>(static_cast<int>(tables) - 1);
+          CHECK(count >= skip);
+          std::vector<double> t(2 * gate_table_entries(static_cast<int>(tables) - 1));
+          std::memcpy(t.data(), o, t.size() * sizeof(double));
+          auto at = [&](size_t i) { return cplx(t[2 * i], t[2 * i + 1]); };
+          f *= at(tid % kGateTableLanes) * at(kGateTableLanes + tid / kGateTableLanes);
+          for (uint32_t g = 1; g < tables; ++g)
+               f *= at(kGateTableLanes + kGateTableWaves + ((g - 1) << kGateTableBits) +
+                       ((tix >> ((g - 1) * kGateTableBits)) & ((1u << kGateTableBits) - 1)));
+          o += skip;
+          count -= skip;
+     }
      for (uint32_t e = 0; e < count; ++e)
           if ((base & o[e].omask) == o[e].oval && (tid & (o[e].tcond & 0xffff)) == (o[e].tcond >> 16)) {
                double u[2];
@@ -186,7 +199,7 @@ void interpret(State& psi, int n, const GatePass& P, const std::vector<GateStage
                          }
                          else if (code < kGateG2) {
                               cplx f = c0;
-                              if (code >= kGatePA) f = factor(list, count, base, t);
+                              if (code >= kGatePA) f = factor(list, count, base, tix, t, aux);
                               for (uint32_t k = 0; k < A; ++k) {
                                    bool on = true;
                                    if (code == kGatePT) on = (k & rm) == rv;
@@ -313,18 +326,37 @@ struct Maker {
 
 // permute: the last pass also takes the bits of the index to other places, if
 // it can; returns whether it did.
+// Controlled phases between all pairs of a register whose qubits come in
+// rotated order, with Hadamards: lists of many factors.
+struct Qft {
+     int n, turn;
+     std::vector<Gate> gates() const
+     {
+          std::vector<Gate> out;
+          const double r = std::sqrt(0.5);
+          for (int j = n - 1; j >= 0; --j) {
+               const int q = (j + turn) % n;
+               out.push_back({{r, r, r, -r}, {q}, {}});
+               for (int m = j - 1; m >= 0; --m)
+                    out.push_back({{1, 0, 0, std::polar(1.0, 2 * 3.14159265358979323846 / double(uint64_t(1) << (j - m + 1)))}, {q}, {(m + turn) % n}});
+          }
+          return out;
+     }
+};
+
 bool run_case(int n, int ngates, int span, int first, Prec prec, unsigned seed, size_t min_passes = 1,
-              bool permute = false)
+              bool permute = false, int qft_turn = -1)
 {
      Maker mk{std::mt19937(seed), n};
      mk.first = first;
-     std::vector<Gate> gates;
+     std::vector<Gate> gates = qft_turn >= 0 ? Qft{n, qft_turn}.gates() : std::vector<Gate>();
+     if (qft_turn >= 0) ngates = static_cast<int>(gates.size());
+     else
+          for (int i = 0; i < ngates; ++i) gates.push_back(mk.gate(span));
      std::vector<GateUnit> units;
-     for (int i = 0; i < ngates; ++i) {
-          Gate g = mk.gate(span);
+     for (const Gate& g: gates) {
           GateUnit u;
           CHECK(make_gate_unit(g.m.data(), g.t, g.c, u));
-          gates.push_back(g);
           units.push_back(u);
      }
      State psi(size_t(1) << n), ref;
@@ -401,6 +433,12 @@ int main()
           }
           run_case(18, 80, 18, 0, prec, seed++, 2);
      }
+     // long lists: tables and records
+     for (Prec prec: {Prec::C128, Prec::C64})
+          for (int n: {gate_tile_bits(prec), 16, 18})
+               for (int turn: {0, 5, n - 3}) {
+                    run_case(n, 0, n, 0, prec, seed++, 1, false, turn);
+               }
      // the last pass permutes
      seed = 1000;
      for (Prec prec: {Prec::C128, Prec::C64}) {
