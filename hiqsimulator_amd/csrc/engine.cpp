@@ -1163,7 +1163,7 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, c
           if (!make_gate_unit(items[i].m.a.data(), items[i].t, items[i].c, units[i])) return false;
      // The passes go out in groups of 1, 2, 4, ...: the first runs while the
      // others are planned and compiled.
-     GatePassPlanner planner(units, n, prec_);
+     GatePassPlanner planner(units, n, prec_, GatePassPlanner::worth_splits(n, prec_));
      GatePassPlan plan;
      for (size_t group = 1; planner.remaining().size() > keep; group *= 2) {
           std::vector<GatePass> gp;

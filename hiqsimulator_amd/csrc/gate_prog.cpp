@@ -126,8 +126,13 @@ bool make_gate_unit(const cplx* m, const std::vector<int64_t>& targets, const st
 // ---------------------------------------------------------------------------
 // Planning
 // ---------------------------------------------------------------------------
-GatePassPlanner::GatePassPlanner(const std::vector<GateUnit>& units, int n, Prec prec)
-    : units_(units), n_(n), prec_(prec)
+bool GatePassPlanner::worth_splits(int n, Prec prec)
+{
+     return std::ldexp(static_cast<double>(amp_bytes(prec)), n) >= 0x1p30;
+}
+
+GatePassPlanner::GatePassPlanner(const std::vector<GateUnit>& units, int n, Prec prec, bool splits)
+    : units_(units), n_(n), prec_(prec), splits_(splits)
 {
      if (n < gate_tile_bits(prec) || n > 62) throw std::runtime_error("gate program: the state is smaller than a tile");
      const uint64_t lim = (uint64_t(1) << n) - 1;
@@ -140,8 +145,9 @@ GatePassPlanner::GatePassPlanner(const std::vector<GateUnit>& units, int n, Prec
 // k bits of `allowed` (beside `fixed`) such that many units can be taken from
 // the front of the list: from the first unit's bits, the bit that lets the
 // most units be taken is added until k are there; then bits are exchanged
-// while that takes more.
-uint64_t GatePassPlanner::choose(const std::vector<int>& list, uint64_t fixed, uint64_t allowed, int k) const
+// while that takes more.  `start`: other bits to begin with.
+uint64_t GatePassPlanner::choose(const std::vector<int>& list, uint64_t fixed, uint64_t allowed, int k,
+                                 uint64_t start) const
 {
      constexpr int kWindow = 96;  // mixing units whose bits are candidates
      uint64_t pool = 0, H = 0;
@@ -149,7 +155,7 @@ uint64_t GatePassPlanner::choose(const std::vector<int>& list, uint64_t fixed, u
      for (int i: list) {
           const uint64_t a = units_[i].a;
           if (!a) continue;
-          if (!seen) H = a & ~fixed;
+          if (!seen) H = (start ? start : a) & ~fixed;
           pool |= a;
           if (++seen >= kWindow) break;
      }
@@ -222,6 +228,50 @@ void GatePassPlanner::take(std::vector<int>& list, uint64_t S, size_t cap, std::
      list.swap(rest);
 }
 
+// Splits a pass's units into stages, from the back of the list if `back`; with
+// `avoid` the first one found keeps off the low bits.  What does not fit stays
+// in the list.  Returns the groupings of the pass: one a stage, and one more at
+// an end whose registers hold low bits (the compiler's empty stages); 0: none.
+size_t GatePassPlanner::make_stages(std::vector<int>& list, GatePassPlan& out, bool back, bool avoid) const
+{
+     const uint64_t low = (uint64_t(1) << kGateLow) - 1;
+     out.regs.clear();
+     out.stages.clear();
+     if (back) std::reverse(list.begin(), list.end());
+     while (!list.empty() && out.stages.size() < kGateMaxStages - 2) {
+          uint64_t R;
+          if (avoid && out.stages.empty()) {
+               uint64_t ba = 0, bd = 0, start = 0;
+               for (int i: list) {
+                    const GateUnit& g = units_[i];
+                    if (g.a && !(g.a & (low | ba | bd)) && !(g.d & ba)) {
+                         start = g.a;
+                         break;
+                    }
+                    ba |= g.a;
+                    bd |= g.d;
+               }
+               if (!start) return 0;
+               R = choose(list, 0, out.bits & ~low, gate_reg(prec_), start);
+          }
+          else {
+               R = choose(list, 0, out.bits, gate_reg(prec_));
+          }
+          std::vector<int> stage;
+          take(list, R, kGateMaxStageUnits, stage);
+          if (stage.empty()) throw std::runtime_error("gate program: no gate could be staged");
+          if (back) std::reverse(stage.begin(), stage.end());
+          out.regs.push_back(R);
+          out.stages.push_back(std::move(stage));
+     }
+     if (back) {
+          std::reverse(list.begin(), list.end());
+          std::reverse(out.regs.begin(), out.regs.end());
+          std::reverse(out.stages.begin(), out.stages.end());
+     }
+     return out.stages.size() + ((out.regs.front() & low) != 0) + ((out.regs.back() & low) != 0);
+}
+
 bool GatePassPlanner::next(GatePassPlan& out)
 {
      if (rem_.empty()) return false;
@@ -233,14 +283,19 @@ bool GatePassPlanner::next(GatePassPlan& out)
      std::vector<int> taken;
      take(rem_, out.bits, rem_.size(), taken);
      if (taken.empty()) throw std::runtime_error("gate program: no gate could be planned");
-     while (!taken.empty() && out.stages.size() < kGateMaxStages - 2) {
-          const uint64_t R = choose(taken, 0, out.bits, gate_reg(prec_));
-          std::vector<int> stage;
-          take(taken, R, kGateMaxStageUnits, stage);
-          if (stage.empty()) throw std::runtime_error("gate program: no gate could be staged");
-          out.regs.push_back(R);
-          out.stages.push_back(std::move(stage));
-     }
+     const std::vector<int> whole = splits_ ? taken : std::vector<int>();
+     size_t groupings = make_stages(taken, out, false, false);
+     if (splits_ && taken.empty())
+          for (int way = 1; way < 4; ++way) {
+               GatePassPlan other;
+               other.bits = out.bits;
+               std::vector<int> list = whole;
+               const size_t g = make_stages(list, other, way & 2, way & 1);
+               if (g && list.empty() && g < groupings) {
+                    groupings = g;
+                    out = std::move(other);
+               }
+          }
      if (!taken.empty()) {  // more stages than a pass holds: the rest stays
           std::vector<int> all_rest(taken.size() + rem_.size());
           std::merge(taken.begin(), taken.end(), rem_.begin(), rem_.end(), all_rest.begin());

@@ -202,17 +202,25 @@ struct GatePassPlan {
 // neither mixes a bit that the other touches.
 class GatePassPlanner {
 public:
-     GatePassPlanner(const std::vector<GateUnit>& units, int n, Prec prec);
+     // splits: every pass is split into stages in four ways, and the one with the
+     // fewest groupings kept (worth_splits).
+     GatePassPlanner(const std::vector<GateUnit>& units, int n, Prec prec, bool splits = false);
+     // Where a pass takes longer than its planning: a grouping less saves 0.4 to
+     // 0.9 ms of a pass on 30 qubits in complex128, and 0.04 ms of planning find
+     // 0.4 of one on average (of 4.1; complex64, 23 qubits: 0.6 of 5.6).
+     static bool worth_splits(int n, Prec prec);
      bool next(GatePassPlan& out);
      // Indices of the units not planned yet, in program order.
      const std::vector<int>& remaining() const { return rem_; }
 
 private:
-     uint64_t choose(const std::vector<int>& list, uint64_t fixed, uint64_t allowed, int k) const;
+     uint64_t choose(const std::vector<int>& list, uint64_t fixed, uint64_t allowed, int k, uint64_t start = 0) const;
+     size_t make_stages(std::vector<int>& list, GatePassPlan& out, bool back, bool avoid) const;
      void take(std::vector<int>& list, uint64_t S, size_t cap, std::vector<int>& out) const;
      const std::vector<GateUnit>& units_;
      int n_;
      Prec prec_;
+     bool splits_;
      std::vector<int> rem_;
 };
 

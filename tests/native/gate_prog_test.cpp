@@ -345,7 +345,7 @@ struct Qft {
 };
 
 bool run_case(int n, int ngates, int span, int first, Prec prec, unsigned seed, size_t min_passes = 1,
-              bool permute = false, int qft_turn = -1)
+              bool permute = false, int qft_turn = -1, bool splits = false)
 {
      Maker mk{std::mt19937(seed), n};
      mk.first = first;
@@ -363,7 +363,7 @@ bool run_case(int n, int ngates, int span, int first, Prec prec, unsigned seed, 
      for (auto& z: psi) z = cplx(mk.u(-1, 1), mk.u(-1, 1));
      ref = psi;
      for (const auto& g: gates) apply(ref, g);
-     GatePassPlanner planner(units, n, prec);
+     GatePassPlanner planner(units, n, prec, splits);
      GatePassPlan plan;
      std::vector<GateStage> stages;
      std::vector<char> ops;
@@ -439,6 +439,13 @@ int main()
                for (int turn: {0, 5, n - 3}) {
                     run_case(n, 0, n, 0, prec, seed++, 1, false, turn);
                }
+     // the best of four ways to split a pass into stages
+     for (Prec prec: {Prec::C128, Prec::C64})
+          for (int n: {gate_tile_bits(prec), 16}) {
+               for (int r = 0; r < 4; ++r) run_case(n, 1 + 24 * r, n, 0, prec, seed++, 1, r == 2, -1, true);
+               run_case(n, 60, 5, 0, prec, seed++, 1, false, -1, true);
+               run_case(n, 0, n, 0, prec, seed++, 1, false, 3, true);
+          }
      // the last pass permutes
      seed = 1000;
      for (Prec prec: {Prec::C128, Prec::C64}) {
