@@ -1453,18 +1453,19 @@ hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, in
                          double* sums, uint64_t* out, hipStream_t s)
 {
      if (njobs <= 0 || max_shots == 0) return hipSuccess;
-     if (njobs > 65535) return hipErrorInvalidValue;
      hipLaunchKernelGGL(k_sample_cdf, dim3(njobs), dim3(kSampleThreads), 0, s, jobs, sums);
-     const hipError_t e = hipGetLastError();
-     if (e != hipSuccess) return e;
-     const dim3 grid((max_shots + 3) / 4, static_cast<unsigned>(njobs));
-     if (prec == Prec::C128)
-          hipLaunchKernelGGL((k_sample_shots<double>), grid, dim3(256), 0, s, static_cast<const double2*>(arena), jobs,
-                             sums, out);
-     else
-          hipLaunchKernelGGL((k_sample_shots<float>), grid, dim3(256), 0, s, static_cast<const float2*>(arena), jobs,
-                             sums, out);
-     return hipGetLastError();
+     hipError_t e = hipGetLastError();
+     for (int j = 0; e == hipSuccess && j < njobs; j += 65535) {  // the limit of a grid's y
+          const dim3 grid((max_shots + 3) / 4, static_cast<unsigned>(njobs - j < 65535 ? njobs - j : 65535));
+          if (prec == Prec::C128)
+               hipLaunchKernelGGL((k_sample_shots<double>), grid, dim3(256), 0, s, static_cast<const double2*>(arena),
+                                  jobs + j, sums, out);
+          else
+               hipLaunchKernelGGL((k_sample_shots<float>), grid, dim3(256), 0, s, static_cast<const float2*>(arena),
+                                  jobs + j, sums, out);
+          e = hipGetLastError();
+     }
+     return e;
 }
 
 hipError_t launch_measure(const void* psi, Prec prec, double* sums, int log_blocks, int log_block_amps, double u,
