@@ -1,10 +1,10 @@
 // gfx950 kernels of the gate programs (gate_prog.hpp).
 //
 // Bound: HBM (one read and one write of the state a pass) up to about forty
-// gates a pass: 30 random qubits in complex128 take 7.9 ms a pass then, of
+// gates a pass: 30 random qubits in complex128 take 7.8 ms a pass then, of
 // which a bare copy in this shape takes 6.8 ms.  Vector issue (the gates and the
-// regrouping between stages) comes on top with more, 11.5 ms for 75 gates.
-// The 1780 gates of a 30-qubit circuit take 24 passes and 277 ms; as fused
+// regrouping between stages) comes on top with more, 11.2 ms for 74 gates.
+// The 1780 gates of a 30-qubit circuit take 24 passes and 269 ms; as fused
 // dense ops on LDS tiles they took 50 passes and 426 ms.
 #include <hip/hip_runtime.h>
 
