@@ -149,7 +149,8 @@ public:
      // this for ProjectQ's TimeEvolution gate (_simulator_mpi.py:469-475)
      // but its C++ never defines it.  Identity terms become a phase; the
      // rest is a Chebyshev series for real coefficients and planned sums
-     // (pauli_prog.hpp), else a Taylor series in s = ceil(|t| sum|c|) steps,
+     // (pauli_prog.hpp; in segments of |t| sum|c| <= 256), else a Taylor
+     // series in s = ceil(|t| sum|c|) steps,
      // each summed until a term's norm drops below 1e-12 (at most 64 terms).
      void time_evolution(const std::vector<uint64_t>& xm, const std::vector<uint64_t>& zm,
                          const std::vector<cplx>& coeff, double t, const std::vector<int64_t>& ids,

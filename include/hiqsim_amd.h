@@ -204,8 +204,9 @@ int hiqsim_apply_pauli_sum(hiqsim_t* h, const uint64_t* xmask, const uint64_t* z
  * as above (Hermitian for a unitary result).  Identity terms become a phase;
  * the rest is a Chebyshev series in H / sum|coeff| to 1e-17 for real
  * coefficients (on 9 or more qubits, X parts within 12 index bits, |time|
- * sum|coeff| up to 1e6), otherwise a Taylor series in ceil(|time| sum|coeff|)
- * steps, each summed until a term's norm is below 1e-12. */
+ * sum|coeff| up to 1e6; in segments of at most 256 of it), otherwise a Taylor
+ * series in ceil(|time| sum|coeff|) steps, each summed until a term's norm is
+ * below 1e-12. */
 int hiqsim_emulate_time_evolution(hiqsim_t* h, const uint64_t* xmask, const uint64_t* zmask,
                                   const double* coeff, size_t nterms, double time, const int64_t* ids,
                                   size_t nids, const int64_t* ctrls, size_t nctrls);
