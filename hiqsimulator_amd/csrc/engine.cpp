@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <deque>
 #include <numeric>
 #include <sstream>
 #include <stdexcept>
@@ -113,9 +114,10 @@ Engine::~Engine()
      if (d_samples_) (void)hipFree(d_samples_);
      for (auto& ps: prog_) {
           if (ps.ev) (void)hipEventDestroy(ps.ev);
-          if (ps.h) (void)hipHostFree(ps.h);
-          if (ps.d) (void)hipFree(ps.d);
+          free_slot(ps);
      }
+     if (h_prog_) (void)hipHostFree(h_prog_);
+     if (d_prog_) (void)hipFree(d_prog_);
      if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -1129,22 +1131,51 @@ int Engine::apply_tiled(const std::vector<Gate>& gates, int op_width)
 
 Engine::ProgSlot& Engine::program_slot(size_t need)
 {
+     if (!h_prog_) {
+          char *h = nullptr, *d = nullptr;
+          check(hipHostMalloc(reinterpret_cast<void**>(&h), kProgSlots * kProgBytes, hipHostMallocDefault),
+                "hipHostMalloc(program)");
+          hipError_t e = hipMalloc(reinterpret_cast<void**>(&d), kProgSlots * kProgBytes);
+          for (int i = 0; e == hipSuccess && i < kProgSlots; ++i)
+               if (!prog_[i].ev) e = hipEventCreateWithFlags(&prog_[i].ev, hipEventDisableTiming);
+          if (e != hipSuccess) {
+               (void)hipHostFree(h);
+               if (d) (void)hipFree(d);
+               check(e, "hipMalloc(program)");
+          }
+          h_prog_ = h;
+          d_prog_ = d;
+          for (int i = 0; i < kProgSlots; ++i) {
+               prog_[i].h = h + i * kProgBytes;
+               prog_[i].d = d + i * kProgBytes;
+               prog_[i].cap = kProgBytes;
+          }
+     }
      ProgSlot& ps = prog_[prog_next_];
      prog_next_ = (prog_next_ + 1) % kProgSlots;
      if (ps.busy) check(hipEventSynchronize(ps.ev), "hipEventSynchronize");
      ps.busy = false;
      if (need > ps.cap) {
-          if (ps.h) check(hipHostFree(ps.h), "hipHostFree");
-          if (ps.d) check(hipFree(ps.d), "hipFree");
-          ps.h = ps.d = nullptr;
-          ps.cap = 0;
+          // (the old memory stays until the new is there)
           const size_t cap = std::max(need, size_t(1) << 20);
-          check(hipHostMalloc(reinterpret_cast<void**>(&ps.h), cap, hipHostMallocDefault), "hipHostMalloc(program)");
-          check(hipMalloc(reinterpret_cast<void**>(&ps.d), cap), "hipMalloc(program)");
+          char *h = nullptr, *d = nullptr;
+          check(hipHostMalloc(reinterpret_cast<void**>(&h), cap, hipHostMallocDefault), "hipHostMalloc(program)");
+          const hipError_t e = hipMalloc(reinterpret_cast<void**>(&d), cap);
+          if (e != hipSuccess) (void)hipHostFree(h);
+          check(e, "hipMalloc(program)");
+          free_slot(ps);
+          ps.h = h;
+          ps.d = d;
           ps.cap = cap;
      }
-     if (!ps.ev) check(hipEventCreateWithFlags(&ps.ev, hipEventDisableTiming), "hipEventCreate");
      return ps;
+}
+
+void Engine::free_slot(ProgSlot& ps)
+{
+     if (ps.cap <= kProgBytes) return;  // part of the block
+     (void)hipHostFree(ps.h);
+     (void)hipFree(ps.d);
 }
 
 void Engine::program_done(ProgSlot& ps)
@@ -1161,42 +1192,88 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, c
      std::vector<GateUnit> units(items.size());
      for (size_t i = 0; i < items.size(); ++i)
           if (!make_gate_unit(items[i].m.a.data(), items[i].t, items[i].c, units[i])) return false;
+     // What is on the stream leaves the list, also when something fails on the way.
+     struct Rest {
+          std::vector<PosGate>& items;
+          std::vector<char> done;
+          void mark(const GatePassPlan& p)
+          {
+               for (const auto& st: p.stages)
+                    for (int i: st) done[i] = 1;
+          }
+          ~Rest()
+          {
+               size_t j = 0;
+               for (size_t i = 0; i < items.size(); ++i) {
+                    if (done[i]) continue;
+                    if (j != i) items[j] = std::move(items[i]);
+                    ++j;
+               }
+               items.resize(j);
+          }
+     } rest{items, std::vector<char>(items.size(), 0)};
      // The passes go out in groups of 1, 2, 4, ...: the first runs while the
-     // others are planned and compiled.
+     // others are planned and compiled.  A group fits a staging slot as it is,
+     // so that no allocation comes between them.
      GatePassPlanner planner(units, n, prec_, GatePassPlanner::worth_splits(n, prec_));
-     GatePassPlan plan;
-     for (size_t group = 1; planner.remaining().size() > keep; group *= 2) {
+     std::deque<GatePassPlan> ahead;  // planned, not compiled
+     GatePassPlan last;               // the one that permutes
+     auto more = [&] { return !ahead.empty() || planner.remaining().size() > keep; };
+     for (size_t group = 1; more(); group *= 2) {
           std::vector<GatePass> gp;
+          std::vector<GatePassPlan> plans;
           std::vector<GateStage> stages;
           std::vector<char> ops;
-          while (gp.size() < group && planner.remaining().size() > keep && planner.next(plan)) {
-               gp.emplace_back();
+          auto stage_bytes = [&] { return (stages.size() * sizeof(GateStage) + 255) / 256 * 256; };
+          while (gp.size() < group && more()) {
+               if (ahead.empty()) {
+                    GatePassPlan next;
+                    planner.next(next);
+                    ahead.push_back(std::move(next));
+               }
+               GatePassPlan& plan = ahead.front();
                // the last pass may store the state permuted
-               const bool perm = src_pos && planner.remaining().empty() && widen_for_permutation(units, plan, n, prec_, src_pos);
+               const bool perm = src_pos && ahead.size() == 1 && planner.remaining().empty() &&
+                                 widen_for_permutation(units, plan, n, prec_, src_pos);
+               const size_t s0 = stages.size(), o0 = ops.size();
+               gp.emplace_back();
                compile_gate_pass(units, plan, n, prec_, gp.back(), stages, ops, perm ? src_pos : nullptr);
+               if (stage_bytes() + ops.size() > kProgBytes) {
+                    gp.pop_back();
+                    stages.resize(s0);
+                    ops.resize(o0);
+                    if (!gp.empty()) break;  // the next group begins with it
+                    GatePassPlan second;
+                    if (!split_gate_pass(plan, second)) throw std::runtime_error("gate program: a gate exceeds its staging slot");
+                    ahead.insert(ahead.begin() + 1, std::move(second));
+                    continue;
+               }
+               plans.push_back(std::move(plan));
+               ahead.pop_front();
           }
           for (const auto& p: gp) check_gate_pass(p, stages, ops, prec_, n);
-          const size_t stage_bytes = (stages.size() * sizeof(GateStage) + 255) / 256 * 256;
-          const size_t need = stage_bytes + ops.size();
+          const size_t sb = stage_bytes(), need = sb + ops.size();
           ProgSlot& ps = program_slot(need);
           std::memcpy(ps.h, stages.data(), stages.size() * sizeof(GateStage));
-          std::memcpy(ps.h + stage_bytes, ops.data(), ops.size());
+          std::memcpy(ps.h + sb, ops.data(), ops.size());
           check(hipMemcpyAsync(ps.d, ps.h, need, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync(program)");
-          for (const auto& p: gp) {
+          for (size_t i = 0; i < gp.size(); ++i) {
+               const GatePass& p = gp[i];
                begin_timed(kTile);
-               check(launch_gate_pass(d_state_, prec_, n, p, reinterpret_cast<const GateStage*>(ps.d), ps.d + stage_bytes,
+               check(launch_gate_pass(d_state_, prec_, n, p, reinterpret_cast<const GateStage*>(ps.d), ps.d + sb,
                                       stream_, p.permuted ? d_tmp_ : d_state_),
                      "gate pass");
+               if (p.permuted) last = std::move(plans[i]);  // (the state has not changed yet)
+               else rest.mark(plans[i]);
                end_timed();
-               if (p.permuted) *permuted = true;
                ++passes;
           }
           program_done(ps);
      }
-     std::vector<PosGate> rest;
-     rest.reserve(planner.remaining().size());
-     for (int i: planner.remaining()) rest.push_back(std::move(items[i]));
-     items.swap(rest);
+     if (!last.stages.empty()) {
+          rest.mark(last);
+          *permuted = true;
+     }
      return true;
 }
 

@@ -203,7 +203,8 @@ private:
      int tile_items(std::vector<PosGate>& items, int op_width, size_t keep);
      // The same by gate programs (gate_prog.hpp), for states of at least
      // gate_min_qubits and lists whose gates mix at most two qubits each;
-     // false (and nothing done) for others.
+     // false (and nothing done) for others.  When it throws, `items` holds what
+     // has not been applied.
      // src_pos: the last pass also permutes the index bits (launch_permute) into
      // d_tmp_ if it can; *permuted tells.
      bool gate_items(std::vector<PosGate>& items, size_t keep, int& passes, const uint8_t* src_pos = nullptr,
@@ -216,6 +217,7 @@ private:
      // after the launches that use it.
      ProgSlot& upload_pauli(const PauliPlan& plan, const PauliTerm*& terms);
      void program_done(ProgSlot& ps);
+     void free_slot(ProgSlot& ps);
      void release_buffer(void*& p);
      void collect_retired();
      // A same-size out-of-place result in d_tmp_ becomes the state: the
@@ -292,6 +294,11 @@ private:
           bool busy = false;
      };
      static constexpr int kProgSlots = 3;
+     // One block holds all slots: a first program allocates once, before any of
+     // its passes runs.  Plans beyond a slot's share (tile programs, Pauli sums
+     // of ten thousand terms) give it memory of its own.
+     static constexpr size_t kProgBytes = size_t(320) << 10;
+     char *h_prog_ = nullptr, *d_prog_ = nullptr;
      ProgSlot prog_[kProgSlots];
      int prog_next_ = 0;
 

@@ -930,6 +930,27 @@ void compile_gate_pass(const std::vector<GateUnit>& units, const GatePassPlan& p
      Compiler(units, plan, n, prec, pass, stages, ops, src_pos).run();
 }
 
+bool split_gate_pass(GatePassPlan& plan, GatePassPlan& second)
+{
+     second = GatePassPlan();
+     second.bits = plan.bits;
+     if (plan.stages.size() > 1) {
+          const size_t half = plan.stages.size() / 2;
+          second.regs.assign(plan.regs.begin() + static_cast<long>(half), plan.regs.end());
+          second.stages.assign(plan.stages.begin() + static_cast<long>(half), plan.stages.end());
+          plan.regs.resize(half);
+          plan.stages.resize(half);
+          return true;
+     }
+     std::vector<int>& only = plan.stages.at(0);
+     if (only.size() < 2) return false;
+     const auto half = only.begin() + static_cast<long>(only.size() / 2);
+     second.regs = plan.regs;
+     second.stages.emplace_back(half, only.end());
+     only.erase(half, only.end());
+     return true;
+}
+
 bool widen_for_permutation(const std::vector<GateUnit>& units, GatePassPlan& plan, int n, Prec prec,
                            const uint8_t* src_pos)
 {

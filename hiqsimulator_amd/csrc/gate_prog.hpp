@@ -235,6 +235,10 @@ private:
 void compile_gate_pass(const std::vector<GateUnit>& units, const GatePassPlan& plan, int n, Prec prec,
                        GatePass& pass, std::vector<GateStage>& stages, std::vector<char>& ops,
                        const uint8_t* src_pos = nullptr);
+// Leaves the plan the first half of its stages (or of the units of its only
+// one) and puts the other half into `second`, to run right behind it; false for
+// a single unit.
+bool split_gate_pass(GatePassPlan& plan, GatePassPlan& second);
 // Puts bits src_pos[0..kGateLow) into the plan's tile, in the place of bits that
 // its units do not mix, so that the permuted state is stored in runs of 2^kGateLow
 // amplitudes; false, and nothing changed, when they do not fit.  At 30 qubits
