@@ -1192,6 +1192,8 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, c
      std::vector<GateUnit> units(items.size());
      for (size_t i = 0; i < items.size(); ++i)
           if (!make_gate_unit(items[i].m.a.data(), items[i].t, items[i].c, units[i])) return false;
+     Prec held;
+     if (!gate_route(gate_list_cost(units), n, prec_, held)) return false;
      // What is on the stream leaves the list, also when something fails on the way.
      struct Rest {
           std::vector<PosGate>& items;
@@ -1215,7 +1217,7 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, c
      // The passes go out in groups of 1, 2, 4, ...: the first runs while the
      // others are planned and compiled.  A group fits a staging slot as it is,
      // so that no allocation comes between them.
-     GatePassPlanner planner(units, n, prec_, GatePassPlanner::worth_splits(n, prec_));
+     GatePassPlanner planner(units, n, held, GatePassPlanner::worth_splits(n, prec_));
      std::deque<GatePassPlan> ahead;  // planned, not compiled
      GatePassPlan last;               // the one that permutes
      auto more = [&] { return !ahead.empty() || planner.remaining().size() > keep; };
@@ -1234,10 +1236,10 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, c
                GatePassPlan& plan = ahead.front();
                // the last pass may store the state permuted
                const bool perm = src_pos && ahead.size() == 1 && planner.remaining().empty() &&
-                                 widen_for_permutation(units, plan, n, prec_, src_pos);
+                                 widen_for_permutation(units, plan, n, held, src_pos);
                const size_t s0 = stages.size(), o0 = ops.size();
                gp.emplace_back();
-               compile_gate_pass(units, plan, n, prec_, gp.back(), stages, ops, perm ? src_pos : nullptr);
+               compile_gate_pass(units, plan, n, held, gp.back(), stages, ops, perm ? src_pos : nullptr);
                if (stage_bytes() + ops.size() > kProgBytes) {
                     gp.pop_back();
                     stages.resize(s0);
@@ -1251,7 +1253,7 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, c
                plans.push_back(std::move(plan));
                ahead.pop_front();
           }
-          for (const auto& p: gp) check_gate_pass(p, stages, ops, prec_, n);
+          for (const auto& p: gp) check_gate_pass(p, stages, ops, held, n);
           const size_t sb = stage_bytes(), need = sb + ops.size();
           ProgSlot& ps = program_slot(need);
           std::memcpy(ps.h, stages.data(), stages.size() * sizeof(GateStage));
@@ -1260,7 +1262,7 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, c
           for (size_t i = 0; i < gp.size(); ++i) {
                const GatePass& p = gp[i];
                begin_timed(kTile);
-               check(launch_gate_pass(d_state_, prec_, n, p, reinterpret_cast<const GateStage*>(ps.d), ps.d + sb,
+               check(launch_gate_pass(d_state_, prec_, held, n, p, reinterpret_cast<const GateStage*>(ps.d), ps.d + sb,
                                       stream_, p.permuted ? d_tmp_ : d_state_),
                      "gate pass");
                if (p.permuted) last = std::move(plans[i]);  // (the state has not changed yet)

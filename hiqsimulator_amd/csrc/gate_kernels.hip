@@ -569,15 +569,26 @@ __device__ __forceinline__ uint64_t reg_index(int k, const uint8_t (&pos)[kGateM
      return i;
 }
 
+template <typename R, typename V>
+__device__ __forceinline__ VT<R> converted(const V& a)
+{
+     VT<R> r;
+     r.x = static_cast<R>(a.x);
+     r.y = static_cast<R>(a.y);
+     return r;
+}
+
+// S: the state's type; R: the type that the amplitudes have while the pass
+// holds them.
 // Copies that the register allocator cannot merge away.  The loads and stores
 // work on whole amplitudes in consecutive registers while the regrouping
 // moves real and imaginary parts separately; tied to the loads' registers the
 // whole array ends up twice in the register file, and spills.
-template <typename R>
-__device__ __forceinline__ void gate_program(VT<R>* psi, const GatePass& P,
+template <typename S, typename R>
+__device__ __forceinline__ void gate_program(VT<S>* psi, const GatePass& P,
                                              const GateStage* __restrict__ stages,
                                              const GateOp<R>* __restrict__ ops, const uint64_t tix, char* lds,
-                                             VT<R>* dst)
+                                             VT<S>* dst)
 {
      using V = VT<R>;
      constexpr int E = Shape<R>::E, A = 1 << E, H = Shape<R>::T - kGateLow;
@@ -590,14 +601,15 @@ __device__ __forceinline__ void gate_program(VT<R>* psi, const GatePass& P,
      }
      V x[A];
      {
-          const V* const p = psi + base + thread_index(tid, P.in_thr);
+          const VT<S>* const p = psi + base + thread_index(tid, P.in_thr);
+          VT<S> in[A];
 #pragma unroll
           for (int k = 0; k < A; ++k) {
-               x[k] = ld_nt(p + reg_index(k, P.in_reg));
+               in[k] = ld_nt(p + reg_index(k, P.in_reg));
                if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
           }
 #pragma unroll
-          for (int k = 0; k < A; ++k) x[k] = copy_amp(x[k]);
+          for (int k = 0; k < A; ++k) x[k] = copy_amp(converted<R>(in[k]));
      }
      uint32_t s = 0, slot = 0;
      do {
@@ -613,33 +625,33 @@ __device__ __forceinline__ void gate_program(VT<R>* psi, const GatePass& P,
 #pragma unroll
           for (int j = 0; j < kGateMaxBase; ++j) to |= ((tix >> j) & 1) << P.base_out[j];
      }
-     V* const p = dst + to + thread_index(fresh(tid), P.out_thr);
+     VT<S>* const p = dst + to + thread_index(fresh(tid), P.out_thr);
 #pragma unroll
      for (int k = 0; k < A; ++k) {
-          st_nt(p + reg_index(k, P.out_reg), copy_amp(x[k]));
+          st_nt(p + reg_index(k, P.out_reg), converted<S>(copy_amp(x[k])));
           if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
      }
 }
 
-template <typename R>
+template <typename S, typename R>
 __global__ void __launch_bounds__(kGateThreads) __attribute__((amdgpu_waves_per_eu(4)))
-    k_gate_pass(VT<R>* psi, const GatePass P, const GateStage* __restrict__ stages,
-                const GateOp<R>* __restrict__ ops, const int swz, const uint64_t nblocks, VT<R>* dst)
+    k_gate_pass(VT<S>* psi, const GatePass P, const GateStage* __restrict__ stages,
+                const GateOp<R>* __restrict__ ops, const int swz, const uint64_t nblocks, VT<S>* dst)
 {
      __shared__ __align__(16) char lds[sizeof(R) << Shape<R>::T];
      const uint64_t b = block_linear();
      if (b >= nblocks) return;  // padding of the 2-D grid (whole block)
-     gate_program<R>(psi, P, stages + P.stage_first, ops, swizzle_block(b, swz), lds, dst);
+     gate_program<S, R>(psi, P, stages + P.stage_first, ops, swizzle_block(b, swz), lds, dst);
 }
 
 }  // namespace
 
-hipError_t launch_gate_pass(void* psi, Prec prec, int n_qubits, const GatePass& pass, const GateStage* stages,
+hipError_t launch_gate_pass(void* psi, Prec prec, Prec held, int n_qubits, const GatePass& pass, const GateStage* stages,
                             const void* ops, hipStream_t s, void* dst)
 {
      if (pass.permuted ? (!dst || dst == psi) : (dst && dst != psi)) return hipErrorInvalidValue;
      if (!dst) dst = psi;
-     const int T = gate_tile_bits(prec);
+     const int T = gate_tile_bits(held);
      if (n_qubits < T || n_qubits > 40 || pass.nstages < 1) return hipErrorInvalidValue;
      for (int j = 0; j < T - kGateLow; ++j)
           if (pass.hpos[j] < kGateLow || pass.hpos[j] >= n_qubits || (j && pass.hpos[j] <= pass.hpos[j - 1]))
@@ -647,14 +659,19 @@ hipError_t launch_gate_pass(void* psi, Prec prec, int n_qubits, const GatePass& 
      const uint64_t blocks = 1ull << (n_qubits - T);
      const int bits = get_block_swizzle();
      const int swz = (bits > 0 && bits <= 16 && blocks % (1ull << bits) == 0) ? bits : 0;
-     if (prec == Prec::C128)
-          hipLaunchKernelGGL((k_gate_pass<double>), grid_2d(blocks), dim3(kGateThreads), 0, s,
+     if (prec == Prec::C128 && held == Prec::C128)
+          hipLaunchKernelGGL((k_gate_pass<double, double>), grid_2d(blocks), dim3(kGateThreads), 0, s,
                              static_cast<double2*>(psi), pass, stages, static_cast<const GateOp<double>*>(ops), swz,
                              blocks, static_cast<double2*>(dst));
-     else
-          hipLaunchKernelGGL((k_gate_pass<float>), grid_2d(blocks), dim3(kGateThreads), 0, s,
+     else if (prec == Prec::C64 && held == Prec::C128)
+          hipLaunchKernelGGL((k_gate_pass<float, double>), grid_2d(blocks), dim3(kGateThreads), 0, s,
+                             static_cast<float2*>(psi), pass, stages, static_cast<const GateOp<double>*>(ops), swz,
+                             blocks, static_cast<float2*>(dst));
+     else if (prec == Prec::C64)
+          hipLaunchKernelGGL((k_gate_pass<float, float>), grid_2d(blocks), dim3(kGateThreads), 0, s,
                              static_cast<float2*>(psi), pass, stages, static_cast<const GateOp<float>*>(ops), swz,
                              blocks, static_cast<float2*>(dst));
+     else return hipErrorInvalidValue;
      return hipGetLastError();
 }
 

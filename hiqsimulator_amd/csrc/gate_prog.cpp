@@ -124,6 +124,106 @@ bool make_gate_unit(const cplx* m, const std::vector<int64_t>& targets, const st
 }
 
 // ---------------------------------------------------------------------------
+// Which way
+// ---------------------------------------------------------------------------
+namespace {
+
+bool is_flip(const GateBranch& b) { return b.u[0] == 0.0 && b.u[3] == 0.0 && is_one(b.u[1]) && is_one(b.u[2]); }
+
+// What an unconditional gate on one qubit is merged with (put_one, layer_phase).
+enum Run : uint8_t { kRunNone, kRunPhase, kRunReal, kRunCross, kRunGeneral };
+
+Run run_of(const GateUnit& g)
+{
+     const auto& u = g.br[0].u;
+     if (g.na == 0) return kRunPhase;
+     if (u[0].imag() == 0.0 && u[3].imag() == 0.0) {
+          if (u[1].imag() == 0.0 && u[2].imag() == 0.0) return kRunReal;
+          if (u[1].real() == 0.0 && u[2].real() == 0.0) return kRunCross;
+     }
+     return kRunGeneral;
+}
+
+}  // namespace
+
+GateListCost gate_list_cost(const std::vector<GateUnit>& units)
+{
+     constexpr int kWidth = 4;
+     GateListCost c;
+     Run run[64] = {};  // of each qubit's last gate, while it can still take another
+     auto end_run = [&](uint64_t bits) {
+          for (; bits; bits &= bits - 1) {
+               Run& r = run[__builtin_ctzll(bits)];
+               if (r == kRunGeneral) c.rounds += 2;
+               else if (r != kRunNone) c.rounds += 1;
+               r = kRunNone;
+          }
+     };
+     std::vector<uint64_t> groups;  // qubits of the fused products
+     int last[64];                  // a qubit's last one
+     std::fill_n(last, 64, -1);
+     auto open = [&](int i) {
+          for (uint64_t m = groups[i]; m; m &= m - 1)
+               if (last[__builtin_ctzll(m)] != i) return false;
+          return true;
+     };
+     double slots = 0;
+     for (const GateUnit& g: units) {
+          const uint64_t bits = g.a | g.d;
+          if (g.br.empty() || !bits) continue;  // (a factor of all amplitudes costs nothing)
+          const bool single = popc(bits) == 1 && (g.na == 0 || (g.br.size() == 1 && !g.br[0].cmask));
+          if (single) {
+               Run& r = run[__builtin_ctzll(bits)];
+               const Run now = run_of(g);
+               if (r != kRunNone && r != now) {
+                    if (r != kRunPhase && now != kRunPhase && (r == kRunGeneral || now == kRunGeneral)) r = kRunGeneral;
+                    else end_run(bits);
+               }
+               if (r == kRunNone) r = now;
+          }
+          else {
+               end_run(g.na ? bits : 0);
+               for (const auto& b: g.br) {
+                    if (g.na == 0) c.rounds += 0.25;
+                    else if (g.na == 2) c.rounds += 4;
+                    else if (!is_flip(b)) c.rounds += 2;
+               }
+          }
+          // the fused product that it would go into
+          const int first = last[__builtin_ctzll(bits)];
+          bool inside = first >= 0;
+          for (uint64_t m = bits; m; m &= m - 1) inside = inside && last[__builtin_ctzll(m)] == first;
+          if (inside) continue;
+          uint64_t u = bits;
+          for (uint64_t m = bits; m; m &= m - 1) {
+               const int i = last[__builtin_ctzll(m)];
+               if (i < 0 || !(groups[i] & ~u) || !open(i) || popc(u | groups[i]) > kWidth) continue;
+               u |= groups[i];
+          }
+          for (uint64_t m = u; m; m &= m - 1) {
+               const int i = last[__builtin_ctzll(m)];
+               if (i < 0 || (groups[i] & ~u) || !open(i)) continue;
+               slots -= popc(groups[i]);  // grows into the new one
+               groups[i] = 0;
+          }
+          slots += popc(u);
+          for (uint64_t m = u; m; m &= m - 1) last[__builtin_ctzll(m)] = static_cast<int>(groups.size());
+          groups.push_back(u);
+     }
+     c.products = slots / 4;
+     end_run(~uint64_t(0));
+     return c;
+}
+
+bool gate_route(const GateListCost& cost, int n, Prec prec, Prec& held)
+{
+     held = Prec::C128;
+     if (n < gate_min_qubits(prec) || n > 40) return false;
+     if (prec == Prec::C64 && cost.rounds <= 1.5 * cost.products) held = Prec::C64;
+     return true;
+}
+
+// ---------------------------------------------------------------------------
 // Planning
 // ---------------------------------------------------------------------------
 bool GatePassPlanner::worth_splits(int n, Prec prec)

@@ -11,6 +11,10 @@
 // and diagonal qubits are conditions on the index, which a tile can evaluate
 // wherever they are, so a pass takes gates that a dense plan cannot.
 //
+// Below, a precision is the one that the amplitudes have in a pass.  A
+// complex64 state is held in complex128 for most lists (gate_route): in FP32,
+// gate after gate, its roundings are more than those of the fused products.
+//
 // A pass covers tiles of 2^13 amplitudes in complex128 and 2^14 in complex64:
 // index bits 0..3 (runs of 16 amplitudes: 256 and 128 bytes) and nine or ten
 // chosen bits.  A workgroup of 512 threads holds its tile in registers, 16 or
@@ -190,6 +194,28 @@ struct GateUnit {
 bool make_gate_unit(const std::complex<double>* m, const std::vector<int64_t>& targets,
                     const std::vector<int64_t>& ctrls, GateUnit& out);
 
+// ---- host: which way a list goes --------------------------------------------
+// What a list takes either way, counted in one sweep over its units.
+//   products  fused products on four qubits that a tile program needs about:
+//             a quarter of the qubits of greedily grown groups of up to four.
+//   rounds    roundings of an amplitude that a gate program makes in the
+//             precision it is held in.
+struct GateListCost {
+     double products = 0, rounds = 0;
+};
+GateListCost gate_list_cost(const std::vector<GateUnit>& units);
+// The precision that a gate program of the list would hold the amplitudes of
+// an n-qubit state in; false: the list runs as tile programs.
+//
+// Roundings.  Error of gate programs held in FP32 over that of tile programs (l2,
+// complex64, 25 qubits): QFT 0.54, layers with random angles 0.75, three
+// rotations 1.1, 40 Trotter steps of an Ising chain 2.9 (a coefficient's rounding
+// comes back in every step), 200 layers on 4 qubits 6.4.  Held in FP64: 0.05 to
+// 0.2 for all of them.  So FP32 only up to 1.5 roundings a product (QFT 1.2;
+// Ising steps 4, layers 10), where even roundings that add up stay below the
+// products'.
+bool gate_route(const GateListCost& cost, int n, Prec prec, Prec& held);
+
 // ---- host: planning ---------------------------------------------------------
 struct GatePassPlan {
      uint64_t bits = 0;                     // the tile's index bits
@@ -253,9 +279,11 @@ void check_gate_pass(const GatePass& pass, const std::vector<GateStage>& stages,
                      Prec prec, int n);
 
 // ---- launches (gate_kernels.hip) --------------------------------------------
-// One pass over a state of 2^n amplitudes (gate_tile_bits <= n <= 40); stages and ops are
-// device arrays, ops with one spare record at the end.  dst: where a permuted
+// One pass over a state of 2^n amplitudes (gate_tile_bits(held) <= n <= 40) of
+// precision prec, planned and compiled for precision held, which the
+// amplitudes have while the pass holds them; stages and ops are device arrays,
+// ops with one spare record at the end.  dst: where a permuted
 // pass stores (another buffer than psi).
-hipError_t launch_gate_pass(void* psi, Prec prec, int n_qubits, const GatePass& pass, const GateStage* stages,
+hipError_t launch_gate_pass(void* psi, Prec prec, Prec held, int n_qubits, const GatePass& pass, const GateStage* stages,
                             const void* ops, hipStream_t s, void* dst = nullptr);
 }  // namespace hq

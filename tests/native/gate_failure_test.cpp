@@ -14,10 +14,10 @@ namespace hq {
 long passes_run = 0, fail_launch = -1;  // passes until one fails
 long allocations_at_first_pass = 0;
 
-hipError_t launch_gate_pass(void* psi, Prec prec, int n, const GatePass& pass, const GateStage* stages, const void* ops,
+hipError_t launch_gate_pass(void* psi, Prec prec, Prec held, int n, const GatePass& pass, const GateStage* stages, const void* ops,
                             hipStream_t, void* dst)
 {
-     CHECK(prec == Prec::C128);
+     CHECK(prec == Prec::C128 && held == Prec::C128);
      if (fail_launch >= 0 && fail_launch-- == 0) return hipErrorLaunchFailure;
      if (passes_run++ == 0) allocations_at_first_pass = fake::allocations;
      auto* const p = static_cast<cplx*>(psi);
