@@ -1193,7 +1193,7 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, c
      for (size_t i = 0; i < items.size(); ++i)
           if (!make_gate_unit(items[i].m.a.data(), items[i].t, items[i].c, units[i])) return false;
      Prec held;
-     if (!gate_route(gate_list_cost(units), n, prec_, held)) return false;
+     if (!gate_route(gate_list_cost(units), units.size(), n, prec_, held)) return false;
      // What is on the stream leaves the list, also when something fails on the way.
      struct Rest {
           std::vector<PosGate>& items;

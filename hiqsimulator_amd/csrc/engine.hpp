@@ -202,7 +202,8 @@ private:
      // Returns the number of HBM passes launched.
      int tile_items(std::vector<PosGate>& items, int op_width, size_t keep);
      // The same by gate programs (gate_prog.hpp), for states of at least
-     // gate_min_qubits and lists whose gates mix at most two qubits each;
+     // gate_min_qubits and lists whose gates mix at most two qubits each, where
+     // that is the faster way (gate_route);
      // false (and nothing done) for others.  When it throws, `items` holds what
      // has not been applied.
      // src_pos: the last pass also permutes the index bits (launch_permute) into

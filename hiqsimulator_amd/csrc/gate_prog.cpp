@@ -148,14 +148,15 @@ Run run_of(const GateUnit& g)
 
 GateListCost gate_list_cost(const std::vector<GateUnit>& units)
 {
+     constexpr double kGeneral = 3.7, kTwo = 6.5, kFactor = 0.5, kTested = 2.0;
      constexpr int kWidth = 4;
      GateListCost c;
      Run run[64] = {};  // of each qubit's last gate, while it can still take another
      auto end_run = [&](uint64_t bits) {
           for (; bits; bits &= bits - 1) {
                Run& r = run[__builtin_ctzll(bits)];
-               if (r == kRunGeneral) c.rounds += 2;
-               else if (r != kRunNone) c.rounds += 1;
+               if (r == kRunGeneral) c.work += kGeneral, c.rounds += 2;
+               else if (r != kRunNone) c.work += 1, c.rounds += 1;
                r = kRunNone;
           }
      };
@@ -168,6 +169,7 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units)
           return true;
      };
      double slots = 0;
+     uint64_t mixed = 0;  // by the units so far
      for (const GateUnit& g: units) {
           const uint64_t bits = g.a | g.d;
           if (g.br.empty() || !bits) continue;  // (a factor of all amplitudes costs nothing)
@@ -184,11 +186,13 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units)
           else {
                end_run(g.na ? bits : 0);
                for (const auto& b: g.br) {
-                    if (g.na == 0) c.rounds += 0.25;
-                    else if (g.na == 2) c.rounds += 4;
-                    else if (!is_flip(b)) c.rounds += 2;
+                    if (g.na == 0) c.work += bits & ~mixed ? kFactor : kTested, c.rounds += 0.25;
+                    else if (g.na == 2) c.work += kTwo, c.rounds += 4;
+                    else if (is_flip(b)) c.work += 1;
+                    else c.work += kGeneral, c.rounds += 2;
                }
           }
+          mixed |= g.a;
           // the fused product that it would go into
           const int first = last[__builtin_ctzll(bits)];
           bool inside = first >= 0;
@@ -215,12 +219,16 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units)
      return c;
 }
 
-bool gate_route(const GateListCost& cost, int n, Prec prec, Prec& held)
+bool gate_route(const GateListCost& cost, size_t gates, int n, Prec prec, Prec& held)
 {
      held = Prec::C128;
      if (n < gate_min_qubits(prec) || n > 40) return false;
-     if (prec == Prec::C64 && cost.rounds <= 1.5 * cost.products) held = Prec::C64;
-     return true;
+     if (prec == Prec::C64 && cost.rounds <= 1.5 * cost.products) {
+          held = Prec::C64;
+          return true;
+     }
+     if (n <= 22 && cost.work <= 4.0 * static_cast<double>(gates)) return true;  // bound by the host
+     return n > 18 && cost.work <= (prec == Prec::C128 ? 24.0 : 13.0) * cost.products;
 }
 
 // ---------------------------------------------------------------------------

@@ -196,16 +196,33 @@ bool make_gate_unit(const std::complex<double>* m, const std::vector<int64_t>& t
 
 // ---- host: which way a list goes --------------------------------------------
 // What a list takes either way, counted in one sweep over its units.
+//   work      of a gate program: a rotation, a phase or a CNOT is 1, a general
+//             2 x 2 block 3.7, a 4 x 4 block 6.5, a conditional factor 0.5, or 2
+//             when its qubits are all mixed by gates before it (they are then
+//             often in registers together, where the factor is applied by
+//             itself); runs that become one matrix count once.
 //   products  fused products on four qubits that a tile program needs about:
 //             a quarter of the qubits of greedily grown groups of up to four.
 //   rounds    roundings of an amplitude that a gate program makes in the
 //             precision it is held in.
 struct GateListCost {
-     double products = 0, rounds = 0;
+     double work = 0, products = 0, rounds = 0;
 };
 GateListCost gate_list_cost(const std::vector<GateUnit>& units);
 // The precision that a gate program of the list would hold the amplitudes of
 // an n-qubit state in; false: the list runs as tile programs.
+//
+// Time.  Tile programs over gate programs, with work per product in brackets.
+// Complex128, 28 qubits: QFT (2) 7.5, CNOT ladder (3) 2.2, layers of rotations
+// and CNOTs (12) 1.6, Trotter steps of an Ising chain (14) 1.4, 2-qubit Haar
+// bricks (23) 1.2, three rotations a qubit and layer (27) 0.92, one-qubit Haar
+// and CNOT (31) 0.82, five rotations (40) 0.72, 200 layers on 4 qubits (1046)
+// 0.12: up to 24.  Complex64 held in FP64 against products in FP32, 28 qubits:
+// CNOT ladder 1.6, layers 1.0, Ising steps 0.75, 2-qubit bricks 0.71, three
+// rotations 0.58: up to 13.  Up to 22 qubits the host and a workgroup's latency
+// bound both ways (0.5 us a unit of work against 1.25 us a gate for the fusion):
+// of these lists only those of dense 2-qubit blocks are faster as products (0.66
+// at 13 qubits, 0.9 at 16, 1.1 at 20).
 //
 // Roundings.  Error of gate programs held in FP32 over that of tile programs (l2,
 // complex64, 25 qubits): QFT 0.54, layers with random angles 0.75, three
@@ -214,7 +231,7 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units);
 // 0.2 for all of them.  So FP32 only up to 1.5 roundings a product (QFT 1.2;
 // Ising steps 4, layers 10), where even roundings that add up stay below the
 // products'.
-bool gate_route(const GateListCost& cost, int n, Prec prec, Prec& held);
+bool gate_route(const GateListCost& cost, size_t gates, int n, Prec prec, Prec& held);
 
 // ---- host: planning ---------------------------------------------------------
 struct GatePassPlan {

@@ -264,7 +264,8 @@ int hiqsim_plan_clusters(const int64_t* gate_ids, const size_t* gate_off, const 
  * the handle's qubit ids.  From 13 qubits on in complex128 and 21 in
  * complex64, lists whose gates mix at most two qubits each (controls and
  * block-diagonal targets do not count) run gate by gate on tiles of 2^13 or
- * 2^14 amplitudes in registers.  Otherwise each HBM pass loads tiles of index
+ * 2^14 amplitudes in registers, unless they fuse into so few products that
+ * those are faster.  Otherwise each HBM pass loads tiles of index
  * bits {0..5} plus 6 planned bits into LDS and applies there every op its plan
  * holds (ops of at most op_width qubits, fused in FP64); the plan is the
  * cluster scheduler's rule with the tile as the local set.  Pending gates are

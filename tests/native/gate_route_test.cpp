@@ -1,0 +1,148 @@
+// Which way gate lists go, on the host: gate programs or tile programs, and for
+// complex64 states the precision that the amplitudes are held in.
+#define main gate_prog_main
+#include "gate_prog_test.cpp"
+#undef main
+
+namespace {
+
+struct Lists {
+     int n;
+     std::mt19937 rng{7};
+     double u() { return std::uniform_real_distribution<double>(0, 6.28)(rng); }
+     std::vector<cplx> rx(double t) { return {std::cos(t), cplx(0, -std::sin(t)), cplx(0, -std::sin(t)), std::cos(t)}; }
+     std::vector<cplx> ry(double t) { return {std::cos(t), -std::sin(t), std::sin(t), std::cos(t)}; }
+     std::vector<cplx> rz(double t) { return {std::polar(1.0, -t), 0, 0, std::polar(1.0, t)}; }
+     const std::vector<cplx> x{0, 1, 1, 0};
+     std::vector<cplx> dense(int d)
+     {
+          std::vector<cplx> m(d * d);
+          for (auto& z: m) z = cplx(u(), u());
+          return m;
+     }
+     // one of `one` for every qubit, then CNOTs, layer by layer
+     template <typename F>
+     std::vector<Gate> layers(int count, const std::vector<int64_t>& qs, F&& one)
+     {
+          std::vector<Gate> out;
+          for (int l = 0; l < count; ++l) {
+               for (int64_t q: qs) one(out, q);
+               for (size_t i = l % 2; i + 1 < qs.size(); i += 2) out.push_back({x, {qs[i + 1]}, {qs[i]}});
+          }
+          return out;
+     }
+     std::vector<int64_t> all() const
+     {
+          std::vector<int64_t> q(n);
+          for (int i = 0; i < n; ++i) q[i] = i;
+          return q;
+     }
+     std::vector<Gate> random_layers(int count)
+     {
+          return layers(count, all(), [&](std::vector<Gate>& out, int64_t q) {
+               const int k = static_cast<int>(rng() % 3);
+               out.push_back({k == 0 ? rx(u()) : (k == 1 ? ry(u()) : rz(u())), {q}, {}});
+          });
+     }
+     std::vector<Gate> zxzxz(int count, const std::vector<int64_t>& qs)
+     {
+          return layers(count, qs, [&](std::vector<Gate>& out, int64_t q) {
+               for (int i = 0; i < 5; ++i) out.push_back({i % 2 ? rx(u()) : rz(u()), {q}, {}});
+          });
+     }
+     std::vector<Gate> ising(int steps)
+     {
+          std::vector<Gate> out;
+          const cplx a = std::polar(1.0, 0.3), b = std::polar(1.0, -0.3);
+          for (int s = 0; s < steps; ++s) {
+               for (int i = 0; i + 1 < n; ++i) out.push_back({{a, 0, 0, 0, 0, b, 0, 0, 0, 0, b, 0, 0, 0, 0, a}, {i, i + 1}, {}});
+               for (int i = 0; i < n; ++i) out.push_back({rx(0.4), {i}, {}});
+          }
+          return out;
+     }
+     std::vector<Gate> ladder()
+     {
+          std::vector<Gate> out;
+          for (int r = 0; r < 8; ++r)
+               for (int i = 0; i + 1 < n; ++i) out.push_back({x, {i + 1}, {i}});
+          return out;
+     }
+     std::vector<Gate> bricks(const std::vector<int64_t>& qs, int count)
+     {
+          std::vector<Gate> out;
+          for (int l = 0; l < count; ++l)
+               for (size_t i = l % 2; i + 1 < qs.size(); i += 2) out.push_back({dense(4), {qs[i], qs[i + 1]}, {}});
+          return out;
+     }
+     std::vector<Gate> pair(int count)
+     {
+          std::vector<Gate> out;
+          for (int i = 0; i < count; ++i) out.push_back({dense(4), {1, n - 2}, {}});
+          return out;
+     }
+};
+
+enum Way { kTiles, kFp64, kFp32 };
+
+Way way(const std::vector<Gate>& gates, int n, Prec prec)
+{
+     std::vector<GateUnit> units(gates.size());
+     for (size_t i = 0; i < gates.size(); ++i) CHECK(make_gate_unit(gates[i].m.data(), gates[i].t, gates[i].c, units[i]));
+     const GateListCost c = gate_list_cost(units);
+     CHECK(c.work >= 0 && c.products >= 0 && c.rounds >= 0);
+     Prec held;
+     if (!gate_route(c, gates.size(), n, prec, held)) return kTiles;
+     return held == Prec::C128 ? kFp64 : kFp32;
+}
+
+}  // namespace
+
+int main()
+{
+     for (int n: {21, 24, 28, 34}) {
+          Lists l{n};
+          const std::vector<int64_t> few = {1, 5, n - 2, n / 2};
+          const bool large = n > 22;
+          // roundings of many rotations, of repeated ones and of long lists on few
+          // qubits are never made in FP32
+          for (int count: {2, 4, 20, 60}) CHECK(way(l.random_layers(count), n, Prec::C64) == kFp64);
+          for (int steps: {1, 5, 40}) CHECK(way(l.ising(steps), n, Prec::C64) != kFp32);
+          for (int count: {1, 10, 200}) CHECK(way(l.zxzxz(count, few), n, Prec::C64) != kFp32);
+          CHECK(way(Qft{n, 0}.gates(), n, Prec::C64) == kFp32);
+          CHECK(way(Qft{n, 5}.gates(), n, Prec::C64) == kFp32);
+          CHECK(way(l.ladder(), n, Prec::C64) == kFp32);
+          // lists that fuse into few products run as those
+          for (Prec prec: {Prec::C128, Prec::C64}) {
+               CHECK((way(l.zxzxz(200, few), n, prec) == kTiles) == large);
+               CHECK((way(l.zxzxz(6, l.all()), n, prec) == kTiles) == large);
+               CHECK(way(l.pair(40), n, prec) == kTiles);
+          }
+          // and those that do not as gate programs
+          CHECK(way(l.random_layers(20), n, Prec::C128) == kFp64);
+          CHECK(way(l.ising(5), n, Prec::C128) == kFp64);
+          CHECK(way(l.ladder(), n, Prec::C128) == kFp64);
+          CHECK(way(Qft{n, 3}.gates(), n, Prec::C128) == kFp64);
+          CHECK(way(l.bricks(l.all(), 6), n, Prec::C128) == kFp64);
+     }
+     // small states
+     for (int n: {13, 16, 18}) {
+          Lists l{n};
+          CHECK(way(l.random_layers(20), n, Prec::C128) == kFp64);
+          CHECK(way(l.zxzxz(200, {1, 5, n - 2, n / 2}), n, Prec::C128) == kFp64);
+          CHECK(way(l.bricks(l.all(), 6), n, Prec::C128) == kTiles);
+          CHECK(way(l.random_layers(20), n, Prec::C64) == kTiles);
+     }
+     CHECK(way(Lists{12}.random_layers(3), 12, Prec::C128) == kTiles);
+     // empty lists, identities and factors of everything
+     {
+          Lists l{24};
+          Prec held;
+          CHECK(gate_route(gate_list_cost({}), 0, 24, Prec::C128, held));
+          std::vector<Gate> id(10, Gate{{1, 0, 0, 1}, {3}, {}});
+          CHECK(way(id, 24, Prec::C64) == kFp32);
+          id.push_back(Gate{{cplx(0, 1), 0, 0, cplx(0, 1)}, {2}, {}});
+          CHECK(way(id, 24, Prec::C128) == kFp64);
+     }
+     std::printf("gate routes ok\n");
+     return 0;
+}
