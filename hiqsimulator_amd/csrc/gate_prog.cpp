@@ -269,12 +269,13 @@ uint64_t GatePassPlanner::choose(const std::vector<int>& list, uint64_t fixed, u
      }
      pool &= allowed & ~fixed;
      // Units that bit set S takes, mixing units counted first; the scan ends
-     // when every bit of S is blocked.
+     // when every bit of S is blocked, or where a pass is full.
+     const size_t window = std::min(list.size(), kGateMaxPassUnits);
      auto score = [&](uint64_t S) {
           uint64_t ba = 0, bd = 0;
           int s = 0;
-          for (int i: list) {
-               const GateUnit& g = units_[i];
+          for (size_t at = 0; at < window; ++at) {
+               const GateUnit& g = units_[list[at]];
                if (!(g.a & ~S) && !(g.a & (ba | bd)) && !(g.d & ba)) {
                     s += g.a ? 256 : 1;
                }
@@ -389,7 +390,7 @@ bool GatePassPlanner::next(GatePassPlan& out)
      out.bits = low | choose(rem_, low, all, gate_high(prec_));
      for (int p = kGateLow; p < n_ && popc(out.bits) < gate_tile_bits(prec_); ++p) out.bits |= uint64_t(1) << p;
      std::vector<int> taken;
-     take(rem_, out.bits, rem_.size(), taken);
+     take(rem_, out.bits, kGateMaxPassUnits, taken);
      if (taken.empty()) throw std::runtime_error("gate program: no gate could be planned");
      const std::vector<int> whole = splits_ ? taken : std::vector<int>();
      size_t groupings = make_stages(taken, out, false, false);
