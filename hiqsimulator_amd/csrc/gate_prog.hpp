@@ -59,7 +59,7 @@ constexpr size_t kGateMaxStages = 255;      // a pass's stage count is a byte
 constexpr size_t kGateMaxStageUnits = 512;  // and a stage's record count 16 bits
 // Units of a pass: far beyond what its reads and writes are worth, and a bound
 // for the planner's scans (100000 gates on 13 qubits were planned in 1.2 s, each
-// pass over all that were left; 0.25 s now).
+// pass over all that were left; 0.13 s now).
 constexpr size_t kGateMaxPassUnits = 4096;
 
 // ---- device records ---------------------------------------------------------

@@ -62,19 +62,24 @@ PauliPlan plan_pauli(const std::vector<PauliTermIn>& in, int n, bool apply)
           if (diagonal) here.push_back(0);
           diagonal = false;
           for (;;) {
+               // (a sweep takes all that need none: at most H + 1 sweeps a pass)
                int best = -1, need = H + 1;
-               for (size_t i = 0; i < left.size(); ++i) {
-                    const int k = popc(left[i] & ~bits);
-                    if (popc(bits | left[i]) <= T && k < need) {
-                         need = k;
-                         best = static_cast<int>(i);
-                         if (k == 0) break;
+               size_t kept = 0;
+               for (uint64_t x: left) {
+                    const int k = popc(x & ~bits);
+                    if (k == 0) {
+                         here.push_back(x);
+                         continue;
                     }
+                    if (popc(bits) + k <= T && k < need) {
+                         need = k;
+                         best = static_cast<int>(kept);
+                    }
+                    left[kept++] = x;
                }
+               left.resize(kept);
                if (best < 0) break;
                bits |= left[best];
-               here.push_back(left[best]);
-               left.erase(left.begin() + best);
           }
           for (int p = 0; p < n && popc(bits) < T; ++p) bits |= uint64_t(1) << p;
           int rank[64], r = 0;

@@ -1,4 +1,5 @@
-// Planning time of long gate lists on few qubits, on the host: eight times the length may take at most sixteen times as
+// Planning time of long gate lists on few qubits and of Pauli sums with many
+// strings, on the host: eight times the length may take at most sixteen times as
 // long (a plan that looks at everything left at every step takes sixty-four).
 #include <chrono>
 #include <cmath>
@@ -6,6 +7,7 @@
 #include <random>
 
 #include "../../hiqsimulator_amd/csrc/gate_prog.hpp"
+#include "../../hiqsimulator_amd/csrc/pauli_prog.hpp"
 
 using namespace hq;
 using cplx = std::complex<double>;
@@ -45,6 +47,22 @@ double plan_gates(int n, int count)
      });
 }
 
+double plan_strings(int n, int count)
+{
+     std::mt19937 rng(2);
+     std::vector<PauliTermIn> in;
+     for (int i = 0; i < count; ++i) {
+          uint64_t x = 0, z = 0;
+          for (int k = 0; k < 8; ++k) {
+               const int q = static_cast<int>(rng() % n), s = static_cast<int>(rng() % 3);
+               if (s < 2) x |= uint64_t(1) << q;
+               if (s > 0) z |= uint64_t(1) << q;
+          }
+          in.push_back({x, z, cplx(0.1, 0)});
+     }
+     return best_of_three([&] { (void)plan_pauli(in, n, true); });
+}
+
 bool scales(const char* what, double small, double large)
 {
      std::printf("%s: %.1f and %.1f ms\n", what, 1e3 * small, 1e3 * large);
@@ -55,7 +73,8 @@ bool scales(const char* what, double small, double large)
 
 int main()
 {
-     const bool ok = scales("gates", plan_gates(14, 12500), plan_gates(14, 100000));
+     bool ok = scales("gates", plan_gates(14, 12500), plan_gates(14, 100000));
+     ok = scales("strings", plan_strings(20, 5000), plan_strings(20, 40000)) && ok;
      if (ok) std::printf("planning scales\n");
      return ok ? 0 : 1;
 }

@@ -1,4 +1,4 @@
-"""Planning time of gate programs over long lists, on the host
+"""Planning time of gate programs and Pauli sums over long inputs, on the host
 (tests/native/plan_scaling_test.cpp)."""
 import os
 import subprocess
@@ -15,7 +15,7 @@ def test_planning_scales(tmp_path):
         pytest.skip("HIP headers not installed")
     exe = str(tmp_path / "plan_scaling_test")
     subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I" + hip_inc] +
-                   [os.path.join(CSRC, s) for s in ("gate_prog.cpp",)] +
+                   [os.path.join(CSRC, s) for s in ("gate_prog.cpp", "pauli_prog.cpp")] +
                    [os.path.join(HERE, "native", "plan_scaling_test.cpp"), "-o", exe], check=True)
     out = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0 and "planning scales" in out.stdout, out.stdout + out.stderr[-4000:]
