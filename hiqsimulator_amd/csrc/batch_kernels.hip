@@ -17,6 +17,7 @@
 #include <cstdint>
 
 #include "batch.hpp"
+#include "running_sums.hpp"
 #include "device_common.hpp"
 
 namespace hq {
@@ -1049,8 +1050,8 @@ __global__ void __launch_bounds__(kBatchLayerBlock)
 
 constexpr int kSampleThreads = 1024;
 
-// Running sums of each job's block probabilities, in place; one workgroup per
-// job, a run of `per` consecutive blocks per thread.  From eight a thread on,
+// Running sums of each job's block probabilities, in place (running_sums.hpp);
+// one workgroup per job, a run of `per` consecutive blocks per thread.  From eight a thread on,
 // a wave moves its runs through LDS eight columns at a time, so that global
 // memory sees whole 64-byte pieces: each thread at its own run took 64 us for
 // the 2^15 blocks of a 28-qubit complex64 state, 19 us now.
@@ -1076,20 +1077,21 @@ __device__ __forceinline__ void running_sums(double* __restrict__ cdf, const uin
      const uint32_t t = threadIdx.x, lane = t & 63;
      const uint32_t first = t * per;
      __shared__ double part[kSampleThreads];
+     __shared__ double wave_end[kSampleThreads / 64];
      __shared__ double cols[kSampleThreads / 64][64 * (kCdfCols + 1)];
      double* const lds = cols[t >> 6];
      double* const base = cdf + static_cast<uint64_t>(t - lane) * per;
-     double local = 0.0;
+     BlockRun local;
      if (per >= kCdfCols)  // (a power of two: whole groups of columns)
           for (uint32_t i = 0; i < per; i += kCdfCols) {
                double v[kCdfCols];
                cdf_columns(base, per, i, lds, lane, v);
 #pragma unroll
-               for (int j = 0; j < kCdfCols; ++j) local += v[j];
+               for (uint32_t j = 0; j < kCdfCols; ++j) local.add(v[j], static_cast<int>(i + j));
           }
      else if (first < nb)
-          for (uint32_t i = 0; i < per; ++i) local += cdf[first + i];
-     part[t] = local;
+          for (uint32_t i = 0; i < per; ++i) local.add(cdf[first + i], static_cast<int>(i));
+     part[t] = local.sum;
      __syncthreads();
      for (uint32_t o = 1; o < kSampleThreads; o <<= 1) {
           const double add = t >= o ? part[t - o] : 0.0;
@@ -1097,6 +1099,17 @@ __device__ __forceinline__ void running_sums(double* __restrict__ cdf, const uin
           part[t] += add;
           __syncthreads();
      }
+     // the ends of the runs: the largest so far
+     double end = local.end(part[t]);
+     for (int o = 1; o < 64; o <<= 1) {
+          const double e = __shfl_up(end, o, 64);
+          if (lane >= static_cast<uint32_t>(o)) end = larger(e, end);
+     }
+     if (lane == 63) wave_end[t >> 6] = end;
+     __syncthreads();
+     for (uint32_t w = 0; w < (t >> 6); ++w) end = larger(wave_end[w], end);
+     part[t] = end;
+     __syncthreads();
      double run = t ? part[t - 1] : 0.0;
      if (per >= kCdfCols)
           for (uint32_t i = 0; i < per; i += kCdfCols) {
@@ -1105,7 +1118,7 @@ __device__ __forceinline__ void running_sums(double* __restrict__ cdf, const uin
 #pragma unroll
                for (uint32_t j = 0; j < kCdfCols; ++j) {
                     run += v[j];
-                    lds[lane * (kCdfCols + 1) + j] = run;
+                    lds[lane * (kCdfCols + 1) + j] = running_sum(run, static_cast<int>(i + j), local.last, end);
                }
                __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -1118,7 +1131,7 @@ __device__ __forceinline__ void running_sums(double* __restrict__ cdf, const uin
      else if (first < nb)
           for (uint32_t i = 0; i < per; ++i) {
                run += cdf[first + i];
-               cdf[first + i] = run;
+               cdf[first + i] = running_sum(run, static_cast<int>(i), local.last, end);
           }
 }
 
@@ -1226,7 +1239,8 @@ __global__ void __launch_bounds__(kSampleThreads)
      running_sums(sums, nb);
      __syncthreads();
      if (threadIdx.x >= 64) return;
-     const uint64_t at = find_outcome<R, true>(psi, sums, nb, 1ull << log_block_amps, u, threadIdx.x);
+     // (0 as the smallest number above it: its block holds something)
+     const uint64_t at = find_outcome<R, true>(psi, sums, nb, 1ull << log_block_amps, u > 0.0 ? u : 0x1p-1074, threadIdx.x);
      if (threadIdx.x == 0) {
           __hip_atomic_store(out, at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
           __hip_atomic_store(out + 1, static_cast<uint64_t>(__double_as_longlong(sums[nb - 1])), __ATOMIC_RELAXED,
