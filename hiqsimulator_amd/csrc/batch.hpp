@@ -135,6 +135,7 @@ struct SampleJob {
      uint32_t log_block_amps;
      uint32_t shots;
      uint32_t pad;
+     uint64_t shot_first;  // shots of the jobs before it
 };
 // Probability blocks of a sample job over 2^n amplitudes: blocks of at
 // least 256 amplitudes, at most 2^15 blocks.
@@ -144,8 +145,8 @@ inline uint32_t sample_log_blocks(int n)
      return static_cast<uint32_t>(lb < 0 ? 0 : (lb > 15 ? 15 : lb));
 }
 // The jobs' block probabilities become running sums in place;
-// out[out_off + s] = outcome of shot s.  max_shots: the largest job's.
-hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, int njobs, uint32_t max_shots,
+// out[out_off + s] = outcome of shot s.  total_shots: of all jobs.  Two launches.
+hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, int njobs, uint64_t total_shots,
                          double* sums, uint64_t* out, hipStream_t s);
 // The outcome at the point u of the running probability of one state: the
 // first index whose running sum reaches u.  sums: the probabilities of its

@@ -1202,26 +1202,35 @@ __global__ void __launch_bounds__(kSampleThreads)
      running_sums(sums + jb.sums_off, 1u << jb.log_blocks);
 }
 
-// One wave per shot, four shots a workgroup; blockIdx.y = the job.  A single
-// thread that scanned the block for its shot took 4.2 ms for 1024 shots of a
-// 28-qubit complex64 state (8192 amplitudes a block, all loads in a chain);
-// this takes 0.02 ms.
+// One wave per shot, four at a time a workgroup, over the shots of all jobs in a
+// row.  A single thread that scanned the block for its shot took 4.2 ms for
+// 1024 shots of a 28-qubit complex64 state (8192 amplitudes a block, all loads
+// in a chain); this takes 0.02 ms.
+constexpr uint64_t kSampleBlocks = uint64_t(1) << 20;  // more shots go round (the limit is 2^32 threads)
 template <typename R>
 __global__ void __launch_bounds__(256)
-    k_sample_shots(const VT<R>* __restrict__ arena, const SampleJob* __restrict__ jobs,
-                   const double* __restrict__ sums, uint64_t* __restrict__ out)
+    k_sample_shots(const VT<R>* __restrict__ arena, const SampleJob* __restrict__ jobs, const uint32_t njobs,
+                   const uint64_t total, const double* __restrict__ sums, uint64_t* __restrict__ out)
 {
-     const SampleJob jb = jobs[blockIdx.y];
-     const uint32_t s = blockIdx.x * 4 + (threadIdx.x >> 6);
      const uint32_t lane = threadIdx.x & 63;
-     if (s >= jb.shots) return;  // (whole waves; no barrier below)
-     const double* const cdf = sums + jb.sums_off;
-     const uint32_t nb = 1u << jb.log_blocks;
-     const uint2 key = make_uint2(static_cast<uint32_t>(jb.seed), static_cast<uint32_t>(jb.seed >> 32));
-     const uint4 r = philox4x32_10(make_uint4(s, 0u, 0x5a3du, 0u), key);
-     const double u = uniform53(r.x, r.y) * cdf[nb - 1];
-     const uint64_t at = find_outcome<R, false>(arena + jb.state_off, cdf, nb, 1ull << jb.log_block_amps, u, lane);
-     if (lane == 0) out[jb.out_off + s] = at;
+     const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
+     for (uint64_t g = static_cast<uint64_t>(blockIdx.x) * 4 + wave; g < total; g += static_cast<uint64_t>(gridDim.x) * 4) {
+          uint32_t lo = 0, hi = njobs;  // the last job that begins at or before shot g
+          while (hi - lo > 1) {
+               const uint32_t mid = (lo + hi) / 2;
+               if (jobs[mid].shot_first <= g) lo = mid;
+               else hi = mid;
+          }
+          const SampleJob jb = jobs[lo];
+          const uint32_t s = static_cast<uint32_t>(g - jb.shot_first);
+          const double* const cdf = sums + jb.sums_off;
+          const uint32_t nb = 1u << jb.log_blocks;
+          const uint2 key = make_uint2(static_cast<uint32_t>(jb.seed), static_cast<uint32_t>(jb.seed >> 32));
+          const uint4 r = philox4x32_10(make_uint4(s, 0u, 0x5a3du, 0u), key);
+          const double u = uniform53(r.x, r.y) * cdf[nb - 1];
+          const uint64_t at = find_outcome<R, false>(arena + jb.state_off, cdf, nb, 1ull << jb.log_block_amps, u, lane);
+          if (lane == 0) out[jb.out_off + s] = at;
+     }
 }
 
 // A measurement's outcome: the running sums, then the search, in one
@@ -1463,23 +1472,22 @@ hipError_t launch_block_sums_multi(const void* arena, Prec prec, const BatchItem
      return hipGetLastError();
 }
 
-hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, int njobs, uint32_t max_shots,
+hipError_t launch_sample(const void* arena, Prec prec, const SampleJob* jobs, int njobs, uint64_t total_shots,
                          double* sums, uint64_t* out, hipStream_t s)
 {
-     if (njobs <= 0 || max_shots == 0) return hipSuccess;
+     if (njobs <= 0 || total_shots == 0) return hipSuccess;
      hipLaunchKernelGGL(k_sample_cdf, dim3(njobs), dim3(kSampleThreads), 0, s, jobs, sums);
-     hipError_t e = hipGetLastError();
-     for (int j = 0; e == hipSuccess && j < njobs; j += 65535) {  // the limit of a grid's y
-          const dim3 grid((max_shots + 3) / 4, static_cast<unsigned>(njobs - j < 65535 ? njobs - j : 65535));
-          if (prec == Prec::C128)
-               hipLaunchKernelGGL((k_sample_shots<double>), grid, dim3(256), 0, s, static_cast<const double2*>(arena),
-                                  jobs + j, sums, out);
-          else
-               hipLaunchKernelGGL((k_sample_shots<float>), grid, dim3(256), 0, s, static_cast<const float2*>(arena),
-                                  jobs + j, sums, out);
-          e = hipGetLastError();
-     }
-     return e;
+     const hipError_t e = hipGetLastError();
+     if (e != hipSuccess) return e;
+     const uint64_t blocks = (total_shots + 3) / 4;
+     const dim3 grid(static_cast<unsigned>(blocks < kSampleBlocks ? blocks : kSampleBlocks));
+     if (prec == Prec::C128)
+          hipLaunchKernelGGL((k_sample_shots<double>), grid, dim3(256), 0, s, static_cast<const double2*>(arena), jobs,
+                             static_cast<uint32_t>(njobs), total_shots, sums, out);
+     else
+          hipLaunchKernelGGL((k_sample_shots<float>), grid, dim3(256), 0, s, static_cast<const float2*>(arena), jobs,
+                             static_cast<uint32_t>(njobs), total_shots, sums, out);
+     return hipGetLastError();
 }
 
 hipError_t launch_measure(const void* psi, Prec prec, double* sums, int log_blocks, int log_block_amps, double u,

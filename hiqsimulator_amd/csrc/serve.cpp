@@ -540,7 +540,7 @@ std::vector<int64_t> Server::step(bool block)
      // Outputs of the requests that finish in this step.
      ItemList sums;
      std::vector<SampleJob> jobs;
-     uint32_t max_shots = 0;
+     uint64_t total_shots = 0;
      std::vector<std::pair<int64_t, size_t>> outs;
      size_t out_bytes = 0;
      uint64_t sums_needed = 0;
@@ -562,7 +562,8 @@ std::vector<int64_t> Server::step(bool block)
                j.log_blocks = lb;
                j.log_block_amps = static_cast<uint32_t>(r.n) - lb;
                j.shots = r.shots;
-               max_shots = std::max(max_shots, j.shots);
+               j.shot_first = total_shots;
+               total_shots += j.shots;
                jobs.push_back(j);
                sums_needed += uint64_t(1) << lb;
                out_bytes += align_up(r.shots * sizeof(uint64_t), 256);
@@ -668,7 +669,7 @@ std::vector<int64_t> Server::step(bool block)
                                         sums.blocks, d_sums_, stream_),
                 "launch_block_sums_multi");
           check(launch_sample(d_states_, prec_, reinterpret_cast<const SampleJob*>(slot.d_desc + o_jobs),
-                              static_cast<int>(jobs.size()), max_shots, d_sums_,
+                              static_cast<int>(jobs.size()), total_shots, d_sums_,
                               reinterpret_cast<uint64_t*>(slot.d_out), stream_),
                 "launch_sample");
           stats_.launches += 2;
