@@ -1051,10 +1051,10 @@ __global__ void __launch_bounds__(kBatchLayerBlock)
 constexpr int kSampleThreads = 1024;
 
 // Running sums of each job's block probabilities, in place (running_sums.hpp);
-// one workgroup per job, a run of `per` consecutive blocks per thread.  From eight a thread on,
-// a wave moves its runs through LDS eight columns at a time, so that global
-// memory sees whole 64-byte pieces: each thread at its own run took 64 us for
-// the 2^15 blocks of a 28-qubit complex64 state, 19 us now.
+// one workgroup per job, a run of `per` consecutive blocks per thread.  From
+// eight a thread on, a wave moves its runs through LDS eight columns at a time,
+// so that global memory sees whole 64-byte pieces: each thread at its own run
+// took 64 us for the 2^15 blocks of a 28-qubit complex64 state, 20 us now.
 constexpr int kCdfCols = 8;
 
 __device__ __forceinline__ void cdf_columns(double* __restrict__ base, uint32_t per, uint32_t i0, double* lds,
@@ -1074,12 +1074,12 @@ __device__ __forceinline__ void cdf_columns(double* __restrict__ base, uint32_t 
 __device__ __forceinline__ void running_sums(double* __restrict__ cdf, const uint32_t nb)
 {
      const uint32_t per = nb > kSampleThreads ? nb / kSampleThreads : 1u;
-     const uint32_t t = threadIdx.x, lane = t & 63;
+     constexpr int kWaves = kSampleThreads / 64;
+     const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
      const uint32_t first = t * per;
-     __shared__ double part[kSampleThreads];
-     __shared__ double wave_end[kSampleThreads / 64];
-     __shared__ double cols[kSampleThreads / 64][64 * (kCdfCols + 1)];
-     double* const lds = cols[t >> 6];
+     __shared__ double wave_sum[kWaves], wave_end[kWaves];
+     __shared__ double cols[kWaves][64 * (kCdfCols + 1)];
+     double* const lds = cols[wave];
      double* const base = cdf + static_cast<uint64_t>(t - lane) * per;
      BlockRun local;
      if (per >= kCdfCols)  // (a power of two: whole groups of columns)
@@ -1091,26 +1091,39 @@ __device__ __forceinline__ void running_sums(double* __restrict__ cdf, const uin
           }
      else if (first < nb)
           for (uint32_t i = 0; i < per; ++i) local.add(cdf[first + i], static_cast<int>(i));
-     part[t] = local.sum;
-     __syncthreads();
-     for (uint32_t o = 1; o < kSampleThreads; o <<= 1) {
-          const double add = t >= o ? part[t - o] : 0.0;
-          __syncthreads();
-          part[t] += add;
-          __syncthreads();
-     }
-     // the ends of the runs: the largest so far
-     double end = local.end(part[t]);
+     // the runs' sums, scanned inside the wave and over the waves; then their
+     // ends, the largest so far
+     double scan = local.sum;
      for (int o = 1; o < 64; o <<= 1) {
-          const double e = __shfl_up(end, o, 64);
-          if (lane >= static_cast<uint32_t>(o)) end = larger(e, end);
+          const double v = __shfl_up(scan, o, 64);
+          if (lane >= static_cast<uint32_t>(o)) scan += v;
      }
-     if (lane == 63) wave_end[t >> 6] = end;
+     if (lane == 63) wave_sum[wave] = scan;
      __syncthreads();
-     for (uint32_t w = 0; w < (t >> 6); ++w) end = larger(wave_end[w], end);
-     part[t] = end;
+     double w = lane < kWaves ? wave_sum[lane] : 0.0;
+     for (int o = 1; o < kWaves; o <<= 1) {
+          const double v = __shfl_up(w, o, 64);
+          if (lane >= static_cast<uint32_t>(o)) w += v;
+     }
+     const double sum_before = __shfl(w, wave ? static_cast<int>(wave) - 1 : 0, 64);
+     if (wave) scan += sum_before;
+     double end = local.end(scan);
+     for (int o = 1; o < 64; o <<= 1) {
+          const double v = __shfl_up(end, o, 64);
+          if (lane >= static_cast<uint32_t>(o)) end = larger(v, end);
+     }
+     if (lane == 63) wave_end[wave] = end;
      __syncthreads();
-     double run = t ? part[t - 1] : 0.0;
+     w = lane < kWaves ? wave_end[lane] : 0.0;
+     for (int o = 1; o < kWaves; o <<= 1) {
+          const double v = __shfl_up(w, o, 64);
+          if (lane >= static_cast<uint32_t>(o)) w = larger(v, w);
+     }
+     double before = __shfl(w, wave ? static_cast<int>(wave) - 1 : 0, 64);
+     if (!wave) before = 0.0;
+     end = larger(before, end);
+     double run = __shfl_up(end, 1, 64);
+     if (lane == 0) run = before;
      if (per >= kCdfCols)
           for (uint32_t i = 0; i < per; i += kCdfCols) {
                double v[kCdfCols];

@@ -36,11 +36,18 @@ std::vector<double> running(const std::vector<double>& p)
           for (int i = 0; i < per && t * per + i < nb; ++i) run[t].add(p[t * per + i], i);
           part[t] = run[t].sum;
      }
-     for (int o = 1; o < kThreads; o <<= 1) {
-          std::vector<double> next = part;
-          for (int t = o; t < kThreads; ++t) next[t] += part[t - o];
-          part.swap(next);
+     // inside the waves, then over them
+     auto scan = [](std::vector<double>& v, int first, int count) {
+          for (int o = 1; o < count; o <<= 1)
+               for (int i = count - 1; i >= o; --i) v[first + i] += v[first + i - o];
+     };
+     std::vector<double> waves(kThreads / 64);
+     for (int w = 0; w < kThreads / 64; ++w) {
+          scan(part, 64 * w, 64);
+          waves[w] = part[64 * w + 63];
      }
+     scan(waves, 0, kThreads / 64);
+     for (int t = 64; t < kThreads; ++t) part[t] += waves[t / 64 - 1];
      for (int t = 0; t < kThreads; ++t) {
           end[t] = run[t].end(part[t]);
           if (t) end[t] = larger(end[t - 1], end[t]);
