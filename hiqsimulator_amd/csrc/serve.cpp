@@ -672,7 +672,7 @@ std::vector<int64_t> Server::step(bool block)
                               static_cast<int>(jobs.size()), total_shots, d_sums_,
                               reinterpret_cast<uint64_t*>(slot.d_out), stream_),
                 "launch_sample");
-          stats_.launches += 2;
+          stats_.launches += 3;  // block sums, running sums, shots
      }
      for (const auto& fo: outs) {
           const Req& r = reqs_.at(fo.first);
