@@ -45,26 +45,30 @@ Readback::~Readback()
 {
      for (auto e: ev_)
           if (e) (void)hipEventDestroy(e);
+     if (h_one_) (void)hipHostFree(h_one_);
      if (h_) (void)hipHostFree(h_);
 }
 
-void Readback::ensure()
+// What the first small or large read needs.
+void Readback::ensure(bool one)
 {
-     if (h_) return;
+     if (one && !h_one_) {
+          ok(hipHostMalloc(reinterpret_cast<void**>(&h_one_), kOneGroup * 16 + 64, hipHostMallocDefault),
+             "hipHostMalloc(readback)");
+          std::memset(h_one_ + kOneGroup * 16, 0, 64);
+     }
+     if (one || h_) return;
      for (auto& e: ev_)
           if (!e) ok(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
-     ok(hipHostMalloc(reinterpret_cast<void**>(&h_), 2 * kChunk * 16 + 64, hipHostMallocDefault),
-        "hipHostMalloc(readback)");
-     std::memset(h_ + 2 * kChunk * 16, 0, 64);
+     ok(hipHostMalloc(reinterpret_cast<void**>(&h_), 2 * kChunk * 16, hipHostMallocDefault), "hipHostMalloc(readback)");
 }
 
 void Readback::read(const void* psi, Prec prec, uint64_t n, std::complex<double>* out, hipStream_t s)
 {
-     std::lock_guard<std::mutex> lk(m_);
-     ensure();
-     auto* const flag = reinterpret_cast<uint64_t*>(h_ + 2 * kChunk * 16);
+     ensure(n <= kOneGroup);
      if (n <= kOneGroup) {
-          auto* const d = reinterpret_cast<double2*>(h_);
+          auto* const flag = reinterpret_cast<uint64_t*>(h_one_ + kOneGroup * 16);
+          auto* const d = reinterpret_cast<double2*>(h_one_);
           ++seq_;
           if (prec == Prec::C128)
                hipLaunchKernelGGL((k_read_out_one<double2>), dim3(1), dim3(kThreads), 0, s, d,
@@ -79,7 +83,7 @@ void Readback::read(const void* psi, Prec prec, uint64_t n, std::complex<double>
                     ok(hipStreamSynchronize(s), "hipStreamSynchronize");
                     break;
                }
-          std::memcpy(out, h_, n * 16);
+          std::memcpy(out, h_one_, n * 16);
           return;
      }
      const uint64_t chunks = (n + kChunk - 1) / kChunk;

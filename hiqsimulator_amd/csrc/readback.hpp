@@ -4,7 +4,6 @@
 #include <hip/hip_runtime.h>
 #include <complex>
 #include <cstdint>
-#include <mutex>
 
 namespace hq {
 
@@ -15,8 +14,8 @@ namespace hq {
 // Times of get_state before (copy into pageable memory) and now: 2^4
 // amplitudes 20 / 7 us, complex128 2^15 226 / 31 us, 2^20 0.94 / 0.70 ms, 2^27
 // 206 / 162 ms; complex64 2^12 130 / 14 us, 2^18 0.41 / 0.18 ms, 2^27 389 / 162
-// ms.  The buffers (2 MiB) are allocated by the first read and freed with the
-// object.  Safe for several threads.
+// ms.  The buffers (16 KiB for states of one workgroup, 2 MiB for others) are
+// allocated by the first read that needs them and freed with the object.
 class Readback {
 public:
      Readback() = default;
@@ -32,9 +31,9 @@ public:
      static constexpr uint64_t kOneGroup = 1024;
 
 private:
-     void ensure();
-     std::mutex m_;
-     char* h_ = nullptr;  // two chunks, then the flag
+     void ensure(bool one);
+     char* h_one_ = nullptr;  // kOneGroup amplitudes, then the flag
+     char* h_ = nullptr;      // two chunks
      hipEvent_t ev_[2] = {nullptr, nullptr};
      uint64_t seq_ = 0;
 };
