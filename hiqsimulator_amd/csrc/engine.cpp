@@ -1656,14 +1656,14 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
           constexpr double kSegment = 256.0;
           const double whole = std::abs(t) * bound;
           const uint64_t segments = static_cast<uint64_t>(std::ceil(whole / kSegment));
-          Buf t1(bytes), w_own(cmask ? bytes : 0), out_own(cmask ? bytes : 0);
+          // The state itself is only read until the whole sum is there.
+          Buf t1(bytes), t2(bytes), own(cmask ? bytes : 0), sum(cmask ? bytes : 0), other(segments > 1 ? bytes : 0);
           if (!cmask) ensure_tmp(n_amps_);
-          void* w = cmask ? w_own.p : d_state_;  // T_0, destroyed
-          void* out = cmask ? out_own.p : d_tmp_;
+          const void* from = cmask ? own.p : d_state_;  // T_0 of a segment
+          void* const last_out = cmask ? sum.p : d_tmp_;
           if (cmask) {
-               check(launch_copy(w, d_state_, prec_, n_amps_, stream_), "copy");
-               check(launch_normalize(w, prec_, n_amps_, cmask, cmask, 1.0, nullptr, stream_), "select");
-               check(launch_pauli_accumulate(d_state_, w, prec_, n_amps_, 0, 0, -1.0, 0.0, stream_), "subtract");
+               check(launch_copy(own.p, d_state_, prec_, n_amps_, stream_), "copy");
+               check(launch_normalize(own.p, prec_, n_amps_, cmask, cmask, 1.0, nullptr, stream_), "select");
           }
           const std::vector<double> bes = bessel_series(whole / static_cast<double>(segments));
           const PauliTerm* terms = nullptr;
@@ -1679,20 +1679,20 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
                return 2.0 * (k < bes.size() ? bes[k] : 0.0) * ipow(t < 0 ? e : (4 - e) & 3);
           };
           for (uint64_t seg = 0; seg < segments; ++seg) {
-               if (seg > 0) std::swap(w, out);
-               void* cur = w;
-               void* next = t1.p;
+               void* const out = (segments - 1 - seg) % 2 ? other.p : last_out;
                for (size_t k = 1; k <= last; ++k) {
+                    void* const dst = k % 2 ? t1.p : t2.p;  // T_k, and T_{k-2} before
+                    const void* const src = k == 1 ? from : (k % 2 ? t2.p : t1.p);
                     for (size_t p = 0; p < plan.passes.size(); ++p) {
                          PauliApply q;
-                         q.src = cur;
-                         q.dst = next;
+                         q.src = src;
+                         q.dst = dst;
                          q.fr = k == 1 ? 1.0 : 2.0;
                          if (p > 0) {
-                              q.add = next;
+                              q.add = dst;
                          }
                          else if (k > 1) {
-                              q.add = next;  // T_{k-2}
+                              q.add = k == 2 ? from : dst;
                               q.g = -1.0;
                          }
                          if (p + 1 == plan.passes.size() && (k % 2 == 1 || k == last)) {
@@ -1706,16 +1706,19 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
                          }
                          check(launch_pauli_apply(q, prec_, n_qubits(), plan.passes[p], terms, stream_), "pauli_apply");
                     }
-                    std::swap(cur, next);
                }
+               from = out;
           }
           program_done(ps);
           if (c0 != cplx(0, 0)) {
                const cplx ph = std::exp(cplx(0, -t) * c0);
-               check(launch_scale(out, prec_, n_amps_, ph.real(), ph.imag(), stream_), "phase");
+               check(launch_scale(last_out, prec_, n_amps_, ph.real(), ph.imag(), stream_), "phase");
           }
-          if (cmask) check(launch_pauli_accumulate(d_state_, out, prec_, n_amps_, 0, 0, 1.0, 0.0, stream_), "add");
-          else if (out == d_tmp_) commit_tmp();  // (else the sum lies in the state already)
+          if (cmask) {
+               check(launch_pauli_accumulate(d_state_, own.p, prec_, n_amps_, 0, 0, -1.0, 0.0, stream_), "subtract");
+               check(launch_pauli_accumulate(d_state_, last_out, prec_, n_amps_, 0, 0, 1.0, 0.0, stream_), "add");
+          }
+          else commit_tmp();
           check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
           return;
      }

@@ -11,7 +11,8 @@ CSRC = os.path.join(os.path.dirname(HERE), "hiqsimulator_amd", "csrc")
 SAN = ["-fsanitize=address,undefined", "-fno-sanitize-recover=all", "-fno-omit-frame-pointer"]
 
 
-@pytest.mark.parametrize("unit,said", [("gate_failure", "gate failures ok")])
+@pytest.mark.parametrize("unit,said", [("gate_failure", "gate failures ok"),
+                                       ("evolve_failure", "evolution failures ok")])
 def test_failures_on_the_way(tmp_path, unit, said):
     hip_inc = "/opt/rocm/include"
     if not os.path.isdir(os.path.join(hip_inc, "hip")):
