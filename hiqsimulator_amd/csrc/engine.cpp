@@ -1189,6 +1189,8 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, c
      passes = 0;
      const int n = n_qubits();
      if (n < gate_min_qubits(prec_) || n > 40) return false;
+     for (const auto& g: items)
+          if (!gate_fits(g.m.a.data(), g.t.size())) return false;
      std::vector<GateUnit> units(items.size());
      for (size_t i = 0; i < items.size(); ++i)
           if (!make_gate_unit(items[i].m.a.data(), items[i].t, items[i].c, units[i])) return false;

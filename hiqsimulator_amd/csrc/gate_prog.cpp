@@ -22,6 +22,21 @@ bool finite(const cplx& z) { return std::isfinite(z.real()) && std::isfinite(z.i
 
 }  // namespace
 
+namespace {
+// index bits that some nonzero entry changes
+size_t mixed_bits(const cplx* m, size_t targets)
+{
+     const size_t dim = size_t(1) << targets;
+     size_t mixed = 0;
+     for (size_t i = 0; i < dim; ++i)
+          for (size_t j = 0; j < dim; ++j)
+               if (i != j && !(m[i * dim + j] == 0.0)) mixed |= i ^ j;
+     return mixed;
+}
+}  // namespace
+
+bool gate_fits(const cplx* m, size_t targets) { return targets <= 2 || (targets <= 5 && popc(mixed_bits(m, targets)) <= 2); }
+
 bool make_gate_unit(const cplx* m, const std::vector<int64_t>& targets, const std::vector<int64_t>& ctrls, GateUnit& out)
 {
      const int t = static_cast<int>(targets.size());
@@ -34,11 +49,7 @@ bool make_gate_unit(const cplx* m, const std::vector<int64_t>& targets, const st
           if (p < 0 || p >= 62) return false;
           cm |= uint64_t(1) << p;
      }
-     // index bits that some nonzero entry changes
-     size_t mixed = 0;
-     for (size_t i = 0; i < dim; ++i)
-          for (size_t j = 0; j < dim; ++j)
-               if (i != j && !(m[i * dim + j] == 0.0)) mixed |= i ^ j;
+     const size_t mixed = mixed_bits(m, targets.size());
      const int na = popc(mixed);
      if (na > 2) return false;
      out = GateUnit();

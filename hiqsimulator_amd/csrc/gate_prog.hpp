@@ -198,6 +198,11 @@ struct GateUnit {
 bool make_gate_unit(const std::complex<double>* m, const std::vector<int64_t>& targets,
                     const std::vector<int64_t>& ctrls, GateUnit& out);
 
+// Whether the matrix mixes at most two of its targets.  Asked before the units
+// of a list are made: a list with one gate that mixes three spent 0.1 ms on 470
+// units (0.92 ms as tile programs on 16 qubits).
+bool gate_fits(const std::complex<double>* m, size_t targets);
+
 // ---- host: which way a list goes --------------------------------------------
 // What a list takes either way, counted in one sweep over its units.
 //   work      of a gate program: a rotation, a phase or a CNOT is 1, a general

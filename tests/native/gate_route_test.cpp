@@ -133,6 +133,34 @@ int main()
           CHECK(way(l.random_layers(20), n, Prec::C64) == kTiles);
      }
      CHECK(way(Lists{12}.random_layers(3), 12, Prec::C128) == kTiles);
+     // what is asked before the units are made agrees with them
+     {
+          Maker mk{std::mt19937(3), 9};
+          int fit = 0, total = 0;
+          auto ask = [&](const std::vector<cplx>& m, size_t k) {
+               GateUnit u;
+               const std::vector<int64_t> t = {2, 0, 5, 7, 1};
+               const bool made = make_gate_unit(m.data(), {t.begin(), t.begin() + static_cast<long>(k)}, {}, u);
+               CHECK(gate_fits(m.data(), k) == made);
+               fit += made;
+               ++total;
+          };
+          for (int i = 0; i < 200; ++i) {
+               const Gate g = mk.gate(9);
+               ask(g.m, g.t.size());
+          }
+          for (size_t k: {3u, 4u, 5u}) {
+               const size_t d = size_t(1) << k;
+               std::vector<cplx> m(d * d);
+               for (size_t i = 0; i < d; ++i) m[i * d + i] = 1;
+               ask(m, k);
+               m[1] = 0.5, ask(m, k);      // one qubit
+               m[d + 3] = 0.5, ask(m, k);  // two
+               m[3 * d + 7] = 0.5, ask(m, k);
+               ask(mk.random(static_cast<int>(d)), k);
+          }
+          CHECK(fit > 100 && fit < total);
+     }
      // empty lists, identities and factors of everything
      {
           Lists l{24};
