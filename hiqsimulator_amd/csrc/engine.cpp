@@ -1195,7 +1195,7 @@ bool Engine::gate_items(std::vector<PosGate>& items, size_t keep, int& passes, c
      for (size_t i = 0; i < items.size(); ++i)
           if (!make_gate_unit(items[i].m.a.data(), items[i].t, items[i].c, units[i])) return false;
      Prec held;
-     if (!gate_route(gate_list_cost(units), units.size(), n, prec_, held)) return false;
+     if (!gate_route(gate_list_cost(units, n, prec_), units.size(), n, prec_, held)) return false;
      // What is on the stream leaves the list, also when something fails on the way.
      struct Rest {
           std::vector<PosGate>& items;
@@ -1659,13 +1659,23 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
           const double whole = std::abs(t) * bound;
           const uint64_t segments = static_cast<uint64_t>(std::ceil(whole / kSegment));
           // The state itself is only read until the whole sum is there.
-          Buf t1(bytes), t2(bytes), own(cmask ? bytes : 0), sum(cmask ? bytes : 0), other(segments > 1 ? bytes : 0);
+          Buf work(bytes * (2 + (segments > 1 ? 1 : 0) + (cmask ? 2 : 0)));
           if (!cmask) ensure_tmp(n_amps_);
-          const void* from = cmask ? own.p : d_state_;  // T_0 of a segment
-          void* const last_out = cmask ? sum.p : d_tmp_;
+          char* next_part = static_cast<char*>(work.p);
+          auto part = [&] {
+               char* const p = next_part;
+               next_part += bytes;
+               return static_cast<void*>(p);
+          };
+          void* const t1 = part();
+          void* const t2 = part();
+          void* const other = segments > 1 ? part() : nullptr;
+          void* const own = cmask ? part() : d_state_;
+          void* const last_out = cmask ? part() : d_tmp_;
+          const void* from = own;  // T_0 of a segment
           if (cmask) {
-               check(launch_copy(own.p, d_state_, prec_, n_amps_, stream_), "copy");
-               check(launch_normalize(own.p, prec_, n_amps_, cmask, cmask, 1.0, nullptr, stream_), "select");
+               check(launch_copy(own, d_state_, prec_, n_amps_, stream_), "copy");
+               check(launch_normalize(own, prec_, n_amps_, cmask, cmask, 1.0, nullptr, stream_), "select");
           }
           const std::vector<double> bes = bessel_series(whole / static_cast<double>(segments));
           const PauliTerm* terms = nullptr;
@@ -1681,10 +1691,10 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
                return 2.0 * (k < bes.size() ? bes[k] : 0.0) * ipow(t < 0 ? e : (4 - e) & 3);
           };
           for (uint64_t seg = 0; seg < segments; ++seg) {
-               void* const out = (segments - 1 - seg) % 2 ? other.p : last_out;
+               void* const out = (segments - 1 - seg) % 2 ? other : last_out;
                for (size_t k = 1; k <= last; ++k) {
-                    void* const dst = k % 2 ? t1.p : t2.p;  // T_k, and T_{k-2} before
-                    const void* const src = k == 1 ? from : (k % 2 ? t2.p : t1.p);
+                    void* const dst = k % 2 ? t1 : t2;  // T_k, and T_{k-2} before
+                    const void* const src = k == 1 ? from : (k % 2 ? t2 : t1);
                     for (size_t p = 0; p < plan.passes.size(); ++p) {
                          PauliApply q;
                          q.src = src;
@@ -1717,7 +1727,7 @@ void Engine::time_evolution(const std::vector<uint64_t>& xm, const std::vector<u
                check(launch_scale(last_out, prec_, n_amps_, ph.real(), ph.imag(), stream_), "phase");
           }
           if (cmask) {
-               check(launch_pauli_accumulate(d_state_, own.p, prec_, n_amps_, 0, 0, -1.0, 0.0, stream_), "subtract");
+               check(launch_pauli_accumulate(d_state_, own, prec_, n_amps_, 0, 0, -1.0, 0.0, stream_), "subtract");
                check(launch_pauli_accumulate(d_state_, last_out, prec_, n_amps_, 0, 0, 1.0, 0.0, stream_), "add");
           }
           else commit_tmp();

@@ -141,6 +141,8 @@ namespace {
 
 bool is_flip(const GateBranch& b) { return b.u[0] == 0.0 && b.u[3] == 0.0 && is_one(b.u[1]) && is_one(b.u[2]); }
 
+constexpr int kGateHostBound = 18;  // up to here the work a gate decides alone
+
 // What an unconditional gate on one qubit is merged with (put_one, layer_phase).
 enum Run : uint8_t { kRunNone, kRunPhase, kRunReal, kRunCross, kRunGeneral };
 
@@ -157,11 +159,12 @@ Run run_of(const GateUnit& g)
 
 }  // namespace
 
-GateListCost gate_list_cost(const std::vector<GateUnit>& units)
+GateListCost gate_list_cost(const std::vector<GateUnit>& units, int n, Prec prec)
 {
      constexpr double kGeneral = 3.7, kTwo = 6.5, kFactor = 0.5, kTested = 2.0;
      constexpr int kWidth = 4;
      GateListCost c;
+     const bool need_products = n > kGateHostBound || prec == Prec::C64;
      Run run[64] = {};  // of each qubit's last gate, while it can still take another
      auto end_run = [&](uint64_t bits) {
           for (; bits; bits &= bits - 1) {
@@ -204,6 +207,7 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units)
                }
           }
           mixed |= g.a;
+          if (!need_products) continue;
           // the fused product that it would go into
           const int first = last[__builtin_ctzll(bits)];
           bool inside = first >= 0;
@@ -239,7 +243,7 @@ bool gate_route(const GateListCost& cost, size_t gates, int n, Prec prec, Prec& 
           return true;
      }
      if (n <= 22 && cost.work <= 4.0 * static_cast<double>(gates)) return true;  // bound by the host
-     return n > 18 && cost.work <= (prec == Prec::C128 ? 24.0 : 13.0) * cost.products;
+     return n > kGateHostBound && cost.work <= (prec == Prec::C128 ? 24.0 : 13.0) * cost.products;
 }
 
 // ---------------------------------------------------------------------------

@@ -217,7 +217,8 @@ bool gate_fits(const std::complex<double>* m, size_t targets);
 struct GateListCost {
      double work = 0, products = 0, rounds = 0;
 };
-GateListCost gate_list_cost(const std::vector<GateUnit>& units);
+// (products are left 0 where gate_route does not ask for them)
+GateListCost gate_list_cost(const std::vector<GateUnit>& units, int n, Prec prec);
 // The precision that a gate program of the list would hold the amplitudes of
 // an n-qubit state in; false: the list runs as tile programs.
 //

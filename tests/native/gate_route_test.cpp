@@ -88,7 +88,7 @@ Way way(const std::vector<Gate>& gates, int n, Prec prec)
 {
      std::vector<GateUnit> units(gates.size());
      for (size_t i = 0; i < gates.size(); ++i) CHECK(make_gate_unit(gates[i].m.data(), gates[i].t, gates[i].c, units[i]));
-     const GateListCost c = gate_list_cost(units);
+     const GateListCost c = gate_list_cost(units, n, prec);
      CHECK(c.work >= 0 && c.products >= 0 && c.rounds >= 0);
      Prec held;
      if (!gate_route(c, gates.size(), n, prec, held)) return kTiles;
@@ -165,7 +165,7 @@ int main()
      {
           Lists l{24};
           Prec held;
-          CHECK(gate_route(gate_list_cost({}), 0, 24, Prec::C128, held));
+          CHECK(gate_route(gate_list_cost({}, 24, Prec::C128), 0, 24, Prec::C128, held));
           std::vector<Gate> id(10, Gate{{1, 0, 0, 1}, {3}, {}});
           CHECK(way(id, 24, Prec::C64) == kFp32);
           id.push_back(Gate{{cplx(0, 1), 0, 0, cplx(0, 1)}, {2}, {}});
