@@ -72,8 +72,7 @@ bool make_gate_unit(const cplx* m, const std::vector<int64_t>& targets, const st
      }
      const int ad = 1 << na;
      // the block of each setting of the unmixed targets
-     auto branch = [&](int s) {
-          GateBranch b;
+     auto branch = [&](int s, GateBranch& b) {
           b.cmask = cm;
           b.cval = cm;
           size_t row0 = 0;
@@ -94,9 +93,9 @@ bool make_gate_unit(const cplx* m, const std::vector<int64_t>& targets, const st
                     }
                     b.u[i * ad + j] = m[r * dim + c];
                }
-          return b;
      };
-     for (int s = 0; s < (1 << nd); ++s) out.br.push_back(branch(s));
+     out.br.resize(size_t(1) << nd);
+     for (int s = 0; s < (1 << nd); ++s) branch(s, out.br[static_cast<size_t>(s)]);
      // the same block in every setting: the unmixed targets do not matter
      bool same = na > 0 && nd > 0;
      for (const auto& b: out.br)
@@ -116,15 +115,13 @@ bool make_gate_unit(const cplx* m, const std::vector<int64_t>& targets, const st
           }
      }
      // identity branches do nothing
-     std::vector<GateBranch> keep;
-     for (const auto& b: out.br) {
-          bool id = true;
+     auto identity = [&](const GateBranch& b) {
           for (int i = 0; i < ad; ++i)
                for (int j = 0; j < ad; ++j)
-                    if (!(i == j ? is_one(b.u[i * ad + j]) : b.u[i * ad + j] == 0.0)) id = false;
-          if (!id) keep.push_back(b);
-     }
-     out.br.swap(keep);
+                    if (!(i == j ? is_one(b.u[i * ad + j]) : b.u[i * ad + j] == 0.0)) return false;
+          return true;
+     };
+     out.br.erase(std::remove_if(out.br.begin(), out.br.end(), identity), out.br.end());
      // a bit that no branch depends on any more is free (e.g. both settings
      // of a target became identity)
      uint64_t dep = 0;
