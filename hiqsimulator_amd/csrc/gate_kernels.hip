@@ -602,14 +602,25 @@ __device__ __forceinline__ void gate_program(VT<S>* psi, const GatePass& P,
      V x[A];
      {
           const VT<S>* const p = psi + base + thread_index(tid, P.in_thr);
-          VT<S> in[A];
+          if constexpr (sizeof(S) == sizeof(R)) {
 #pragma unroll
-          for (int k = 0; k < A; ++k) {
-               in[k] = ld_nt(p + reg_index(k, P.in_reg));
-               if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+               for (int k = 0; k < A; ++k) {
+                    x[k] = ld_nt(p + reg_index(k, P.in_reg));
+                    if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+               }
+#pragma unroll
+               for (int k = 0; k < A; ++k) x[k] = copy_amp(x[k]);
           }
+          else {
+               VT<S> in[A];
 #pragma unroll
-          for (int k = 0; k < A; ++k) x[k] = copy_amp(converted<R>(in[k]));
+               for (int k = 0; k < A; ++k) {
+                    in[k] = ld_nt(p + reg_index(k, P.in_reg));
+                    if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+               }
+#pragma unroll
+               for (int k = 0; k < A; ++k) x[k] = converted<R>(in[k]);
+          }
      }
      uint32_t s = 0, slot = 0;
      do {

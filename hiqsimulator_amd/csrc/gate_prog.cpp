@@ -156,19 +156,70 @@ Run run_of(const GateUnit& g)
 
 }  // namespace
 
+// Whether the block is applied without rounded coefficients: entries that are
+// zero or the first one's turns by quarters.
+bool without_rounded(const GateUnit& g, const GateBranch& b)
+{
+     const int entries = 1 << (2 * g.na);
+     cplx p = 1.0;
+     for (int i = 0; g.na && i < entries; ++i)
+          if (!(b.u[i] == 0.0)) {
+               p = b.u[i];
+               break;
+          }
+     for (int i = 0; i < entries; ++i) {
+          const cplx z = b.u[i];
+          if (!(z == 0.0 || z == p || z == -p || z == cplx(-p.imag(), p.real()) || z == cplx(p.imag(), -p.real()))) return false;
+     }
+     return true;
+}
+
+// 0 for a unit without rounded coefficients.
+uint64_t hash_of(const GateUnit& g)
+{
+     uint64_t h = 0;
+     for (const auto& b: g.br) {
+          if (without_rounded(g, b)) continue;
+          const int words = 2 << (2 * g.na);
+          uint64_t v[32];
+          std::memcpy(v, b.u, static_cast<size_t>(words) * 8);
+          for (int i = 0; i < words; ++i) {
+               h = (h ^ v[i]) * 0x9e3779b97f4a7c15ull;
+               h ^= h >> 29;
+          }
+          h |= 1;
+     }
+     return h;
+}
+
 GateListCost gate_list_cost(const std::vector<GateUnit>& units, int n, Prec prec)
 {
      constexpr double kGeneral = 3.7, kTwo = 6.5, kFactor = 0.5, kTested = 2.0;
      constexpr int kWidth = 4;
      GateListCost c;
-     const bool need_products = n > kGateHostBound || prec == Prec::C64;
-     Run run[64] = {};  // of each qubit's last gate, while it can still take another
+     const bool need_products = n > kGateHostBound || prec == Prec::C64, need_rounds = prec == Prec::C64;
+     // The roundings of gates with the same coefficients come out the same and add
+     // up: m of them count as m^2.
+     struct Rounding {
+          uint64_t same;
+          double count;
+     };
+     std::vector<Rounding> roundings;
+     auto round = [&](uint64_t same, double count) {
+          if (!need_rounds) return;
+          if (same) roundings.push_back({same, count});
+          else c.rounds += count;
+     };
+     Run run[64] = {};    // of each qubit's last gate, while it can still take another
+     uint64_t same[64];   // the run's coefficients
      auto end_run = [&](uint64_t bits) {
           for (; bits; bits &= bits - 1) {
-               Run& r = run[__builtin_ctzll(bits)];
-               if (r == kRunGeneral) c.work += kGeneral, c.rounds += 2;
-               else if (r != kRunNone) c.work += 1, c.rounds += 1;
-               r = kRunNone;
+               const int p = __builtin_ctzll(bits);
+               if (run[p] == kRunNone) continue;
+               const bool general = run[p] == kRunGeneral;
+               c.work += general ? kGeneral : 1;
+               round(same[p], general ? 2 : 1);
+               run[p] = kRunNone;
           }
      };
      std::vector<uint64_t> groups;  // qubits of the fused products
@@ -184,23 +235,31 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units, int n, Prec prec
      for (const GateUnit& g: units) {
           const uint64_t bits = g.a | g.d;
           if (g.br.empty() || !bits) continue;  // (a factor of all amplitudes costs nothing)
-          const bool single = popc(bits) == 1 && (g.na == 0 || (g.br.size() == 1 && !g.br[0].cmask));
-          if (single) {
-               Run& r = run[__builtin_ctzll(bits)];
+          const uint64_t h = need_rounds ? hash_of(g) : 0;
+          if (popc(bits) == 1 && (g.na == 0 || (g.br.size() == 1 && !g.br[0].cmask))) {
+               const int p = __builtin_ctzll(bits);
                const Run now = run_of(g);
-               if (r != kRunNone && r != now) {
-                    if (r != kRunPhase && now != kRunPhase && (r == kRunGeneral || now == kRunGeneral)) r = kRunGeneral;
+               if (run[p] != kRunNone && run[p] != now) {
+                    if (run[p] != kRunPhase && now != kRunPhase && (run[p] == kRunGeneral || now == kRunGeneral)) run[p] = kRunGeneral;
                     else end_run(bits);
                }
-               if (r == kRunNone) r = now;
+               if (run[p] == kRunNone) {
+                    run[p] = now;
+                    same[p] = h;
+               }
+               else {
+                    same[p] = (same[p] * 0x9e3779b97f4a7c15ull) ^ h;
+               }
           }
           else {
-               end_run(g.na ? bits : 0);
+               end_run(bits);
+               // (a factor on a qubit that nothing has mixed yet goes into a list's product, in FP64)
+               const bool listed = g.na == 0 && (bits & ~mixed);
                for (const auto& b: g.br) {
-                    if (g.na == 0) c.work += bits & ~mixed ? kFactor : kTested, c.rounds += 0.25;
-                    else if (g.na == 2) c.work += kTwo, c.rounds += 4;
+                    if (g.na == 0) c.work += listed ? kFactor : kTested, round(listed ? 0 : h, 0.25);
+                    else if (g.na == 2) c.work += kTwo, round(h, 4);
                     else if (is_flip(b)) c.work += 1;
-                    else c.work += kGeneral, c.rounds += 2;
+                    else c.work += kGeneral, round(h, 2);
                }
           }
           mixed |= g.a;
@@ -228,6 +287,12 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units, int n, Prec prec
      }
      c.products = slots / 4;
      end_run(~uint64_t(0));
+     std::sort(roundings.begin(), roundings.end(), [](const Rounding& a, const Rounding& b) { return a.same < b.same; });
+     for (size_t i = 0, j; i < roundings.size(); i = j) {
+          double sum = 0;
+          for (j = i; j < roundings.size() && roundings[j].same == roundings[i].same; ++j) sum += roundings[j].count;
+          c.rounds += sum * static_cast<double>(j - i);
+     }
      return c;
 }
 
@@ -235,12 +300,13 @@ bool gate_route(const GateListCost& cost, size_t gates, int n, Prec prec, Prec& 
 {
      held = Prec::C128;
      if (n < gate_min_qubits(prec) || n > 40) return false;
-     if (prec == Prec::C64 && cost.rounds <= 1.5 * cost.products) {
+     // (two more for the factor of a whole pass)
+     if (prec == Prec::C64 && cost.rounds + 2 <= 1.5 * cost.products) {
           held = Prec::C64;
           return true;
      }
      if (n <= 22 && cost.work <= 4.0 * static_cast<double>(gates)) return true;  // bound by the host
-     return n > kGateHostBound && cost.work <= (prec == Prec::C128 ? 24.0 : 13.0) * cost.products;
+     return n > kGateHostBound && cost.work <= (prec == Prec::C128 ? 24.0 : (n <= 24 ? 18.0 : 13.0)) * cost.products;
 }
 
 // ---------------------------------------------------------------------------

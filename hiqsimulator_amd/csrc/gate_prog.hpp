@@ -12,8 +12,8 @@
 // wherever they are, so a pass takes gates that a dense plan cannot.
 //
 // Below, a precision is the one that the amplitudes have in a pass.  A
-// complex64 state is held in complex128 for most lists (gate_route): in FP32,
-// gate after gate, its roundings are more than those of the fused products.
+// complex64 state is held in complex128 for lists whose roundings in FP32, gate
+// after gate, could be more than those of the fused products (gate_route).
 //
 // A pass covers tiles of 2^13 amplitudes in complex128 and 2^14 in complex64:
 // index bits 0..3 (runs of 16 amplitudes: 256 and 128 bytes) and nine or ten
@@ -52,7 +52,7 @@ constexpr int gate_high(Prec p) { return gate_tile_bits(p) - kGateLow; }  // cho
 // bound by its host work, which is less (703 against 877 us a call at 16
 // qubits, 1189 against 1265 at 20).  Complex64 keeps the tile programs there:
 // their kernels are ahead by more (20 qubits: 221 against 314 us; 22: 459
-// against 403).
+// against 403, held in FP32).
 constexpr int gate_min_qubits(Prec p) { return p == Prec::C128 ? 13 : 21; }
 constexpr int kGateMaxReg = 5, kGateMaxTile = kGateThr + kGateMaxReg, kGateMaxHigh = kGateMaxTile - kGateLow;
 constexpr size_t kGateMaxStages = 255;      // a pass's stage count is a byte
@@ -213,7 +213,11 @@ bool gate_fits(const std::complex<double>* m, size_t targets);
 //   products  fused products on four qubits that a tile program needs about:
 //             a quarter of the qubits of greedily grown groups of up to four.
 //   rounds    roundings of an amplitude that a gate program makes in the
-//             precision it is held in.
+//             precision it is held in, as their squares add up: one for a
+//             rotation or a phase, two for a general block, four for a 4 x 4
+//             block, a quarter for a factor of two or more qubits; m gates of
+//             the same rounded coefficients make m^2, for theirs are the same
+//             each time.  (For complex64 states.)
 struct GateListCost {
      double work = 0, products = 0, rounds = 0;
 };
@@ -224,23 +228,27 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units, int n, Prec prec
 //
 // Time.  Tile programs over gate programs, with work per product in brackets.
 // Complex128, 28 qubits: QFT (2) 7.5, CNOT ladder (3) 2.2, layers of rotations
-// and CNOTs (12) 1.6, Trotter steps of an Ising chain (14) 1.4, 2-qubit Haar
+// and CNOTs (12) 1.6, Trotter steps of an Ising chain (20) 1.4, 2-qubit Haar
 // bricks (23) 1.2, three rotations a qubit and layer (27) 0.92, one-qubit Haar
 // and CNOT (31) 0.82, five rotations (40) 0.72, 200 layers on 4 qubits (1046)
 // 0.12: up to 24.  Complex64 held in FP64 against products in FP32, 28 qubits:
-// CNOT ladder 1.6, layers 1.0, Ising steps 0.75, 2-qubit bricks 0.71, three
-// rotations 0.58: up to 13.  Up to 22 qubits the host and a workgroup's latency
-// bound both ways (0.5 us a unit of work against 1.25 us a gate for the fusion):
-// of these lists only those of dense 2-qubit blocks are faster as products (0.66
-// at 13 qubits, 0.9 at 16, 1.1 at 20).
+// CNOT ladder 1.6, layers (12) 1.0, H and CZ (14) 0.82, Ising steps 0.75, 2-qubit
+// bricks 0.71, three rotations 0.58: up to 13, and up to 18 for 24 qubits or
+// less, where the host takes a good part of it (Heisenberg steps (17) 1.5 at 23
+// qubits, 1.2 at 24).  Up to 22 qubits the host and a workgroup's latency bound
+// both ways (0.5 us a unit of work against 1.25 us a gate for the fusion): of
+// these lists only those of dense 2-qubit blocks are faster as products (0.66 at
+// 13 qubits, 0.9 at 16, 1.1 at 20).
 //
 // Roundings.  Error of gate programs held in FP32 over that of tile programs (l2,
-// complex64, 25 qubits): QFT 0.54, layers with random angles 0.75, three
-// rotations 1.1, 40 Trotter steps of an Ising chain 2.9 (a coefficient's rounding
-// comes back in every step), 200 layers on 4 qubits 6.4.  Held in FP64: 0.05 to
-// 0.2 for all of them.  So FP32 only up to 1.5 roundings a product (QFT 1.2;
-// Ising steps 4, layers 10), where even roundings that add up stay below the
-// products'.
+// complex64, 25 qubits), with roundings per product in brackets.  Random states:
+// QFT (1) 0.54, layers with random angles and CNOTs (8) 0.75, one-qubit Haar (8)
+// 0.86, one-qubit Haar and CNOT (15) 1.1, three rotations (24) 1.1, five (37) 1.4,
+// 200 layers on 4 qubits (700) 6.4; the same angles again and again: QAOA (240)
+// 1.3, four Heisenberg steps (290) 2.4, 40 Ising steps (9400) 2.9.  From |0..0>:
+// layers of Ry and CNOTs (8) 1.1, one-qubit Haar (8) 1.4, H and CZ (9) 2.7.  Held
+// in FP64: 0.05 to 0.2 throughout.  So FP32 only up to 1.5, QFTs and ladders of
+// CNOTs, which it leaves no further off (and takes 0.75 of the time for).
 bool gate_route(const GateListCost& cost, size_t gates, int n, Prec prec, Prec& held);
 
 // ---- host: planning ---------------------------------------------------------

@@ -44,6 +44,10 @@ struct Lists {
                out.push_back({k == 0 ? rx(u()) : (k == 1 ? ry(u()) : rz(u())), {q}, {}});
           });
      }
+     std::vector<Gate> equal_layers(int count)
+     {
+          return layers(count, all(), [&](std::vector<Gate>& out, int64_t q) { out.push_back({rx(0.4), {q}, {}}); });
+     }
      std::vector<Gate> zxzxz(int count, const std::vector<int64_t>& qs)
      {
           return layers(count, qs, [&](std::vector<Gate>& out, int64_t q) {
@@ -103,10 +107,23 @@ int main()
           Lists l{n};
           const std::vector<int64_t> few = {1, 5, n - 2, n / 2};
           const bool large = n > 22;
-          // roundings of many rotations, of repeated ones and of long lists on few
-          // qubits are never made in FP32
-          for (int count: {2, 4, 20, 60}) CHECK(way(l.random_layers(count), n, Prec::C64) == kFp64);
-          for (int steps: {1, 5, 40}) CHECK(way(l.ising(steps), n, Prec::C64) != kFp32);
+          // rotations, repeated angles and long lists on few qubits are never held in
+          // FP32
+          for (int count: {2, 4, 20, 60}) {
+               CHECK(way(l.random_layers(count), n, Prec::C64) == kFp64);
+               CHECK(way(l.equal_layers(count), n, Prec::C64) == kFp64);
+          }
+          // few rotations among many CNOTs are, if their angles differ
+          for (bool equal: {false, true}) {
+               std::vector<Gate> g;
+               for (int i = 0; i < 200; ++i) {
+                    for (const Gate& x: l.ladder()) g.push_back(x);
+                    g.push_back({l.rx(equal ? 0.4 : 0.4 + 0.01 * i), {i % n}, {}});
+               }
+               CHECK(way(g, n, Prec::C64) == (equal ? kFp64 : kFp32));
+          }
+          CHECK(way(l.ising(1), n, Prec::C64) == kFp64);
+          for (int steps: {5, 40}) CHECK(way(l.ising(steps), n, Prec::C64) == (large ? kTiles : kFp64));
           for (int count: {1, 10, 200}) CHECK(way(l.zxzxz(count, few), n, Prec::C64) != kFp32);
           CHECK(way(Qft{n, 0}.gates(), n, Prec::C64) == kFp32);
           CHECK(way(Qft{n, 5}.gates(), n, Prec::C64) == kFp32);
@@ -167,7 +184,7 @@ int main()
           Prec held;
           CHECK(gate_route(gate_list_cost({}, 24, Prec::C128), 0, 24, Prec::C128, held));
           std::vector<Gate> id(10, Gate{{1, 0, 0, 1}, {3}, {}});
-          CHECK(way(id, 24, Prec::C64) == kFp32);
+          CHECK(way(id, 24, Prec::C64) == kFp64);
           id.push_back(Gate{{cplx(0, 1), 0, 0, cplx(0, 1)}, {2}, {}});
           CHECK(way(id, 24, Prec::C128) == kFp64);
      }
