@@ -303,10 +303,11 @@ private:
      ProgSlot prog_[kProgSlots];
      int prog_next_ = 0;
 
-     // Deferred gates (kPassDeferred): matrices on bit positions.  Planning
-     // over 256+ gates at a time gives nearly the passes of planning the
-     // whole list (56 against 56 for the 30-qubit, 1780-gate circuit through
-     // the GreedyScheduler loop; 101 when whole clusters are queued).
+     // Deferred gates (kPassDeferred): matrices on bit positions.  Planning over
+     // 256+ gates at a time gives the passes of planning the whole list: gate
+     // passes of the 30-qubit, 1780-gate circuit for queues of 128, 256, 512 and
+     // 1780 gates 37, 29, 27, 27 in the GreedyScheduler's order, 40, 28, 26, 25 in
+     // circuit order (tile passes 56 and 56; 101 when whole clusters are queued).
      static constexpr size_t kQueueHigh = 512, kQueueLow = 256;
      int pass_mode_ = kPassDeferred;
      std::vector<PosGate> queue_;

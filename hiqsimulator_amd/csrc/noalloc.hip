@@ -3,7 +3,7 @@
 // hiqsim_sample draws shots through the engine's own device buffers (block
 // probabilities, descriptors, an output array it grows on demand).  Callers
 // that cannot allocate (code under HIP graph capture, request loops that
-// forbid hipMalloc) get the same two kernels here, launched on their stream
+// forbid hipMalloc) get the same three launches here, launched on their stream
 // over their state and output arrays, with every intermediate in one static
 // device array per GPU:
 //   [0, 2^15) doubles       block probabilities, turned into a running sum
