@@ -218,7 +218,7 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units, int n, Prec prec
                if (run[p] == kRunNone) continue;
                const bool general = run[p] == kRunGeneral;
                c.work += general ? kGeneral : 1;
-               round(same[p], general ? 2 : 1);
+               round(same[p], general ? 3 : 1);
                run[p] = kRunNone;
           }
      };
@@ -256,10 +256,10 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units, int n, Prec prec
                // (a factor on a qubit that nothing has mixed yet goes into a list's product, in FP64)
                const bool listed = g.na == 0 && (bits & ~mixed);
                for (const auto& b: g.br) {
-                    if (g.na == 0) c.work += listed ? kFactor : kTested, round(listed ? 0 : h, 0.25);
+                    if (g.na == 0) c.work += listed ? kFactor : kTested, round(listed ? 0 : h, listed ? 0.25 : 0.75);
                     else if (g.na == 2) c.work += kTwo, round(h, 4);
                     else if (is_flip(b)) c.work += 1;
-                    else c.work += kGeneral, round(h, 2);
+                    else c.work += kGeneral, round(h, 3);
                }
           }
           mixed |= g.a;
@@ -301,7 +301,7 @@ bool gate_route(const GateListCost& cost, size_t gates, int n, Prec prec, Prec& 
      held = Prec::C128;
      if (n < gate_min_qubits(prec) || n > 40) return false;
      // (two more for the factor of a whole pass)
-     if (prec == Prec::C64 && cost.rounds + 2 <= 1.5 * cost.products) {
+     if (prec == Prec::C64 && cost.rounds + 2 <= 9.5 * cost.products) {
           held = Prec::C64;
           return true;
      }

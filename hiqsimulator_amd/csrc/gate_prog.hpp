@@ -214,10 +214,10 @@ bool gate_fits(const std::complex<double>* m, size_t targets);
 //             a quarter of the qubits of greedily grown groups of up to four.
 //   rounds    roundings of an amplitude that a gate program makes in the
 //             precision it is held in, as their squares add up: one for a
-//             rotation or a phase, two for a general block, four for a 4 x 4
-//             block, a quarter for a factor of two or more qubits; m gates of
-//             the same rounded coefficients make m^2, for theirs are the same
-//             each time.  (For complex64 states.)
+//             rotation or a phase, three for a general block, four for a 4 x 4
+//             block, 0.25 (or 0.75, where its work is 2) for a conditional
+//             factor; m gates of the same rounded coefficients make m^2, for
+//             theirs are the same each time.  (For complex64 states.)
 struct GateListCost {
      double work = 0, products = 0, rounds = 0;
 };
@@ -241,14 +241,17 @@ GateListCost gate_list_cost(const std::vector<GateUnit>& units, int n, Prec prec
 // 13 qubits, 0.9 at 16, 1.1 at 20).
 //
 // Roundings.  Error of gate programs held in FP32 over that of tile programs (l2,
-// complex64, 25 qubits), with roundings per product in brackets.  Random states:
-// QFT (1) 0.54, layers with random angles and CNOTs (8) 0.75, one-qubit Haar (8)
-// 0.86, one-qubit Haar and CNOT (15) 1.1, three rotations (24) 1.1, five (37) 1.4,
-// 200 layers on 4 qubits (700) 6.4; the same angles again and again: QAOA (240)
-// 1.3, four Heisenberg steps (290) 2.4, 40 Ising steps (9400) 2.9.  From |0..0>:
-// layers of Ry and CNOTs (8) 1.1, one-qubit Haar (8) 1.4, H and CZ (9) 2.7.  Held
-// in FP64: 0.05 to 0.2 throughout.  So FP32 only up to 1.5, QFTs and ladders of
-// CNOTs, which it leaves no further off (and takes 0.75 of the time for).
+// complex64, 25 qubits, random states), with roundings per product in brackets:
+// QFT (1) 0.54, factors on three qubits (3) 0.5, H on every qubit (4) 0.52, layers
+// with random angles and CNOTs (8) 0.75, of Ry alone 0.64, 40 layers on 8 qubits
+// (10) 0.79; one-qubit Haar (12) 0.86 and, from |0..0>, 1.4; H and CZ (10) 0.68
+// and 2.7; one-qubit Haar and CNOT (22) 1.1, three rotations (24) 1.1, five (37)
+// 1.4, 200 layers on 4 qubits (700) 6.4; the same angles again and again: QAOA
+// (240) 1.3, four Heisenberg steps (290) 2.4, 40 Ising steps (9400) 2.9.  So FP32
+// up to 9.5; layers with random angles from |0..0> are within a tenth of tile
+// programs there (0.9 to 1.1).  Held in FP64 the error is 0.05 to 0.2 of that of
+// tile programs, and a list takes 1.25 times (23 qubits) to 1.65 times (28) as long
+// as in FP32.
 bool gate_route(const GateListCost& cost, size_t gates, int n, Prec prec, Prec& held);
 
 // ---- host: planning ---------------------------------------------------------

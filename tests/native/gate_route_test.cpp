@@ -107,18 +107,19 @@ int main()
           Lists l{n};
           const std::vector<int64_t> few = {1, 5, n - 2, n / 2};
           const bool large = n > 22;
-          // rotations, repeated angles and long lists on few qubits are never held in
-          // FP32
+          // repeated angles, many rotations a qubit and long lists on few qubits are
+          // never held in FP32; layers of different angles are
           for (int count: {2, 4, 20, 60}) {
-               CHECK(way(l.random_layers(count), n, Prec::C64) == kFp64);
+               CHECK(way(l.random_layers(count), n, Prec::C64) == kFp32);
                CHECK(way(l.equal_layers(count), n, Prec::C64) == kFp64);
           }
-          // few rotations among many CNOTs are, if their angles differ
+          // and a few rotations among many CNOTs
           for (bool equal: {false, true}) {
                std::vector<Gate> g;
-               for (int i = 0; i < 200; ++i) {
-                    for (const Gate& x: l.ladder()) g.push_back(x);
-                    g.push_back({l.rx(equal ? 0.4 : 0.4 + 0.01 * i), {i % n}, {}});
+               for (int i = 0; i < 1000; ++i) {
+                    const int q = 5 * i % (n - 4);
+                    for (int k = 0; k < 4; ++k) g.push_back({l.x, {q + k + 1}, {q + k}});
+                    g.push_back({l.rx(equal ? 0.4 : 0.4 + 0.001 * i), {q}, {}});
                }
                CHECK(way(g, n, Prec::C64) == (equal ? kFp64 : kFp32));
           }
